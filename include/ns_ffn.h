@@ -121,7 +121,9 @@ int ns_ctx_workspace_bytes(const ns_ctx *ctx, uint64_t *bytes);
  * FFN block as two launches), "block_spin" (> 0: the one-launch block's bound on
  * a wait, in polls; tests shorten it to exercise the bound), "gemm_rs" (0: split-K
  * FP16-mode prefill GEMMs finish by the last part to arrive instead of the
- * reduce-scatter; > 1: the reduce-scatter's bound on its wait).  Results stay within
+ * reduce-scatter; > 1: the reduce-scatter's bound on its wait), "gemm_skinny" (-1 plan, 0 never
+ * the few-token prefill GEMM, > 0 up to that many tokens), "skinny_wk" (4 / 8) and "skinny_mi"
+ * (1 / 2 / 4): its super-block groups and its token tile in 32-token units.  Results stay within
  * the same tolerances; engines leave the defaults. */
 int ns_ctx_set_tuning(ns_ctx *ctx, const char *key, int value);
 

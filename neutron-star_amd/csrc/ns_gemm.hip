@@ -976,6 +976,13 @@ void gemm_workspace_need(int type, int layout, uint32_t cols, uint32_t rows, uin
     gemm_fp32_workspace_need(type, layout, cols, rows, batch, pair, t, &f32_floats, &f32_counters);
     *floats = std::max(f16_floats, f32_floats);
     *counters = std::max(f16_counters, f32_counters);
+    for (int acc : {ACC_FP32, ACC_FP16})
+        if (gemm_skinny_eligible(type, layout, acc, cols, &rows, 1, batch, pair, t)) {
+            size_t f = 0, c = 0;
+            gemm_skinny_workspace_need(type, cols, &rows, 1, batch, pair, acc, t, &f, &c);
+            *floats = std::max(*floats, f);
+            *counters = std::max(*counters, c);
+        }
 }
 
 static void gemm_fp32_workspace_need(int type, int layout, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
@@ -995,6 +1002,9 @@ static void gemm_fp32_workspace_need(int type, int layout, uint32_t cols, uint32
 hipError_t launch_gemm(int type, int layout, int acc, const uint8_t *w, const uint8_t *up, const uint16_t *x,
                        void *out, uint32_t cols, uint32_t rows, uint32_t batch, const Workspace &ws,
                        hipStream_t stream) {
+    if (gemm_skinny_eligible(type, layout, acc, cols, &rows, 1, batch, up != nullptr, ws.tune))
+        return launch_gemm_skinny(type, layout, acc, &w, up, &out, &rows, 1, x, cols, batch, ws.partial, ws.counters,
+                                  ws.tune, stream);
     if (layout == CDNA4 && acc == ACC_FP16)
         return launch_gemm_f16(type, w, up, x, out, cols, rows, batch, ws.partial, ws.counters, ws.err, ws.tune,
                                stream);

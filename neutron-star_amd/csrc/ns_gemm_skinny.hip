@@ -1,0 +1,770 @@
+// ns_gemm_skinny.hip -- prefill GEMM for few tokens (one 32- to 128-token tile per workgroup) on
+// fp16 MFMA, for gfx950: CDNA4 layout in both accumulation modes, ROW_MAJOR in the FP32 mode.
+//
+// Replaces, for small batches, the same reference kernels as ns_gemm_reg.hip, ns_gemm_f16.hip and
+// ns_gemm.hip (metal/gemma4.metal:263-301, 373-395, 432-490; metal_engine.mm:274, :288-289, :311).
+//
+// What bounds it: below ~100 tokens the weight bytes (a 256-token tile spent most of its matrix
+// work on padding, and the 120 column tiles of the gate/up pair left half the CUs idle), so the
+// work is split over the weights and the token tile is only as tall as the batch needs.
+//
+// Work split.  A workgroup is 8 waves = WC column groups x WK groups of super-blocks.  Each wave
+// owns 64 columns (2 MFMA tiles; for the gate/up pair 32 gate rows and the same 32 up rows) and
+// walks every WK-th super-block of the workgroup's K range alone; the WK partial sums meet in LDS
+// at the end, in wk order.  So 64 * WC columns keep all eight waves streaming weights, and the
+// gate/up pair needs no reduction between workgroups.  A shape with too few columns to fill the
+// device splits K over kparts workgroups as well; the last of them to arrive adds the parts in
+// part order (no workgroup ever waits for another).
+//
+// A wave decodes its own B fragments from raw blocks in registers: lane l holds weight row l%32
+// and, of each pair of 16-byte qs (ql, qh) chunks, the chunk l/32, so one 16-byte load per chunk
+// pair feeds four fragments.  The MFMA sums over k in any order as long as A and B agree on it:
+// fragment (group g, e) covers k = 32g + 16(l/32) + 8e + 0..7 for both block types.  x goes
+// through LDS by DMA in stages of KS columns per wk group, two buffers; rows are stored with their
+// 16-byte chunks XOR-swizzled so the fragment reads are conflict-free.
+//
+// Arithmetic.  FP16 mode: the tiles of ns_tile16.hpp, accumulated across super-blocks; the row
+// scale comes from every wave reading the block factors of its share of the row first.  FP32
+// mode: fragments are exact integers times a power of two (Q4_K sc*q*2^-14; Q6_K sc*(v-32)*2^-16,
+// one rounding past 11 bits as in ns_gemm.hip), summed per super-block in S, and y += d*S in fp32.
+// The Q4_K min term -dmin * sum_g m_g * (sum of x over group g) needs no pass over x ahead of the
+// GEMM: each lane adds up the 16 values per group that its own A fragments hold, in fp32, splits
+// the eight sums exactly into three bf16 pieces, and three bf16 MFMAs multiply them by the m_g
+// (exact in bf16) and add the two lane halves.
+#include <algorithm>
+#include <type_traits>
+
+#include "ns_internal.hpp"
+#include "ns_quant.hpp"
+#include "ns_tile16.hpp"
+
+namespace ns {
+namespace {
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+
+constexpr int kWaves = 8;
+constexpr int kThreads = 64 * kWaves;
+constexpr int NJ = 2;  // 32-column MFMA tiles per wave
+constexpr int kMaxSeg = 3;
+
+// Up to three matrices that share x (Q, K and V): one run of column tiles each.
+struct Args {
+    const uint8_t *w[kMaxSeg], *up;
+    void *out[kMaxSeg];
+    uint32_t rows[kMaxSeg], ct_end[kMaxSeg];
+    const uint16_t *x;
+    float *partial;
+    uint32_t *counters;
+    uint32_t cols, batch, ntok, ncol, kparts;
+};
+
+__device__ __forceinline__ rsrc_t make_rsrc(const void *p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, int(bytes), 0x00020000);
+}
+__device__ __forceinline__ u32x4 bload16(rsrc_t r, uint32_t off, uint32_t soff) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, int(off), int(soff), 0);
+}
+__device__ __forceinline__ uint32_t bload4(rsrc_t r, uint32_t off, uint32_t soff) {
+    return __builtin_amdgcn_raw_buffer_load_b32(r, int(off), int(soff), 0);
+}
+__device__ __forceinline__ uint32_t bload2(rsrc_t r, uint32_t off, uint32_t soff) {
+    return __builtin_amdgcn_raw_buffer_load_b16(r, int(off), int(soff), 0);
+}
+
+// One LDS DMA instruction: 16 bytes per lane into the 1 KiB at lds.
+__device__ __forceinline__ void dma16(rsrc_t r, u32x4 *lds, uint32_t voff, uint32_t soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)lds, 16, voff, soff, 0, 0);
+}
+
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+    static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+// The bare barrier (no wait for loads in flight); signal fences keep memory accesses on their side.
+__device__ __forceinline__ void bare_barrier() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    bare_barrier();
+}
+
+__device__ __forceinline__ float round_f16p(float v) {
+    uint32_t b = __builtin_bit_cast(uint32_t, v);
+    b = (b + 0x0fffu + ((b >> 13) & 1u)) & 0xffffe000u;
+    return __builtin_bit_cast(float, b);
+}
+__device__ __forceinline__ uint32_t bits(half2_t v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ half2_t h2(uint32_t v) { return __builtin_bit_cast(half2_t, v); }
+
+// One lane's raw bytes of one super-block of one column: the chunks of its lane half.
+struct RawQ4 {
+    u32x4 hdr, qs[4];  // qs[p]: chunk 1 + 2p + l/32 (groups 2p low nibbles, 2p+1 high)
+};
+struct RawQ6 {
+    u32x4 ql[4];  // [2h + q]: chunk 4h + 2q + l/32 (quarters q low nibbles, q + 2 high)
+    u32x4 qh[2];  // [h]: chunk 8 + 2h + l/32
+    u32x4 sc;
+    uint32_t d;
+    uint32_t x[7];  // ROW_MAJOR: the dword after each 16-byte piece (blocks are 2-byte aligned)
+};
+
+// WC column groups x WK super-block groups of waves; MI 32-token tiles.
+template <int TYPE, int LAYOUT, int ACC, bool PAIR, int MI, int WK>
+__global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
+    constexpr bool Q4 = TYPE == Q4_K, F16 = ACC == ACC_FP16, ROW = LAYOUT == ROW_MAJOR;
+    constexpr int WC = kWaves / WK, TT = 32 * MI;
+    constexpr int KS = MI * WK <= 8 ? 128 : 64;      // columns of x per stage
+    constexpr int NS = 256 / KS, CR = KS / 8;         // stages per super-block, 16-byte chunks per x row
+    constexpr int RPI = 64 / CR;                      // x rows one DMA instruction fills
+    constexpr int ND = TT / RPI / WC;                 // DMA instructions per wave and stage
+    constexpr int kXBuf = WK * TT * CR;               // u32x4 per buffer
+    static_assert(TT % (RPI * WC) == 0 && 2 * kXBuf * 16 <= 131072, "x stages");
+    using Raw = typename std::conditional<Q4, RawQ4, RawQ6>::type;
+    constexpr int kRedF4 = kWaves * NJ * 16 * 64 / 4;  // u32x4 the final sum of one token tile needs
+    // two LDS objects, so that the compiler does not take a DMA into one for a write to the other
+    __shared__ __attribute__((aligned(16))) u32x4 X0[kXBuf > kRedF4 ? kXBuf : kRedF4], X1[kXBuf > kRedF4 ? kXBuf : kRedF4];
+    __shared__ float rmax[kWaves][NJ][32];
+    __shared__ uint32_t last_flag;
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63, hl = lane >> 5, ln = lane & 31;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wc = wave % WC, wk = wave / WC;
+    // XCD-aware order: workgroup L runs on XCD L % 8, which takes a contiguous run of the work items
+    // q = (ct * kparts + kp) * ntok + tt, so the token tiles that share weights share an L2.
+    const uint32_t nwg = gridDim.x, w8 = nwg / 8, L = blockIdx.x;
+    const uint32_t q = L < 8 * w8 ? (L % 8) * w8 + L / 8 : L;
+    const uint32_t tt = q % a.ntok, g = q / a.ntok, kp = g % a.kparts, ctg = g / a.kparts;
+    const uint32_t tile = ctg * a.ntok + tt;
+    const uint32_t seg = ctg < a.ct_end[0] ? 0u : ctg < a.ct_end[1] ? 1u : 2u;
+    const uint32_t ct = ctg - (seg == 0 ? 0u : a.ct_end[seg - 1]);
+    const uint32_t rows = a.rows[seg], cols = a.cols, batch = a.batch, t0 = tt * TT;
+    const uint32_t nb = cols / kQK, kparts = a.kparts;
+    const uint32_t sb0 = kp * nb / kparts, sb1 = (kp + 1) * nb / kparts;
+    const uint32_t iters = (sb1 - sb0 + WK - 1) / WK;
+
+    constexpr uint32_t kRowsPerTile = PAIR ? WC * 32 : WC * 64;
+    auto brow = [&](int j) -> uint32_t {
+        if constexpr (PAIR) return ct * kRowsPerTile + wc * 32 + ln;  // j 0 = gate, 1 = up
+        else return ct * kRowsPerTile + wc * 64 + uint32_t(j) * 32 + ln;
+    };
+    const uint32_t wbytes = rows * nb * block_bytes(TYPE);
+    const rsrc_t wsrc0 = make_rsrc(a.w[seg], wbytes), wsrc1 = make_rsrc(PAIR ? a.up : a.w[seg], wbytes);
+    auto wsrc = [&](int j) { return (PAIR && j == 1) ? wsrc1 : wsrc0; };
+    const rsrc_t xsrc = make_rsrc(a.x, batch * cols * 2);
+
+    // ---- weight addressing: the lane's part is a VGPR, the super-block's a uniform offset.  Rows past
+    // `rows` lie past the descriptor's range and read zeros.
+    constexpr uint32_t kRegion = kRowTile * block_bytes(TYPE);
+    uint32_t voff[NJ];  // first byte of block (row, 0); CDNA4: of its chunk 0
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const uint32_t r = brow(j);
+        voff[j] = ROW ? r * nb * block_bytes(TYPE) : uint32_t(region_offset(TYPE, r / kRowTile, 0, nb)) + (r % kRowTile) * 16;
+    }
+    // byte offset, past voff + the super-block's uniform part, of chunk c
+    auto chunk = [](uint32_t c) { return c * (ROW ? 16u : 1024u); };
+    constexpr uint32_t kBlkStep = ROW ? block_bytes(TYPE) : kRegion;
+    auto load_raw = [&](uint32_t sb, Raw (&raw)[NJ]) {
+        const uint32_t so = sb * kBlkStep;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            if constexpr (Q4) {
+                raw[j].hdr = bload16(wsrc(j), voff[j], so);
+#pragma unroll
+                for (int p = 0; p < 4; ++p) raw[j].qs[p] = bload16(wsrc(j), voff[j] + chunk(hl), so + chunk(1 + 2 * p));
+            } else if constexpr (!ROW) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) raw[j].ql[c] = bload16(wsrc(j), voff[j] + chunk(hl), so + chunk(2 * c));
+#pragma unroll
+                for (int h = 0; h < 2; ++h) raw[j].qh[h] = bload16(wsrc(j), voff[j] + chunk(hl), so + chunk(8 + 2 * h));
+                raw[j].sc = bload16(wsrc(j), voff[j], so + chunk(12));
+                // d of row r: region + 13 KiB + 2*(r%64) = voff - 14*(r%64) + 13 KiB
+                raw[j].d = bload2(wsrc(j), voff[j] - 14 * (brow(j) % kRowTile), so + kQ6Chunks * 1024);
+            } else {
+                // 210-byte blocks: the dword-aligned address at or below each piece, five dwords
+                const uint32_t blk = voff[j] + so, al = blk & ~3u;
+                const uint32_t lo = al + 16 * hl;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    raw[j].ql[c] = bload16(wsrc(j), lo + 32 * c, 0);
+                    raw[j].x[c] = bload4(wsrc(j), lo + 32 * c + 16, 0);
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    raw[j].qh[h] = bload16(wsrc(j), lo + 128 + 32 * h, 0);
+                    raw[j].x[4 + h] = bload4(wsrc(j), lo + 128 + 32 * h + 16, 0);
+                }
+                raw[j].sc = bload16(wsrc(j), al + 192, 0);
+                raw[j].x[6] = bload4(wsrc(j), al + 208, 0);
+                raw[j].d = bload2(wsrc(j), blk + 208, 0);
+            }
+        }
+    };
+    // vector loads of load_raw: the x DMA issued before them has landed once only these are in flight
+    constexpr int kRawLoads = NJ * (Q4 ? 5 : ROW ? 15 : 8);
+    // ROW_MAJOR Q6_K: shift the five dwords of each piece down to the block's 2-byte alignment
+    auto fix_raw = [&](uint32_t sb, Raw (&raw)[NJ]) {
+        if constexpr (!Q4 && ROW) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const uint32_t sh = ((voff[j] + sb * kBlkStep) & 2u) * 8u;
+                auto shift = [&](u32x4 &v, uint32_t hi) {
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) v[i] = __builtin_amdgcn_alignbit(v[i + 1], v[i], sh);
+                    v[3] = __builtin_amdgcn_alignbit(hi, v[3], sh);
+                };
+#pragma unroll
+                for (int c = 0; c < 4; ++c) shift(raw[j].ql[c], raw[j].x[c]);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) shift(raw[j].qh[h], raw[j].x[4 + h]);
+                shift(raw[j].sc, raw[j].x[6]);
+            }
+        }
+    };
+
+    // ---- x staging: instruction i of wave wc fills rows (wc*ND + i)*RPI .. of group wk's tile; lane l
+    // writes position l%CR of row +l/CR and fetches the chunk that the swizzle puts there.
+    auto swz = [](uint32_t R) { return CR == 16 ? (R & 15) : ((R >> 1) & 7); };
+    uint32_t xoff[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+        const uint32_t R = (wc * ND + uint32_t(i)) * RPI + lane / CR, c = (lane % CR) ^ swz(R);
+        xoff[i] = ((t0 + R) * cols + 8 * c) * 2;
+    }
+    auto xbuf = [&](int b) -> u32x4 * { return b ? X1 : X0; };
+    auto dma_x = [&](uint32_t sb, int st) {
+        const uint32_t so = (sb * kQK + uint32_t(st) * KS) * 2;
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+            dma16(xsrc, xbuf(st & 1) + wk * (TT * CR) + (wc * ND + uint32_t(i)) * 64, xoff[i], so);
+    };
+    // A fragment of token tile i: row 32i + ln, chunk 4*gq + 2*hl + e of the stage
+    const uint32_t a0 = wk * (TT * CR) + ln * CR, asw = (2 * hl) ^ swz(ln);
+    auto load_a = [&](int b, int i, int gq, int e) -> half8_t {
+        return __builtin_bit_cast(half8_t, xbuf(b)[a0 + uint32_t(i) * 32 * CR + ((4 * gq + e) ^ asw)]);
+    };
+
+    // ---- prologue: the first super-block in flight, then (FP16 mode) the row scales
+    auto sb_of = [&](uint32_t it) { return __builtin_elementwise_min(sb0 + it * WK + wk, sb1 - 1); };
+    Raw raw[NJ];
+    float c24[NJ], inv_c[NJ];
+    auto first_loads = [&]() {  // in this order: the main loop's first wait counts the raw loads
+        dma_x(sb_of(0), 0);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_sched_barrier(0);
+        load_raw(sb_of(0), raw);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (F16) {
+        // this wave's share of the rows' block factors: super-blocks 2*(wk + WK*u) + hl
+        float M[NJ] = {};
+        for (uint32_t u0 = 0; 2 * WK * u0 < nb; u0 += 2) {
+            uint32_t dd[2][NJ];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const uint32_t b = __builtin_elementwise_min(2 * (wk + WK * (u0 + uint32_t(u))) + hl, nb - 1);
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    if constexpr (Q4) dd[u][j] = bload4(wsrc(j), voff[j] + b * kBlkStep, 0);
+                    else dd[u][j] = bload2(wsrc(j), voff[j] - 14 * (brow(j) % kRowTile) + b * kBlkStep + kQ6Chunks * 1024, 0);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    const float m = __builtin_fabsf(lo_half(dd[u][j]));
+                    M[j] = __builtin_fmaxf(M[j], Q4 ? __builtin_fmaxf(m, __builtin_fabsf(hi_half(dd[u][j]))) : m);
+                }
+            if (u0 == 0) first_loads();  // behind the first factors
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            M[j] = __builtin_fmaxf(M[j], __shfl_xor(M[j], 32));
+            if (hl == 0) rmax[wave][j][ln] = M[j];
+        }
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            float m = 0.f;
+#pragma unroll
+            for (int k = 0; k < WK; ++k) m = __builtin_fmaxf(m, rmax[uint32_t(k) * WC + wc][j][ln]);
+            row_scale(m, c24[j], inv_c[j], !Q4);
+        }
+    } else {
+        first_loads();
+    }
+
+    float16_t acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+    // ---- per super-block factors of column j, and its fragments (group grp, e)
+    struct Factors {
+        half2_t A[NJ][8], B[NJ][8];  // per group; Q4_K FP32 mode: A alone
+    };
+    auto factors = [&](const Raw (&r)[NJ], Factors &F) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            if constexpr (Q4) {
+                const Q4Scales sc = q4_scales(r[j].hdr.y, r[j].hdr.z, r[j].hdr.w);
+                if constexpr (F16) {
+                    const float dc = lo_half(r[j].hdr.x) * c24[j];
+                    const float mc = -hi_half(r[j].hdr.x) * (c24[j] * 5.9604644775390625e-08f);  // c = c24 * 2^-24
+#pragma unroll
+                    for (int gg = 0; gg < 8; ++gg) {
+                        F.A[j][gg] = splat(_Float16(dc * float(q4_sc(sc, gg))));
+                        F.B[j][gg] = splat(_Float16(mc * float(q4_m(sc, gg))));
+                    }
+                } else {
+                    // q*2^-24 (low nibbles) or 16q*2^-24 (high) times this = sc*q*2^-14, exact
+#pragma unroll
+                    for (int gg = 0; gg < 8; ++gg)
+                        F.A[j][gg] = splat(_Float16(float(q4_sc(sc, gg)) * (gg & 1 ? 64.0f : 1024.0f)));
+                }
+            } else {
+                const float d = lo_half(r[j].d);
+#pragma unroll
+                for (int gg = 0; gg < 8; ++gg) {
+                    // group gg = 4h + Q of this lane half: scale 8h + 2Q + hl
+                    const int sc = int8_t(byte_of(r[j].sc[gg >> 1] >> (8 * hl), 2 * (gg & 1)));
+                    if constexpr (F16) {
+                        const float dc = d * c24[j], dm = -32.0f * d * (c24[j] * 5.9604644775390625e-08f);
+                        F.A[j][gg] = splat(_Float16(dc * float(sc)));
+                        F.B[j][gg] = splat(_Float16(dm * float(sc)));
+                    } else {
+                        // v*2^-24 * sc*2^8 - sc*2^-11 = sc*(v-32)*2^-16
+                        F.A[j][gg] = splat(_Float16(float(sc) * 256.0f));
+                        F.B[j][gg] = splat(_Float16(float(sc) * -0.00048828125f));
+                    }
+                }
+            }
+        }
+    };
+    auto frag = [&](const Raw &r, const half2_t (&A)[8], const half2_t (&B)[8], int grp, int e) -> half8_t {
+        u32x4 f;
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            if constexpr (Q4) {
+                const uint32_t w = r.qs[grp >> 1][2 * e + d];
+                const uint32_t p = __builtin_amdgcn_perm(w, w, 0x03010200u);  // bytes [b0, b2, b1, b3]
+                if constexpr (F16) {
+                    const uint32_t s = grp & 1 ? 4 : 0;
+                    f[2 * d] = bits(__builtin_elementwise_fma(h2((p >> s) & 0x000F000Fu), A[grp], B[grp]));
+                    f[2 * d + 1] = bits(__builtin_elementwise_fma(h2((p >> (8 + s)) & 0x000F000Fu), A[grp], B[grp]));
+                } else {
+                    const uint32_t m = grp & 1 ? 0x00F000F0u : 0x000F000Fu;
+                    f[2 * d] = bits(h2(p & m) * A[grp]);
+                    f[2 * d + 1] = bits(h2((p >> 8) & m) * A[grp]);
+                }
+            } else {
+                const int h = grp >> 2, Q = grp & 3;
+                const uint32_t ql = r.ql[2 * h + (Q & 1)][2 * e + d], qh = r.qh[h][2 * e + d];
+                const uint32_t lo4 = (Q >= 2 ? ql >> 4 : ql) & 0x0F0F0F0Fu;
+                const uint32_t hb = Q == 0 ? qh << 4 : Q == 1 ? qh << 2 : Q == 2 ? qh : qh >> 2;
+                uint32_t o[2];
+                q6_f16x4(lo4 | (hb & 0x30303030u), A[grp], B[grp], o);
+                f[2 * d] = o[0];
+                f[2 * d + 1] = o[1];
+            }
+        }
+        return __builtin_bit_cast(half8_t, f);
+    };
+    auto mfma = [](half8_t x, half8_t w, const float16_t &c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(x, w, c, 0, 0, 0); };
+
+    // ---- main loop.  Stage s = (iteration, st): x(s) has been requested one stage earlier and, at
+    // st 0, the super-block's raw blocks during the last stage of the iteration before.  Wait for
+    // this wave's share of x(s) (leaving the raw loads issued after it in flight), meet the other
+    // waves of the column groups at the barrier (which also puts every read of buffer (s+1) % 2, at
+    // stage s-1, before the DMA that refills it), request x(s+1), then compute.
+    constexpr bool kMin = Q4 && !F16;
+    for (uint32_t it = 0; it < iters; ++it) {
+        const bool valid = sb0 + it * WK + wk < sb1;  // wave-uniform
+        const uint32_t sb = sb_of(it), sbn = sb_of(it + 1);
+        Factors F;
+        float16_t S[F16 ? 1 : MI][NJ];
+        float P[kMin ? MI : 1][8];
+#pragma unroll
+        for (int st = 0; st < NS; ++st) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (st == 0) vm_wait<kRawLoads>();
+            else vm_wait<0>();
+            if constexpr (WC > 1) bare_barrier();
+            else __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            if (st + 1 < NS) dma_x(sb, st + 1);
+            else dma_x(sbn, 0);
+            if (st == 0) {
+                // the factors are formed here, behind the DMA: without the pin the compiler hoists
+                // them, and their wait for the raw blocks, above the barrier
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    if constexpr (Q4) asm volatile("" : "+v"(raw[j].hdr));
+                    else asm volatile("" : "+v"(raw[j].sc), "+v"(raw[j].d));
+                }
+                fix_raw(sb, raw);
+                factors(raw, F);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (valid) {
+#pragma unroll
+                for (int gq = 0; gq < KS / 32; ++gq) {
+                    const int grp = st * (KS / 32) + gq;
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        half8_t av[MI], fb[NJ];
+#pragma unroll
+                        for (int i = 0; i < MI; ++i) av[i] = load_a(st & 1, i, gq, e);
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) fb[j] = frag(raw[j], F.A[j], F.B[j], grp, e);
+#pragma unroll
+                        for (int i = 0; i < MI; ++i) {
+                            if constexpr (kMin) {
+                                float p = e == 0 ? 0.f : P[i][grp];
+#pragma unroll
+                                for (int k = 0; k < 8; ++k) p += float(av[i][k]);
+                                P[i][grp] = p;
+                            }
+#pragma unroll
+                            for (int j = 0; j < NJ; ++j) {
+                                if constexpr (F16) acc[i][j] = mfma(av[i], fb[j], acc[i][j]);
+                                else S[i][j] = mfma(av[i], fb[j], grp == 0 && e == 0 ? float16_t{} : S[i][j]);
+                            }
+                        }
+                    }
+                }
+            }
+        }
+        float d[NJ], dmin[NJ];
+        bf8_t mb[NJ];
+        if constexpr (!F16) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                if constexpr (Q4) {
+                    d[j] = lo_half(raw[j].hdr.x) * 16384.0f;
+                    dmin[j] = hi_half(raw[j].hdr.x);
+                    const Q4Scales sc = q4_scales(raw[j].hdr.y, raw[j].hdr.z, raw[j].hdr.w);
+                    u32x4 m;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)  // bf16 of an integer below 64: the upper half of its fp32
+                        m[k] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, float(q4_m(sc, 2 * k + 1))),
+                                                     __builtin_bit_cast(uint32_t, float(q4_m(sc, 2 * k))), 0x07060302u);
+                    // formed before the next blocks are requested: a header still in use would be loaded
+                    // elsewhere and copied, which waits for the load just issued
+                    asm volatile("" : "+v"(d[j]), "+v"(dmin[j]), "+v"(m));
+                    mb[j] = __builtin_bit_cast(bf8_t, m);
+                } else {
+                    d[j] = lo_half(raw[j].d) * 65536.0f;
+                    asm volatile("" : "+v"(d[j]));
+                }
+            }
+        }
+        // the raw blocks are consumed: request the next super-block's (clamped, also past the last)
+        __builtin_amdgcn_sched_barrier(0);
+        load_raw(sbn, raw);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!F16) {
+            if (valid) {
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_fmaf(d[j], S[i][j][v], acc[i][j][v]);
+                    if constexpr (kMin) {
+                        // P = hi + mid + lo, each exact in bf16 (8 of the 24 bits at a time)
+                        u32x4 pc[3];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            uint32_t pb[3][2];
+#pragma unroll
+                            for (int u = 0; u < 2; ++u) {
+                                float r = P[i][2 * k + u];
+#pragma unroll
+                                for (int z = 0; z < 3; ++z) {
+                                    pb[z][u] = __builtin_bit_cast(uint32_t, r) & 0xffff0000u;
+                                    r -= __builtin_bit_cast(float, pb[z][u]);
+                                }
+                            }
+#pragma unroll
+                            for (int z = 0; z < 3; ++z) pc[z][k] = __builtin_amdgcn_perm(pb[z][1], pb[z][0], 0x07060302u);
+                        }
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) {
+                            float16_t mn{};
+#pragma unroll
+                            for (int z = 0; z < 3; ++z)
+                                mn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8_t, pc[z]), mb[j], mn, 0, 0, 0);
+#pragma unroll
+                            for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_fmaf(-dmin[j], mn[v], acc[i][j][v]);
+                        }
+                    }
+                }
+            }
+        }
+    }
+    // Nothing may land in the buffers the sums now go through, and every wave is past its reads.
+    vm_wait<0>();
+    bare_barrier();
+
+    // ---- the WK partial sums of each column group: wave wk finishes elements v = wk*VP .. +VP-1 of
+    // every tile (32x32 D layout: lane holds column ln and token 8*(v/4) + 4*hl + v%4)
+    constexpr int VP = 16 / WK;
+    float fin[MI][VP][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        float *red = reinterpret_cast<float *>(xbuf(i & 1));  // [wave][v][j][64]
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) red[((wave * 16 + v) * NJ + j) * 64 + lane] = acc[i][j][v];
+        lds_barrier();
+#pragma unroll
+        for (int u = 0; u < VP; ++u)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                float s = 0.f;
+#pragma unroll
+                for (int k = 0; k < WK; ++k) s += red[(((uint32_t(k) * WC + wc) * 16 + wk * VP + u) * NJ + j) * 64 + lane];
+                fin[i][u][j] = F16 ? s * inv_c[j] : s;
+            }
+    }
+
+    auto write_out = [&]() {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int u = 0; u < VP; ++u) {
+                const uint32_t v = wk * VP + uint32_t(u), t = t0 + uint32_t(i) * 32 + 8 * (v >> 2) + 4 * hl + (v & 3);
+                if (t >= batch) continue;
+                if constexpr (PAIR) {
+                    const uint32_t r = brow(0);
+                    const float gv = F16 ? round_f16p(fin[i][u][0]) : fin[i][u][0];
+                    const float uv = F16 ? round_f16p(fin[i][u][1]) : fin[i][u][1];
+                    if (r < rows) static_cast<_Float16 *>(a.out[0])[size_t(t) * rows + r] = _Float16(gelu_tanh(gv) * uv);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) {
+                        const uint32_t r = brow(j);
+                        if (r < rows)
+                            static_cast<float *>(a.out[seg])[size_t(t) * rows + r] = F16 ? round_f16p(fin[i][u][j]) : fin[i][u][j];
+                    }
+                }
+            }
+    };
+    if (kparts == 1) {
+        write_out();
+        return;
+    }
+
+    // ---- split K over workgroups: parts [tile][kp][i][u][j][thread], added by the last to arrive.
+    // Device-coherent atomic stores and loads; the wait completes them before the arrival counts.
+    constexpr uint32_t kPart = MI * VP * NJ * kThreads;
+    float *mine = a.partial + (size_t(tile) * kparts + kp) * kPart;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int u = 0; u < VP; ++u)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+                __hip_atomic_store(&mine[((i * VP + u) * NJ + j) * kThreads + tid], fin[i][u][j], __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __syncthreads();
+    if (tid == 0)
+        last_flag = __hip_atomic_fetch_add(&a.counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kparts - 1;
+    __syncthreads();
+    if (!last_flag) return;
+    if (tid == 0) __hip_atomic_store(&a.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const float *parts = a.partial + size_t(tile) * kparts * kPart;
+    for (uint32_t p0 = 0; p0 < kparts; p0 += 4) {  // four parts per round trip, added in part order
+        float pv[4][MI][VP][NJ];
+#pragma unroll
+        for (int z = 0; z < 4; ++z) {
+            const float *p = parts + size_t(__builtin_elementwise_min(p0 + uint32_t(z), kparts - 1)) * kPart;
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int u = 0; u < VP; ++u)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+                        pv[z][i][u][j] = __hip_atomic_load(&p[((i * VP + u) * NJ + j) * kThreads + tid], __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int u = 0; u < VP; ++u)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    float s = p0 == 0 ? 0.f : fin[i][u][j];
+#pragma unroll
+                    for (int z = 0; z < 4; ++z) s = p0 + uint32_t(z) < kparts ? s + pv[z][i][u][j] : s;
+                    fin[i][u][j] = s;
+                }
+    }
+    write_out();
+}
+
+struct Plan {
+    uint32_t mi, wk, ntok, ncol, kparts;
+    uint32_t cost;  // the model's estimate, tenths of a microsecond
+};
+
+int device_cus() {
+    static int cache[64] = {};
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    int &n = cache[dev & 63];
+    if (n == 0 && (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)) n = 256;
+    return n;
+}
+
+uint32_t col_tiles(const uint32_t *rows, int nseg, bool pair, uint32_t wk) {
+    const uint32_t per = (kWaves / wk) * (pair ? 32 : 64);
+    uint32_t n = 0;
+    for (int s = 0; s < nseg; ++s) n += (rows[s] + per - 1) / per;
+    return n;
+}
+
+// Token tile, wave split and split K, by a cost model in tenths of a microsecond fitted to MI355X
+// timings of the gate/up pair, the down projections and 2,048- and 4,096-row projections at 5 to 512
+// tokens (within ~10% of them).  A call costs ~6 us of launch, ramp and tail; each round of workgroups
+// (one per CU) ~6 us more and, per super-block a wave walks, kIter[kind][MI]: bound by the weight
+// bytes at 32 tokens, by the matrix and decode work above.  Splitting K over workgroups (only to fill
+// the first round) adds the hand-off, whose last arrival reads every part.
+Plan plan_skinny(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair, bool f16,
+                 const Tuning &t) {
+    static constexpr uint32_t kIter[3][3] = {{25, 45, 0}, {22, 38, 0}, {23, 36, 71}};  // FP32 Q4_K, FP32 Q6_K, FP16
+    const uint32_t *iter_cost = kIter[f16 ? 2 : type == Q6_K ? 1 : 0];
+    Plan best{};
+    const uint32_t nb = cols / kQK, cus = uint32_t(device_cus());
+    const uint32_t forced = t.gemm_kparts >= 1 && uint32_t(t.gemm_kparts) <= nb ? uint32_t(t.gemm_kparts) : 0;
+    uint32_t best_cost = ~0u;
+    for (uint32_t m = 0; m < (f16 ? 3u : 2u); ++m) {
+        const uint32_t mi = 1u << m, ntok = (batch + 32 * mi - 1) / (32 * mi);
+        // without a forced tile: the shortest one that holds the batch, or a shorter one
+        if (t.skinny_mi > 0 ? mi != uint32_t(t.skinny_mi) : m > 0 && batch <= 16 * mi) continue;
+        for (uint32_t wk : {4u, 8u}) {
+            if (wk == 8 && mi == 4) continue;  // no room for its x stages
+            if (t.skinny_wk > 0 && uint32_t(t.skinny_wk) != wk && mi < 4) continue;
+            const uint32_t ncol = col_tiles(rows, nseg, pair, wk), tiles = ncol * ntok;
+            for (uint32_t kp = forced ? forced : 1; kp <= nb && (forced ? kp == forced : kp == 1 || tiles * kp <= cus); ++kp) {
+                const uint32_t rounds = (tiles * kp + cus - 1) / cus, iters = ((nb + kp - 1) / kp + wk - 1) / wk;
+                const uint32_t cost = 60 + rounds * (60 + iters * iter_cost[m]) + (kp > 1 ? 10 + 4 * kp * mi : 0);
+                if (cost < best_cost) {
+                    best_cost = cost;
+                    best = Plan{mi, wk, ntok, ncol, kp, cost};
+                }
+            }
+        }
+    }
+    if (best.wk == 0) {  // a forced tile this mode does not have
+        Tuning plain = t;
+        plain.skinny_mi = plain.skinny_wk = 0;
+        return plan_skinny(type, cols, rows, nseg, batch, pair, f16, plain);
+    }
+    return best;
+}
+
+template <int TYPE, int LAYOUT, int ACC, bool PAIR>
+hipError_t launch_mi(const Plan &p, const Args &a, hipStream_t stream) {
+    const dim3 grid(p.ntok * p.ncol * p.kparts), block(kThreads);
+    if (p.mi == 1) {
+        if (p.wk == 8) gemm_skinny_kernel<TYPE, LAYOUT, ACC, PAIR, 1, 8><<<grid, block, 0, stream>>>(a);
+        else gemm_skinny_kernel<TYPE, LAYOUT, ACC, PAIR, 1, 4><<<grid, block, 0, stream>>>(a);
+    } else if (p.mi == 2) {
+        if (p.wk == 8) gemm_skinny_kernel<TYPE, LAYOUT, ACC, PAIR, 2, 8><<<grid, block, 0, stream>>>(a);
+        else gemm_skinny_kernel<TYPE, LAYOUT, ACC, PAIR, 2, 4><<<grid, block, 0, stream>>>(a);
+    } else {
+        if constexpr (ACC == ACC_FP16) gemm_skinny_kernel<TYPE, LAYOUT, ACC, PAIR, 4, 4><<<grid, block, 0, stream>>>(a);
+        else return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+// Whether this kernel is the faster one: a bound on the plan's estimate.  The 128- and 256-token
+// tile kernels need many output tiles to fill the device and then cost ~90-115 us; below that they
+// take as long.  MI355X, this kernel against them (us), each bound from both sides:
+//   gate/up FP16   384 tokens: 110 / 114,             512: 145 / 114
+//   gate/up FP32   192: 81 / 94,                      225: 106 / 95
+//   downs          512: 73-96 / 78-127,               775: 157-180 / 134-145, FP16 1024: 137 / 127
+//   4096 x 3840    1536: 89 / 114, row-major 93 / 95;   2048: 121 / 103, row-major 125 / 106
+// A row-major Q6_K tensor runs at 260-273 us at any batch there (2-byte loads) and at 42-80 us here
+// for 2,048 rows at 1,024-2,048 tokens.
+bool gemm_skinny_eligible(int type, int layout, int acc, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch,
+                          bool pair, const Tuning &t) {
+    if (t.gemm_skinny == 0) return false;
+    if (layout == NSMFFN || (layout == ROW_MAJOR && (acc == ACC_FP16 || pair))) return false;
+    if (t.gemm_skinny > 0) return batch <= uint32_t(t.gemm_skinny);
+    if (t.gemm_q4_reg == 0 && type == Q4_K && acc == ACC_FP32) return false;  // the LDS-tile kernel is asked for
+    if (batch > 2048) return false;  // beyond what was measured
+    uint32_t tiles = 0;  // 256 tokens x 256 columns
+    for (int s = 0; s < nseg; ++s) tiles += (batch + 255) / 256 * ((rows[s] * (pair ? 2 : 1) + 255) / 256);
+    const uint32_t cost = plan_skinny(type, cols, rows, nseg, batch, pair, acc == ACC_FP16, t).cost;
+    return cost <= (layout == ROW_MAJOR && type == Q6_K ? 2600u : acc == ACC_FP16 && tiles >= 96 ? 1100u : 960u);
+}
+
+void gemm_skinny_workspace_need(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair,
+                                int acc, const Tuning &t, size_t *part_floats, size_t *counters) {
+    const Plan p = plan_skinny(type, cols, rows, nseg, batch, pair, acc == ACC_FP16, t);
+    const size_t tiles = size_t(p.ncol) * p.ntok;
+    *part_floats = p.kparts > 1 ? tiles * p.kparts * (p.mi * 32 * (kWaves / p.wk) * 64) : 0;
+    *counters = p.kparts > 1 ? tiles : 0;
+}
+
+hipError_t launch_gemm_skinny(int type, int layout, int acc, const uint8_t *const *w, const uint8_t *up, void *const *out,
+                              const uint32_t *rows, int nseg, const uint16_t *x, uint32_t cols, uint32_t batch,
+                              float *partial, uint32_t *counters, const Tuning &t, hipStream_t stream) {
+    const bool pair = up != nullptr, f16 = acc == ACC_FP16;
+    if (nseg < 1 || nseg > kMaxSeg || (pair && nseg != 1)) return hipErrorInvalidValue;
+    const Plan p = plan_skinny(type, cols, rows, nseg, batch, pair, f16, t);
+    Args a{};
+    uint32_t ct = 0;
+    for (int s = 0; s < kMaxSeg; ++s) {
+        const int z = s < nseg ? s : nseg - 1;
+        a.w[s] = w[z];
+        a.out[s] = out[z];
+        a.rows[s] = rows[z];
+        if (s < nseg) ct += col_tiles(rows + s, 1, pair, p.wk);
+        a.ct_end[s] = ct;
+    }
+    a.up = up;
+    a.x = x;
+    a.partial = partial;
+    a.counters = counters;
+    a.cols = cols;
+    a.batch = batch;
+    a.ntok = p.ntok;
+    a.ncol = p.ncol;
+    a.kparts = p.kparts;
+    if (layout == CDNA4) {
+        if (pair)
+            return f16 ? launch_mi<Q4_K, CDNA4, ACC_FP16, true>(p, a, stream) : launch_mi<Q4_K, CDNA4, ACC_FP32, true>(p, a, stream);
+        if (type == Q4_K)
+            return f16 ? launch_mi<Q4_K, CDNA4, ACC_FP16, false>(p, a, stream) : launch_mi<Q4_K, CDNA4, ACC_FP32, false>(p, a, stream);
+        return f16 ? launch_mi<Q6_K, CDNA4, ACC_FP16, false>(p, a, stream) : launch_mi<Q6_K, CDNA4, ACC_FP32, false>(p, a, stream);
+    }
+    if (layout != ROW_MAJOR || f16 || pair) return hipErrorInvalidValue;
+    return type == Q4_K ? launch_mi<Q4_K, ROW_MAJOR, ACC_FP32, false>(p, a, stream)
+                        : launch_mi<Q6_K, ROW_MAJOR, ACC_FP32, false>(p, a, stream);
+}
+
+}  // namespace ns

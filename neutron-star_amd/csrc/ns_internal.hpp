@@ -30,6 +30,9 @@ struct Tuning {
     int block_spin = 0;   // > 0: that launch's bound on a down workgroup's wait (polls)
     int gemm_rs = 1;      // 0: split-K FP16-mode GEMMs finish by the last arrival; > 1: reduce-scatter wait bound
     int wait_free = 0;    // 1 (ns_ctx_set_wait_free): no kernel waits for another workgroup
+    int gemm_skinny = -1; // -1: plan; 0: never the few-token GEMM; > 0: up to this many tokens
+    int skinny_wk = 0;    // 4 / 8: its groups of super-blocks per workgroup
+    int skinny_mi = 0;    // 1 / 2 / 4: its token tile, in 32-token units
     int stack_fused = 1;  // 0: the multi-layer decode as one block launch per layer
 };
 
@@ -176,6 +179,17 @@ void gemm_f16_workspace_need(uint32_t cols, uint32_t rows, uint32_t batch, bool 
 hipError_t launch_gemm_f16(int type, const uint8_t *w, const uint8_t *up, const uint16_t *x, void *out, uint32_t cols,
                            uint32_t rows, uint32_t batch, float *partial, uint32_t *counters, uint32_t *err,
                            const Tuning &t, hipStream_t stream);
+
+// The prefill GEMM for few tokens (ns_gemm_skinny.hip): CDNA4 in both modes, ROW_MAJOR in the FP32
+// mode without the pair.  Up to three matrices of one type that share x (rows, w and out arrays
+// of nseg entries) in one launch; with `up` the gate/up pair (nseg 1).
+bool gemm_skinny_eligible(int type, int layout, int acc, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch,
+                          bool pair, const Tuning &t);
+void gemm_skinny_workspace_need(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair,
+                                int acc, const Tuning &t, size_t *part_floats, size_t *counters);
+hipError_t launch_gemm_skinny(int type, int layout, int acc, const uint8_t *const *w, const uint8_t *up, void *const *out,
+                              const uint32_t *rows, int nseg, const uint16_t *x, uint32_t cols, uint32_t batch,
+                              float *partial, uint32_t *counters, const Tuning &t, hipStream_t stream);
 
 // Prefill GEMM over fp16 x [batch][cols]: plain (fp32 out [batch][rows]) or the
 // gate/up pair with GeGLU (fp16 h [batch][rows]).

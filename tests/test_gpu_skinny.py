@@ -1,0 +1,102 @@
+"""The prefill GEMM for few tokens (csrc/ns_gemm_skinny.hip) against the oracle, at the edges of its
+tiles: one token past a 32-token tile and the largest batch of each tile height, a last column tile
+that is partly past the rows, more super-block groups than super-blocks and a remainder of them,
+split K over workgroups, both wave splits (4 or 8 super-block groups).
+
+Bars: the repository's 1e-3 (FP32 mode) and, against the FP16-mode oracle, 1e-3 (5e-3 for the
+pair, whose h is fp16 of a product of two rounded sums).
+"""
+import numpy as np
+import pytest
+
+import ns_oracle as O
+import nsffn as N
+from helpers import f16_value, rel_err
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+LNAME = {N.CDNA4: "cdna4", N.ROW_MAJOR: "rowmajor"}
+# (rows, cols, batch): tiles of 32, 64 and 128 tokens, 1 to 17 super-blocks
+SHAPES = [(64, 256, 5), (192, 768, 32), (320, 1024, 33), (128, 2304, 64), (192, 1280, 65), (64, 4352, 128)]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    assert torch.cuda.is_available(), "GPU tests need a visible MI355X"
+    c = N.Context(0)
+    yield c
+    torch.cuda.synchronize()
+    c.close()
+
+
+def weights(qtype, seed, rows, cols, layout):
+    host = N.synth_weights(qtype, seed, rows, cols)
+    lay = host if layout == N.ROW_MAJOR else N.retile(host, qtype, cols, rows, N.ROW_MAJOR, layout)
+    return host, torch.from_numpy(np.ascontiguousarray(lay)).cuda()
+
+
+def tokens(seed, batch, cols):
+    bits = N.synth_normal_f16(seed, batch * cols).reshape(batch, cols)
+    return bits, torch.from_numpy(bits.view(np.int16)).cuda()
+
+
+@pytest.mark.parametrize("wk,kparts", [(4, 1), (8, 1), (4, 3), (8, 2), (0, 0)],
+                         ids=["wk4", "wk8", "wk4_split3", "wk8_split2", "plan"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("qtype", [N.Q4_K, N.Q6_K], ids=["q4k", "q6k"])
+@pytest.mark.parametrize("mode", ["fp32_cdna4", "fp16_cdna4", "fp32_rowmajor"])
+def test_skinny_matmul(ctx, tune, mode, qtype, shape, wk, kparts):
+    rows, cols, batch = shape
+    layout, fast = (N.ROW_MAJOR if mode.endswith("rowmajor") else N.CDNA4), mode.startswith("fp16")
+    if layout == N.ROW_MAJOR:
+        rows -= 11  # ragged: the row-major layout has no 64-row rule
+    tune("gemm_skinny", 128)
+    tune("skinny_wk", wk)
+    tune("gemm_kparts", min(kparts, cols // 256))
+    host, w = weights(qtype, 0x51, rows, cols, layout)
+    bits, x = tokens(0x52, batch, cols)
+    y = torch.full((batch + 1, rows), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.ffn_down(w, qtype, layout, cols, rows, batch, x, y, half_input=True, fast_swa=fast)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert np.isnan(got[batch]).all()  # nothing past the batch is written
+    ref = O.gemm(qtype, O.ROW_MAJOR, host, cols, rows, batch, bits, 1 if fast else 0)
+    assert rel_err(got[:batch], ref) <= 1e-3
+
+
+@pytest.mark.parametrize("wk,kparts", [(4, 1), (8, 2), (0, 0)], ids=["wk4", "wk8_split2", "plan"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("fast", [False, True], ids=["fp32", "fp16"])
+def test_skinny_gate_up(ctx, tune, fast, shape, wk, kparts):
+    rows, cols, batch = shape
+    tune("gemm_skinny", 128)
+    tune("skinny_wk", wk)
+    tune("gemm_kparts", min(kparts, cols // 256))
+    hg, wg = weights(N.Q4_K, 0x53, rows, cols, N.CDNA4)
+    hu, wu = weights(N.Q4_K, 0x54, rows, cols, N.CDNA4)
+    bits, x = tokens(0x55, batch, cols)
+    h = torch.full((batch + 1, rows), 0x7E00, dtype=torch.int16, device="cuda")
+    ctx.gate_up_geglu_rm32(wg, wu, N.CDNA4, cols, rows, batch, x, h, fast)
+    torch.cuda.synchronize()
+    got = h.cpu().numpy()
+    assert (got[batch] == 0x7E00).all()
+    ref = O.gate_up_geglu_prefill(O.ROW_MAJOR, hg, hu, cols, rows, batch, bits, 1 if fast else 0)
+    assert rel_err(f16_value(got[:batch].view(np.uint16)), ref) <= (5e-3 if fast else 1e-3)
+
+
+def test_skinny_exact_min_term_and_large_sums(ctx, tune):
+    """FP32 mode, blocks with d = 0 (the output is the min term alone) on activations whose 32-wide
+    groups sum past fp16's range: the three-piece group sums lose nothing (float64 closed form)."""
+    tune("gemm_skinny", 128)
+    cols, rows, batch = 768, 64, 40
+    host = N.synth_weights(N.Q4_K, 0x56, rows, cols).copy()
+    host.reshape(-1, 144)[:, 0:2] = 0
+    w = torch.from_numpy(N.retile(host, N.Q4_K, cols, rows, N.ROW_MAJOR, N.CDNA4)).cuda()
+    x = (np.random.RandomState(7).randn(batch, cols) * 3.0 + 2100.0).astype(np.float16)
+    y = torch.empty((batch, rows), dtype=torch.float32, device="cuda")
+    ctx.matmul(w, N.Q4_K, N.CDNA4, cols, rows, batch, torch.from_numpy(x.view(np.int16)).cuda(), y, half_input=True)
+    torch.cuda.synchronize()
+    want = x.astype(np.float64) @ O.dequant_rows(N.Q4_K, O.ROW_MAJOR, host, cols, rows, 0, rows).astype(np.float64).T
+    # 24 block groups of exact products, each sum and product rounded to 24 bits
+    assert rel_err(y.cpu().numpy(), want) <= 64 * 2.0 ** -24
