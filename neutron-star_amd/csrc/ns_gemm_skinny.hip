@@ -156,9 +156,8 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
         else return ct * kRowsPerTile + wc * 64 + uint32_t(j) * 32 + ln;
     };
     const uint32_t wbytes = rows * nb * block_bytes(TYPE);
-    const rsrc_t wsrc0 = make_rsrc(a.w[seg], wbytes), wsrc1 = make_rsrc(PAIR ? a.up : a.w[seg], wbytes);
-    auto wsrc = [&](int j) { return (PAIR && j == 1) ? wsrc1 : wsrc0; };
-    const rsrc_t xsrc = make_rsrc(a.x, batch * cols * 2);
+    const uint8_t *const w0 = a.w[seg], *const w1 = PAIR ? a.up : a.w[seg];
+    const uint32_t xbytes = batch * cols * 2;
 
     // ---- weight addressing: the lane's part is a VGPR, the super-block's a uniform offset.  Rows past
     // `rows` lie past the descriptor's range and read zeros.
@@ -172,8 +171,11 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
     // byte offset, past voff + the super-block's uniform part, of chunk c
     auto chunk = [](uint32_t c) { return c * (ROW ? 16u : 1024u); };
     constexpr uint32_t kBlkStep = ROW ? block_bytes(TYPE) : kRegion;
-    auto load_raw = [&](uint32_t sb, Raw (&raw)[NJ]) {
+    // live = 0: a range of no bytes, so the loads read zeros and touch no memory (past the last block)
+    auto load_raw = [&](uint32_t sb, bool live, Raw (&raw)[NJ]) {
         const uint32_t so = sb * kBlkStep;
+        const rsrc_t wsrc0 = make_rsrc(w0, live ? wbytes : 0), wsrc1 = make_rsrc(w1, live ? wbytes : 0);
+        auto wsrc = [&](int j) { return (PAIR && j == 1) ? wsrc1 : wsrc0; };
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             if constexpr (Q4) {
@@ -240,8 +242,9 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
         xoff[i] = ((t0 + R) * cols + 8 * c) * 2;
     }
     auto xbuf = [&](int b) -> u32x4 * { return b ? X1 : X0; };
-    auto dma_x = [&](uint32_t sb, int st) {
+    auto dma_x = [&](uint32_t sb, bool live, int st) {
         const uint32_t so = (sb * kQK + uint32_t(st) * KS) * 2;
+        const rsrc_t xsrc = make_rsrc(a.x, live ? xbytes : 0);
 #pragma unroll
         for (int i = 0; i < ND; ++i)
             dma16(xsrc, xbuf(st & 1) + wk * (TT * CR) + (wc * ND + uint32_t(i)) * 64, xoff[i], so);
@@ -253,19 +256,21 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
     };
 
     // ---- prologue: the first super-block in flight, then (FP16 mode) the row scales
-    auto sb_of = [&](uint32_t it) { return __builtin_elementwise_min(sb0 + it * WK + wk, sb1 - 1); };
+    auto sb_of = [&](uint32_t it) { return sb0 + it * WK + wk; };
     Raw raw[NJ];
     float c24[NJ], inv_c[NJ];
     auto first_loads = [&]() {  // in this order: the main loop's first wait counts the raw loads
-        dma_x(sb_of(0), 0);
+        dma_x(sb_of(0), sb_of(0) < sb1, 0);
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_sched_barrier(0);
-        load_raw(sb_of(0), raw);
+        load_raw(sb_of(0), sb_of(0) < sb1, raw);
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_sched_barrier(0);
     };
     if constexpr (F16) {
         // this wave's share of the rows' block factors: super-blocks 2*(wk + WK*u) + hl
+        const rsrc_t wsrc0 = make_rsrc(w0, wbytes), wsrc1 = make_rsrc(w1, wbytes);
+        auto wsrc = [&](int j) { return (PAIR && j == 1) ? wsrc1 : wsrc0; };
         float M[NJ] = {};
         for (uint32_t u0 = 0; 2 * WK * u0 < nb; u0 += 2) {
             uint32_t dd[2][NJ];
@@ -386,14 +391,16 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
     auto mfma = [](half8_t x, half8_t w, const float16_t &c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(x, w, c, 0, 0, 0); };
 
     // ---- main loop.  Stage s = (iteration, st): x(s) has been requested one stage earlier and, at
-    // st 0, the super-block's raw blocks during the last stage of the iteration before.  Wait for
+    // st 0, the super-block's raw blocks once those of the iteration before were consumed.  Wait for
     // this wave's share of x(s) (leaving the raw loads issued after it in flight), meet the other
     // waves of the column groups at the barrier (which also puts every read of buffer (s+1) % 2, at
-    // stage s-1, before the DMA that refills it), request x(s+1), then compute.
+    // stage s-1, before the DMA that refills it), request x(s+1), then compute.  (A second set of raw
+    // registers, filled one super-block earlier, changed nothing: 20.3 us either way for the FP16 pair
+    // at 5 tokens, and the FP32 pair took 23.0 instead of 21.5.)
     constexpr bool kMin = Q4 && !F16;
     for (uint32_t it = 0; it < iters; ++it) {
-        const bool valid = sb0 + it * WK + wk < sb1;  // wave-uniform
         const uint32_t sb = sb_of(it), sbn = sb_of(it + 1);
+        const bool valid = sb < sb1, more = sbn < sb1;  // wave-uniform
         Factors F;
         float16_t S[F16 ? 1 : MI][NJ];
         float P[kMin ? MI : 1][8];
@@ -404,8 +411,8 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
             else vm_wait<0>();
             if constexpr (WC > 1) bare_barrier();
             else __atomic_signal_fence(__ATOMIC_SEQ_CST);
-            if (st + 1 < NS) dma_x(sb, st + 1);
-            else dma_x(sbn, 0);
+            if (st + 1 < NS) dma_x(sb, valid, st + 1);
+            else dma_x(sbn, more, 0);
             if (st == 0) {
                 // the factors are formed here, behind the DMA: without the pin the compiler hoists
                 // them, and their wait for the raw blocks, above the barrier
@@ -471,9 +478,9 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
                 }
             }
         }
-        // the raw blocks are consumed: request the next super-block's (clamped, also past the last)
+        // the raw blocks are consumed: request the next super-block's
         __builtin_amdgcn_sched_barrier(0);
-        load_raw(sbn, raw);
+        load_raw(sbn, more, raw);
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (!F16) {
