@@ -30,6 +30,7 @@ struct Tuning {
     int block_spin = 0;   // > 0: that launch's bound on a down workgroup's wait (polls)
     int gemm_rs = 1;      // 0: split-K FP16-mode GEMMs finish by the last arrival; > 1: reduce-scatter wait bound
     int wait_free = 0;    // 1 (ns_ctx_set_wait_free): no kernel waits for another workgroup
+    int gemv_row = 1;     // 0: decode GEMVs on ROW_MAJOR tensors by the slab kernel
     int gemm_skinny = -1; // -1: plan; 0: never the few-token GEMM; > 0: up to this many tokens
     int skinny_wk = 0;    // 4 / 8: its groups of super-blocks per workgroup
     int skinny_mi = 0;    // 1 / 2 / 4: its token tile, in 32-token units
@@ -81,6 +82,12 @@ struct NormPrologue {
 hipError_t launch_gemv(int type, int layout, const uint8_t *w, const uint8_t *up,
                        const float *x, float *out, uint32_t cols, uint32_t rows,
                        const Workspace &ws, hipStream_t stream, const NormPrologue *np = nullptr);
+
+// Decode GEMV on ROW_MAJOR tensors with a row's blocks across the lanes (ns_gemv_row.hip);
+// launch_gemv routes there (plain, no NormPrologue) when eligible.
+bool gemv_row_eligible(int layout, uint32_t cols, const Tuning &t);
+hipError_t launch_gemv_row(int type, const uint8_t *w, const float *x, float *out, uint32_t cols, uint32_t rows,
+                           hipStream_t stream);
 
 // Required workspace for launch_gemv with these shapes.
 void gemv_workspace_need(int type, int layout, uint32_t cols, uint32_t rows, bool pair, const Tuning &t,

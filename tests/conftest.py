@@ -17,7 +17,8 @@ def pytest_configure(config):
 TUNING_DEFAULTS = {"gemv_pf": -1, "gemv_waves": 0, "gemv_whole": 1, "gemv_qslab": 1, "gemm_kparts": 0,
                    "gemm_q4_reg": 1, "mt_mfma": 1, "mt_parts": 0, "mt_slabs": 0, "mt_spw": 0, "block_fused": 1,
                    "block_spin": 0, "gemm_rs": 1, "stack_fused": 1, "gemm_skinny": -1,
-                   "skinny_wk": 0, "skinny_mi": 0}
+                   "skinny_wk": 0, "skinny_mi": 0,
+                   "gemv_row": 1}
 
 
 @pytest.fixture
