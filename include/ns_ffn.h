@@ -123,7 +123,9 @@ int ns_ctx_workspace_bytes(const ns_ctx *ctx, uint64_t *bytes);
  * FP16-mode prefill GEMMs finish by the last part to arrive instead of the
  * reduce-scatter; > 1: the reduce-scatter's bound on its wait), "gemm_skinny" (-1 plan, 0 never
  * the few-token prefill GEMM, > 0 up to that many tokens), "skinny_wk" (4 / 8) and "skinny_mi"
- * (1 / 2 / 4): its super-block groups and its token tile in 32-token units.  Results stay within
+ * (1 / 2 / 4): its super-block groups and its token tile in 32-token units, "f16_mi" (4 / 8): the
+ * FP16-mode prefill GEMM's token tile in 32-token units, "gemv_row" (0: decode GEMVs on row-major
+ * tensors by the slab kernel).  Results stay within
  * the same tolerances; engines leave the defaults. */
 int ns_ctx_set_tuning(ns_ctx *ctx, const char *key, int value);
 

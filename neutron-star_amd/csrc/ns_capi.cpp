@@ -288,6 +288,7 @@ extern "C" int ns_ctx_set_tuning(ns_ctx *ctx, const char *key, int value) {
     else if (k == "gemm_rs") t.gemm_rs = value;
     else if (k == "stack_fused") t.stack_fused = value;
     else if (k == "gemv_row") t.gemv_row = value;
+    else if (k == "f16_mi") t.f16_mi = value;
     else if (k == "gemm_skinny") t.gemm_skinny = value;
     else if (k == "skinny_wk") t.skinny_wk = value;
     else if (k == "skinny_mi") t.skinny_mi = value;

@@ -13,7 +13,8 @@
 // VALU work is the unpack and that FMA.
 //
 // Work split.  One workgroup = 4 waves, one wave per SIMD, one workgroup per CU
-// (128 KiB of LDS).  A workgroup computes 256 tokens x 256 B columns; each wave
+// (128 KiB of LDS).  A workgroup computes 256 tokens x 256 B columns (or 128 tokens, with half of
+// everything per token tile, where 256-token tiles are too few); each wave
 // owns all 256 tokens (8 MFMA tiles of v_mfma_f32_32x32x16_f16) and 64 columns
 // (2 tiles): for the gate/up pair, 32 gate rows and the same 32 up rows, so
 // GeGLU runs in registers.  The 256 fp32 accumulators of a wave live in AGPRs.
@@ -46,13 +47,10 @@ typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
-constexpr int TT = 256;               // tokens per workgroup (= per wave)
-constexpr int MI = TT / 32;           // 32-token MFMA tiles per wave
 constexpr int NJ = 2;                 // 32-column MFMA tiles per wave
 constexpr int TC = kWaves * NJ * 32;  // B columns per workgroup
 constexpr int KS = 64;                // k per step
 constexpr int XBUF = 4;               // x buffers in LDS (x streams three steps ahead)
-constexpr int XDMA = TT * KS * 2 / 16 / kThreads;  // 16-byte x chunks per thread per step
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, int(bytes), 0x00020000);
@@ -61,6 +59,11 @@ __device__ __forceinline__ u32x4 bload16(rsrc_t r, uint32_t off) { return __buil
 __device__ __forceinline__ u32x2 bload8(rsrc_t r, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b64(r, int(off), 0, 0); }
 __device__ __forceinline__ uint32_t bload4(rsrc_t r, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b32(r, int(off), 0, 0); }
 __device__ __forceinline__ uint32_t bload2(rsrc_t r, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b16(r, int(off), 0, 0); }
+
+// One LDS DMA instruction: 16 bytes per lane into the 1 KiB at lds.
+__device__ __forceinline__ void dma16(rsrc_t r, u32x4 *lds, uint32_t voff, uint32_t soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)lds, 16, voff, soff, 0, 0);
+}
 
 // s_waitcnt vmcnt(N) (gfx9 encoding: vmcnt bits 3:0 and 15:14; expcnt and lgkmcnt left at max).
 template <int N>
@@ -95,13 +98,17 @@ struct RawQ6 {
 };
 typedef unsigned int u32x3 __attribute__((ext_vector_type(3)));
 
-template <int TYPE, bool PAIR>
+// MI: 32-token MFMA tiles per wave (the workgroup's tokens / 32): 8, or 4 where 256-token tiles are too
+// few to fill the device (plan_f16).
+template <int TYPE, bool PAIR, int MI>
 __global__ __launch_bounds__(kThreads, 1) void gemm_f16_kernel(
     const uint8_t *__restrict__ w0, const uint8_t *__restrict__ w1, const uint16_t *__restrict__ x,
     void *__restrict__ out, float *__restrict__ partial, uint32_t *__restrict__ counters, uint32_t cols,
     uint32_t rows, uint32_t batch, uint32_t ntok_tiles, uint32_t ncol_tiles, uint32_t kparts, uint32_t wbytes,
     uint32_t rs_spin, uint32_t *__restrict__ err) {
     constexpr bool Q4 = TYPE == Q4_K;
+    constexpr int TT = 32 * MI;                        // tokens per workgroup (= per wave)
+    constexpr int XDMA = TT * KS * 2 / 16 / kThreads;  // 16-byte x chunks per thread per step
     using Raw = typename std::conditional<Q4, RawQ4, RawQ6>::type;
     // Four separate LDS objects rather than one array: the compiler then sees that a DMA into
     // one buffer cannot alias the fragment reads of another, and issues those reads without
@@ -222,9 +229,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_kernel(
     constexpr int kRawLoads = Q4 ? 3 * NJ : 8 * NJ;  // vector loads per load_raw
     // VALU instructions placed after each MFMA of a k16 sub-step (a scheduling hint: the
     // next step's fragment decode, ~24 (Q4_K) or ~36 (Q6_K) per sub-step)
-    constexpr int kValuPerMfma = Q4 ? 2 : 3;
+    constexpr int kValuPerMfma = (Q4 ? 2 : 3) * (8 / MI);
     // the first sub-step also carries the factors of the next step
-    constexpr int kValuFirst = Q4 ? 4 : 5;
+    constexpr int kValuFirst = (Q4 ? 4 : 5) * (8 / MI);
 
     // ---- fragments of step s from its raw bytes: fb[j][kk] covers k 16kk + 8hl + 0..7.
     // Factors first (one set per column and step, Q6_K one per k16 sub-step), then
@@ -301,13 +308,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_kernel(
         const uint32_t R = 8 * (wave + kWaves * uint32_t(i)) + (lane >> 3), c = (lane & 7) ^ ((R >> 1) & 7);
         xoff[i] = ((t0 + R) * cols + 8 * c) * 2;
     }
-    auto dma_x = [&](uint32_t s, int buf, int i0 = 0, int i1 = XDMA) {  // instructions i0 .. i1-1
+    auto dma_x = [&](uint32_t s, int buf, int i0 = 0, int i1 = 1 << 30) {  // instructions i0 .. i1-1
 #pragma unroll
         for (int i = 0; i < XDMA; ++i) {
             if (i < i0 || i >= i1) continue;
             const uint32_t rbase = 8 * (wave + kWaves * uint32_t(i));
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                xsrc, (__attribute__((address_space(3))) void *)(xbuf(buf) + rbase * 8), 16, xoff[i], s * KS * 2, 0, 0);
+            dma16(xsrc, xbuf(buf) + rbase * 8, xoff[i], s * KS * 2);
         }
     };
     // A fragment (token tile i, k16 sub-step kk) of buffer buf: row R = 32i + l, chunk 2kk + hl
@@ -387,12 +393,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_kernel(
 #pragma unroll
             for (int kk = 0; kk < 4; ++kk) {
                 // The step's global loads, spread over its four sub-steps: x(s+3) into buffer
-                // (s-1) % 4, two instructions per sub-step, and the raw refill, one column per
+                // (s-1) % 4, a quarter of them per sub-step, and the raw refill, one column per
                 // sub-step (Q4_K: slot s % 4, decoded during step s-1; Q6_K at odd steps: the
                 // pair slot of steps s-1 and s).  Issued as one burst after the barrier, the
                 // four waves' loads stalled the matrix pipe for ~15% of every step.
-                static_assert(XDMA == 8, "two x instructions per sub-step");
-                dma_x(s + 3, (jstep + 3) & 3, 2 * kk, 2 * kk + 2);
+                static_assert(XDMA % 4 == 0, "an equal share of the x instructions per sub-step");
+                dma_x(s + 3, (jstep + 3) & 3, XDMA / 4 * kk, XDMA / 4 * (kk + 1));
                 if (kk < NJ) {
                     if constexpr (Q4) load_raw(s + 4, raw[jstep], kk);
                     else if (jstep & 1) load_raw(s + 3, raw[(jstep >> 1) & 1], kk);
@@ -509,29 +515,36 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_kernel(
     auto pbase = [&](uint32_t part) -> char * { return reinterpret_cast<char *>(partial + part * pstride); };
     if (rs_spin != 0) {
         // Reduce-scatter (the host launches it only when the whole grid fits on the device at
-        // once, so the kparts workgroups of a tile run together): part kp owns token sub-tiles
-        // [own_lo, own_hi) of the tile.  Each part stores the sub-tiles it does not own, keeps
-        // its own in LDS (slot k in x buffer k, free after the main loop), counts one arrival on
+        // once, so the kparts workgroups of a tile run together): of the tile's 16-token units (the
+        // lower and upper eight elements of each MFMA tile), part kp owns [own_lo, own_hi).  Each part
+        // stores the units it does not own, keeps its own in LDS (the x buffers, free after the main
+        // loop), counts one arrival on
         // written[tile] once its stores are acknowledged, waits until every part has, then adds
-        // the parts of its own sub-tiles in part order (its own from LDS) and writes them.  Every
+        // the parts of its own units in part order (its own from LDS) and writes them.  Every
         // part reads and writes a 1/kparts share, where the last arrival of the other form reads
         // every part alone.  The wait is bounded: a part whose limit runs out writes its
-        // sub-tiles as NaN.  The last part past the wait clears both counters.
+        // units as NaN.  The last part past the wait clears both counters.
         const uint32_t ntiles = ntok_tiles * ncol_tiles;
         uint32_t *written = counters + tile, *departed = counters + ntiles + tile;
-        const uint32_t own_lo = kp * MI / kparts, own_hi = (kp + 1) * MI / kparts;
+        const uint32_t own_lo = kp * (2 * MI) / kparts, own_hi = (kp + 1) * (2 * MI) / kparts;
+        // unit k of the own ones: 8 elements x NJ columns of every thread, 16 KiB
+        auto slot = [&](uint32_t k) -> float * {
+            if constexpr (MI == 8) return reinterpret_cast<float *>(xbuf(int(k >> 1) & 3) + (k & 1) * 1024);
+            else return reinterpret_cast<float *>(xbuf(int(k) & 3));
+        };
         __syncthreads();  // every wave is past its last read of the x buffers
 #pragma unroll
-        for (int i = 0; i < MI; ++i) {
-            if (uint32_t(i) >= own_lo && uint32_t(i) < own_hi) {
-                float *slot = reinterpret_cast<float *>(xbuf(int(uint32_t(i) - own_lo) & 3));
+        for (int u = 0; u < 2 * MI; ++u) {
+            const int i = u >> 1, v0 = 8 * (u & 1);
+            if (uint32_t(u) >= own_lo && uint32_t(u) < own_hi) {
+                float *sl = slot(uint32_t(u) - own_lo);
 #pragma unroll
-                for (int v = 0; v < 16; ++v)
+                for (int v = 0; v < 8; ++v)
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j) slot[(v * NJ + j) * kThreads + tid] = acc[i][j][v];
+                    for (int j = 0; j < NJ; ++j) sl[(v * NJ + j) * kThreads + tid] = acc[i][j][v0 + v];
             } else {
 #pragma unroll
-                for (int v = 0; v < 16; ++v)
+                for (int v = v0; v < v0 + 8; ++v)
 #pragma unroll
                     for (int j = 0; j < NJ; ++j)
                         __hip_atomic_store(reinterpret_cast<float *>(pbase(kp) + poff(i, v, j)), acc[i][j][v],
@@ -561,38 +574,53 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_kernel(
         }
         __syncthreads();
         const bool late = late_flag != 0;
-        for (uint32_t i = own_lo; i < own_hi; ++i) {
-            const float *slot = reinterpret_cast<const float *>(xbuf(int(i - own_lo) & 3));
-            float sum[16][NJ];
+        // NU units at a time (two where a part owns whole MFMA tiles), four parts per round trip
+        auto finish = [&](uint32_t u0, auto nu) {
+            constexpr int NU = decltype(nu)::value, NV = 8 * NU;
+            auto uoff = [&](int v, int j) -> uint32_t {
+                return (u0 * 16 + 8 * uint32_t(v >> 2) + uint32_t(v & 3)) * rstride + lane_off[j];
+            };
+            float sum[NV][NJ];
             for (uint32_t p0 = 0; p0 < kparts; p0 += 4) {
-                float pv[4][16][NJ];
+                float pv[4][NV][NJ];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    // this part's own slot holds no value for these sub-tiles: read from LDS below
+                    // this part's own slot holds no value for these units: read from LDS below
                     const uint32_t part = __builtin_elementwise_min(p0 + uint32_t(u), kparts - 1);
 #pragma unroll
-                    for (int v = 0; v < 16; ++v)
+                    for (int v = 0; v < NV; ++v)
 #pragma unroll
                         for (int j = 0; j < NJ; ++j)
-                            pv[u][v][j] = __hip_atomic_load(reinterpret_cast<float *>(pbase(part) + poff(int(i), v, j)),
+                            pv[u][v][j] = __hip_atomic_load(reinterpret_cast<float *>(pbase(part) + uoff(v, j)),
                                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
 #pragma unroll
-                for (int v = 0; v < 16; ++v)
+                for (int v = 0; v < NV; ++v)
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
+                        const float *sl = slot(u0 - own_lo + uint32_t(v >> 3));
                         float t = p0 == 0 ? 0.f : sum[v][j];
 #pragma unroll
                         for (int u = 0; u < 4; ++u) {
                             const uint32_t part = p0 + uint32_t(u);
-                            const float val = part == kp ? slot[(v * NJ + j) * kThreads + tid] : pv[u][v][j];
+                            const float val = part == kp ? sl[((v & 7) * NJ + j) * kThreads + tid] : pv[u][v][j];
                             t = part == 0 ? val : part < kparts ? t + val : t;
                         }
                         sum[v][j] = t;
                     }
             }
-            write_out(int(i), [&](int v, int j) { return late ? __builtin_nanf("") : sum[v][j]; });
-        }
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                float val[NJ];
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) val[j] = late ? __builtin_nanf("") : sum[v][j];
+                emit(t0 + u0 * 16 + 8 * uint32_t(v >> 2) + 4 * hl + uint32_t(v & 3), val);
+            }
+        };
+        if (MI % kparts == 0)
+            for (uint32_t u = own_lo; u < own_hi; u += 2) finish(u, std::integral_constant<int, 2>{});
+        else
+            for (uint32_t u = own_lo; u < own_hi; ++u) finish(u, std::integral_constant<int, 1>{});
         return;
     }
 #pragma unroll
@@ -650,13 +678,29 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_kernel(
     }
 }
 
-// Workgroups of one instance the device holds at once (one per CU at 128 KiB of LDS), per device.
-template <class K>
-uint64_t resident_wgs(K kernel) {
-    static int cache[64][3] = {};
+using Kernel = void (*)(const uint8_t *, const uint8_t *, const uint16_t *, void *, float *, uint32_t *, uint32_t, uint32_t,
+                        uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t *);
+
+template <int MI>
+Kernel kernel_of(int type, bool pair) {
+    if (pair) return &gemm_f16_kernel<Q4_K, true, MI>;
+    return type == Q4_K ? &gemm_f16_kernel<Q4_K, false, MI> : &gemm_f16_kernel<Q6_K, false, MI>;
+}
+
+int device_cus() {
+    static int cache[64] = {};
     int dev = 0;
     (void)hipGetDevice(&dev);
-    const int slot = kernel == &gemm_f16_kernel<Q4_K, true> ? 0 : kernel == &gemm_f16_kernel<Q4_K, false> ? 1 : 2;
+    int &n = cache[dev & 63];
+    if (n == 0 && (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)) n = 256;
+    return n;
+}
+
+// Workgroups of one instance the device holds at once, per device.
+uint64_t resident_wgs(Kernel kernel, int slot) {
+    static int cache[64][6] = {};
+    int dev = 0;
+    (void)hipGetDevice(&dev);
     int &n = cache[dev & 63][slot];
     if (n == 0) {
         int wgs = 0, cus = 0;
@@ -670,29 +714,51 @@ uint64_t resident_wgs(K kernel) {
 }
 
 struct F16Plan {
-    uint32_t ntok, ncol, kparts;
+    uint32_t mi, ntok, ncol, kparts;
+    uint32_t cost;  // the estimate, tenths of a microsecond
 };
 
+// Token tile and split K: one workgroup runs per CU, so a plan costs its rounds of workgroups times the
+// super-blocks each walks, plus the hand-off of a split (fitted to MI355X, within ~15%).  A 128-token
+// tile decodes each weight fragment for half the matrix work (3.8 us per super-block against 7.0), so
+// it pays where it fills a round better: gate/up pair at 225 tokens 82 -> 65 us (240 workgroups
+// without split K instead of 120 tiles in two K parts), downs at 225 61-70 -> 49-55, at 320 78-81 -> 64.
+// K is split only while all parts run in one round (downs at 600 tokens: 45 tiles in 8 parts, 360
+// workgroups, took 173-195 us; in 4 parts 102).
 F16Plan plan_f16(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t) {
-    F16Plan p;
-    p.ntok = (batch + TT - 1) / TT;
-    const uint32_t rows_per_tile = pair ? TC / 2 : TC;
-    p.ncol = (rows + rows_per_tile - 1) / rows_per_tile;
-    const uint32_t nb = cols / kQK, tiles = p.ntok * p.ncol;
-    p.kparts = 1;
-    // one workgroup per CU on 256 CUs: split K until the grid covers most of them
-    while (tiles * p.kparts < 200 && p.kparts * 2 <= nb / 4) p.kparts *= 2;
-    if (t.gemm_kparts >= 1 && uint32_t(t.gemm_kparts) <= nb) p.kparts = uint32_t(t.gemm_kparts);
-    if (uint64_t(pair ? 2 : 1) * p.ntok * TT * p.ncol * rows_per_tile * 4 >= (uint64_t(1) << 32)) p.kparts = 1;
-    return p;
+    const uint32_t rows_per_tile = pair ? TC / 2 : TC, ncol = (rows + rows_per_tile - 1) / rows_per_tile;
+    const uint32_t nb = cols / kQK, cus = uint32_t(device_cus());
+    F16Plan best{};
+    uint32_t best_cost = ~0u;
+    for (uint32_t mi : {8u, 4u}) {
+        if (t.f16_mi > 0 && uint32_t(t.f16_mi) != mi) continue;
+        F16Plan p{mi, (batch + 32 * mi - 1) / (32 * mi), ncol, 1, 0};
+        const uint32_t tiles = p.ntok * ncol, sb = mi == 8 ? 70 : 38;
+        for (uint32_t kp = 1; kp == 1 || (kp <= 2 * mi && kp * 2 <= nb && tiles * kp <= cus); kp *= 2) {
+            const uint32_t cost = (tiles * kp + cus - 1) / cus * (60 + (nb + kp - 1) / kp * sb) + (kp > 1 ? 100 : 0);
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = p;
+                best.kparts = kp;
+                best.cost = cost;
+            }
+        }
+    }
+    if (t.gemm_kparts >= 1 && uint32_t(t.gemm_kparts) <= nb) best.kparts = uint32_t(t.gemm_kparts);
+    if (uint64_t(pair ? 2 : 1) * best.ntok * (32 * best.mi) * ncol * rows_per_tile * 4 >= (uint64_t(1) << 32)) best.kparts = 1;
+    return best;
 }
 
 }  // namespace
 
+uint32_t gemm_f16_cost(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t) {
+    return plan_f16(cols, rows, batch, pair, t).cost;
+}
+
 void gemm_f16_workspace_need(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t,
                              size_t *part_floats, size_t *counters) {
     const F16Plan p = plan_f16(cols, rows, batch, pair, t);
-    *part_floats = p.kparts > 1 ? size_t(p.kparts) * (pair ? 2 : 1) * (p.ntok * TT) * (p.ncol * (pair ? TC / 2 : TC)) : 0;
+    *part_floats = p.kparts > 1 ? size_t(p.kparts) * (pair ? 2 : 1) * (p.ntok * 32 * p.mi) * (p.ncol * (pair ? TC / 2 : TC)) : 0;
     *counters = 2 * size_t(p.ntok) * p.ncol;  // arrivals; and departures of the reduce-scatter
 }
 
@@ -703,12 +769,11 @@ hipError_t launch_gemm_f16(int type, const uint8_t *w, const uint8_t *up, const 
     const F16Plan p = plan_f16(cols, rows, batch, pair, t);
     const dim3 grid(p.ntok * p.ncol * p.kparts), block(kThreads);
     const uint32_t wbytes = rows * (cols / kQK) * block_bytes(type);
+    const Kernel kernel = p.mi == 8 ? kernel_of<8>(type, pair) : kernel_of<4>(type, pair);
     // the reduce-scatter needs every part of a tile running at once: the whole grid resident
-    const auto kernel = pair ? &gemm_f16_kernel<Q4_K, true>
-                             : type == Q4_K ? &gemm_f16_kernel<Q4_K, false> : &gemm_f16_kernel<Q6_K, false>;
     uint32_t rs_spin = 0;
-    if (p.kparts > 1 && MI % p.kparts == 0 && t.gemm_rs != 0 && waits_allowed(t) &&
-        uint64_t(grid.x) <= resident_wgs(kernel))
+    if (p.kparts > 1 && (2 * p.mi) % p.kparts == 0 && t.gemm_rs != 0 && waits_allowed(t) &&
+        uint64_t(grid.x) <= resident_wgs(kernel, (pair ? 0 : type == Q4_K ? 1 : 2) + (p.mi == 8 ? 0 : 3)))
         rs_spin = t.gemm_rs > 1 ? uint32_t(t.gemm_rs) : 1u << 22;  // 2^22 polls of s_sleep 2: seconds
     kernel<<<grid, block, 0, stream>>>(w, pair ? up : w, x, out, partial, counters, cols, rows, batch, p.ntok, p.ncol,
                                        p.kparts, wbytes, rs_spin, err);

@@ -657,7 +657,7 @@ uint32_t col_tiles(const uint32_t *rows, int nseg, bool pair, uint32_t wk) {
 // the first round) adds the hand-off, whose last arrival reads every part.
 Plan plan_skinny(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair, bool f16,
                  const Tuning &t) {
-    static constexpr uint32_t kIter[3][3] = {{25, 45, 0}, {22, 38, 0}, {23, 36, 71}};  // FP32 Q4_K, FP32 Q6_K, FP16
+    static constexpr uint32_t kIter[3][3] = {{25, 45, 0}, {22, 38, 0}, {23, 36, 80}};  // FP32 Q4_K, FP32 Q6_K, FP16
     const uint32_t *iter_cost = kIter[f16 ? 2 : type == Q6_K ? 1 : 0];
     Plan best{};
     const uint32_t nb = cols / kQK, cus = uint32_t(device_cus());
@@ -707,12 +707,13 @@ hipError_t launch_mi(const Plan &p, const Args &a, hipStream_t stream) {
 
 }  // namespace
 
-// Whether this kernel is the faster one: a bound on the plan's estimate.  The 128- and 256-token
-// tile kernels need many output tiles to fill the device and then cost ~90-115 us; below that they
-// take as long.  MI355X, this kernel against them (us), each bound from both sides:
-//   gate/up FP16   384 tokens: 110 / 114,             512: 145 / 114
-//   gate/up FP32   192: 81 / 94,                      225: 106 / 95
-//   downs          512: 73-96 / 78-127,               775: 157-180 / 134-145, FP16 1024: 137 / 127
+// Whether this kernel is the faster one.  FP16 mode: by its plan's estimate against the tile kernel's
+// (gate/up 128 tokens: 44 us here, 50 there; 225: 75 / 65; downs 225: 43-46 / 48-55; 320: 63-67 / 63).
+// FP32 mode: a bound on the estimate, because the 128- and 256-token tile kernels need many output
+// tiles to fill the device and then cost ~90-115 us; below that they take as long.  MI355X, this
+// kernel against them (us), each bound from both sides:
+//   gate/up        192 tokens: 81 / 94,               225: 106 / 95
+//   downs          512: 78-96 / 114-127,              775: 157-180 / 134-145
 //   4096 x 3840    1536: 89 / 114, row-major 93 / 95;   2048: 121 / 103, row-major 125 / 106
 // A row-major Q6_K tensor runs at 260-273 us at any batch there (2-byte loads) and at 42-80 us here
 // for 2,048 rows at 1,024-2,048 tokens.
@@ -723,10 +724,11 @@ bool gemm_skinny_eligible(int type, int layout, int acc, uint32_t cols, const ui
     if (t.gemm_skinny > 0) return batch <= uint32_t(t.gemm_skinny);
     if (t.gemm_q4_reg == 0 && type == Q4_K && acc == ACC_FP32) return false;  // the LDS-tile kernel is asked for
     if (batch > 2048) return false;  // beyond what was measured
-    uint32_t tiles = 0;  // 256 tokens x 256 columns
-    for (int s = 0; s < nseg; ++s) tiles += (batch + 255) / 256 * ((rows[s] * (pair ? 2 : 1) + 255) / 256);
     const uint32_t cost = plan_skinny(type, cols, rows, nseg, batch, pair, acc == ACC_FP16, t).cost;
-    return cost <= (layout == ROW_MAJOR && type == Q6_K ? 2600u : acc == ACC_FP16 && tiles >= 96 ? 1100u : 960u);
+    // (and a bound: past two rounds the weights are read once per token tile from beyond L2, which the
+    // estimate leaves out: downs at 600 tokens 124-130 us here, 109 there)
+    if (acc == ACC_FP16) return cost <= std::min(800u, gemm_f16_cost(cols, rows[0], batch, pair, t));
+    return cost <= (layout == ROW_MAJOR && type == Q6_K ? 2600u : 960u);
 }
 
 void gemm_skinny_workspace_need(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair,

@@ -34,6 +34,7 @@ struct Tuning {
     int gemm_skinny = -1; // -1: plan; 0: never the few-token GEMM; > 0: up to this many tokens
     int skinny_wk = 0;    // 4 / 8: its groups of super-blocks per workgroup
     int skinny_mi = 0;    // 1 / 2 / 4: its token tile, in 32-token units
+    int f16_mi = 0;       // 4 / 8: the FP16-mode prefill GEMM's token tile, in 32-token units
     int stack_fused = 1;  // 0: the multi-layer decode as one block launch per layer
 };
 
@@ -183,6 +184,7 @@ hipError_t launch_gemm_reg(const uint8_t *w, const uint8_t *up, const uint16_t *
 // tiles with per-row power-of-two scales (ns_tile16.hpp), no x group sums.
 void gemm_f16_workspace_need(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t,
                              size_t *part_floats, size_t *counters);
+uint32_t gemm_f16_cost(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t);  // estimate, 0.1 us
 hipError_t launch_gemm_f16(int type, const uint8_t *w, const uint8_t *up, const uint16_t *x, void *out, uint32_t cols,
                            uint32_t rows, uint32_t batch, float *partial, uint32_t *counters, uint32_t *err,
                            const Tuning &t, hipStream_t stream);

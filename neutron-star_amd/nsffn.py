@@ -353,7 +353,7 @@ class Context:
         """Test hook: override one kernel-selection choice of this context
         (ns_ctx_set_tuning; keys gemv_pf, gemv_waves, gemv_whole, gemv_qslab,
         gemm_kparts, gemm_q4_reg, mt_mfma, mt_parts, mt_slabs, mt_spw, block_fused, block_spin, gemm_rs,
-        gemm_skinny, skinny_wk, skinny_mi)."""
+        gemm_skinny, skinny_wk, skinny_mi, f16_mi, gemv_row)."""
         check(lib().ns_ctx_set_tuning(self.handle, key.encode(), int(value)))
 
     def workspace_bytes(self):

@@ -18,7 +18,7 @@ TUNING_DEFAULTS = {"gemv_pf": -1, "gemv_waves": 0, "gemv_whole": 1, "gemv_qslab"
                    "gemm_q4_reg": 1, "mt_mfma": 1, "mt_parts": 0, "mt_slabs": 0, "mt_spw": 0, "block_fused": 1,
                    "block_spin": 0, "gemm_rs": 1, "stack_fused": 1, "gemm_skinny": -1,
                    "skinny_wk": 0, "skinny_mi": 0,
-                   "gemv_row": 1}
+                   "gemv_row": 1, "f16_mi": 0}
 
 
 @pytest.fixture
