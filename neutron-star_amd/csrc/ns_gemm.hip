@@ -233,15 +233,13 @@ __device__ __forceinline__ void decode(const RawQ6 &r, uint32_t s, uint32_t hh, 
 // c24 = c * 2^24; same element placement as the exact decode above.
 __device__ __forceinline__ void decode_f16(const RawQ4 &r, uint32_t s, float c24, WRun &out) {
     const uint32_t p = s & 3;
-    const float d = lo_half(r.hdr.x), dmin = hi_half(r.hdr.x);
     const Q4Scales sc = q4_scales(r.hdr.y, r.hdr.z, r.hdr.w);
-    const float dc = d * c24, mc = -dmin * (c24 * 5.9604644775390625e-08f);
-    const half2_t Alo = splat(_Float16(dc * float(q4_sc(sc, int(2 * p))))), Ahi = splat(_Float16(dc * float(q4_sc(sc, int(2 * p + 1)))));
-    const half2_t Blo = splat(_Float16(mc * float(q4_m(sc, int(2 * p))))), Bhi = splat(_Float16(mc * float(q4_m(sc, int(2 * p + 1)))));
+    const Q4Factors g = q4_factors(p < 2 ? sc.sc03 : sc.sc47, (p < 2 ? sc.m03 : sc.m47) << 2, int(p & 1),
+                                   q4_dc(r.hdr.x, c24), q4_mc22(r.hdr.x, c24));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t lo[2], hi[2];
-        q4_f16x8(r.qs[i], Alo, Blo, Ahi, Bhi, lo, hi);
+        q4_f16x8(r.qs[i], g, lo, hi);
         out.v[i >> 1][(i & 1) * 2 + 0] = lo[0];
         out.v[i >> 1][(i & 1) * 2 + 1] = lo[1];
         out.v[2 + (i >> 1)][(i & 1) * 2 + 0] = hi[0];

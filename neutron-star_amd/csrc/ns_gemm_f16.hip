@@ -238,21 +238,18 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_kernel(
     // one fragment at a time, so the decode of the next step can be spread over the
     // MFMAs of this one.
     struct Factors {
-        half2_t A[NJ][Q4 ? 2 : 4], B[NJ][Q4 ? 2 : 4];
+        half2_t A[NJ][Q4 ? 1 : 4], B[NJ][Q4 ? 1 : 4];
     };
     auto factors = [&](uint32_t s, const Raw (&raw)[NJ], Factors &F) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             if constexpr (Q4) {
                 const uint32_t p = s & 3;
-                const float d = lo_half(raw[j].hdr.x), dmin = hi_half(raw[j].hdr.x);
                 const Q4Scales sc = q4_scales(raw[j].hdr.y, raw[j].hdr.z, raw[j].hdr.w);
-                const float dc = d * c24[j], mc = -dmin * (c24[j] * 5.9604644775390625e-08f);  // c = c24 * 2^-24
-#pragma unroll
-                for (int hi = 0; hi < 2; ++hi) {
-                    F.A[j][hi] = splat(_Float16(dc * float(q4_sc(sc, int(2 * p) + hi))));
-                    F.B[j][hi] = splat(_Float16(mc * float(q4_m(sc, int(2 * p) + hi))));
-                }
+                const Q4Factors g = q4_factors(p < 2 ? sc.sc03 : sc.sc47, (p < 2 ? sc.m03 : sc.m47) << 2, int(p & 1),
+                                               q4_dc(raw[j].hdr.x, c24[j]), q4_mc22(raw[j].hdr.x, c24[j]));
+                F.A[j][0] = g.A;
+                F.B[j][0] = g.B;
             } else {
                 // step s: half h = (s%4)/2, quarters Q = 2*(s%2) + kk/2; scale sc[8h + kk%2 + 2Q]
                 const uint32_t sr = s & 3, qb2 = 2 * (sr & 1);
@@ -277,7 +274,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f16_kernel(
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 uint32_t lo[2], hv[2];
-                q4_f16x8(w[e], F.A[j][0], F.B[j][0], F.A[j][1], F.B[j][1], lo, hv);
+                q4_f16x8(w[e], Q4Factors{F.A[j][0], F.B[j][0]}, lo, hv);
                 f[2 * e] = hi ? hv[0] : lo[0];
                 f[2 * e + 1] = hi ? hv[1] : lo[1];
             }

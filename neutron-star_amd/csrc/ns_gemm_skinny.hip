@@ -319,7 +319,7 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
 
     // ---- per super-block factors of column j, and its fragments (group grp, e)
     struct Factors {
-        half2_t A[NJ][8], B[NJ][8];  // per group; Q4_K FP32 mode: A alone
+        half2_t A[NJ][8], B[NJ][8];  // per group; Q4_K FP32 mode: A alone; Q4_K FP16 mode: per group pair
     };
     auto factors = [&](const Raw (&r)[NJ], Factors &F) {
 #pragma unroll
@@ -327,12 +327,13 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
             if constexpr (Q4) {
                 const Q4Scales sc = q4_scales(r[j].hdr.y, r[j].hdr.z, r[j].hdr.w);
                 if constexpr (F16) {
-                    const float dc = lo_half(r[j].hdr.x) * c24[j];
-                    const float mc = -hi_half(r[j].hdr.x) * (c24[j] * 5.9604644775390625e-08f);  // c = c24 * 2^-24
+                    const half2_t dc = q4_dc(r[j].hdr.x, c24[j]), mc = q4_mc22(r[j].hdr.x, c24[j]);
+                    const uint32_t m03 = sc.m03 << 2, m47 = sc.m47 << 2;
 #pragma unroll
-                    for (int gg = 0; gg < 8; ++gg) {
-                        F.A[j][gg] = splat(_Float16(dc * float(q4_sc(sc, gg))));
-                        F.B[j][gg] = splat(_Float16(mc * float(q4_m(sc, gg))));
+                    for (int p = 0; p < 4; ++p) {  // group pair 2p, 2p + 1 (its A times 2^-4)
+                        const Q4Factors g = q4_factors(p < 2 ? sc.sc03 : sc.sc47, p < 2 ? m03 : m47, p & 1, dc, mc);
+                        F.A[j][p] = g.A;
+                        F.B[j][p] = g.B;
                     }
                 } else {
                     // q*2^-24 (low nibbles) or 16q*2^-24 (high) times this = sc*q*2^-14, exact
@@ -365,12 +366,13 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
         for (int d = 0; d < 2; ++d) {
             if constexpr (Q4) {
                 const uint32_t w = r.qs[grp >> 1][2 * e + d];
-                const uint32_t p = __builtin_amdgcn_perm(w, w, 0x03010200u);  // bytes [b0, b2, b1, b3]
                 if constexpr (F16) {
-                    const uint32_t s = grp & 1 ? 4 : 0;
-                    f[2 * d] = bits(__builtin_elementwise_fma(h2((p >> s) & 0x000F000Fu), A[grp], B[grp]));
-                    f[2 * d + 1] = bits(__builtin_elementwise_fma(h2((p >> (8 + s)) & 0x000F000Fu), A[grp], B[grp]));
+                    uint32_t lo[2], hi[2];  // (the two groups of a pair share the unpack: common subexpressions)
+                    q4_f16x8(w, Q4Factors{A[grp >> 1], B[grp >> 1]}, lo, hi);
+                    f[2 * d] = grp & 1 ? hi[0] : lo[0];
+                    f[2 * d + 1] = grp & 1 ? hi[1] : lo[1];
                 } else {
+                    const uint32_t p = __builtin_amdgcn_perm(w, w, 0x03010200u);  // bytes [b0, b2, b1, b3]
                     const uint32_t m = grp & 1 ? 0x00F000F0u : 0x000F000Fu;
                     f[2 * d] = bits(h2(p & m) * A[grp]);
                     f[2 * d + 1] = bits(h2((p >> 8) & m) * A[grp]);
@@ -398,6 +400,8 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
     // registers, filled one super-block earlier, changed nothing: 20.3 us either way for the FP16 pair
     // at 5 tokens, and the FP32 pair took 23.0 instead of 21.5.)
     constexpr bool kMin = Q4 && !F16;
+    float one = 1.0f;  // opaque, so that x * one + p stays one mixed-precision FMA (else a convert and an add)
+    asm volatile("" : "+s"(one));
     for (uint32_t it = 0; it < iters; ++it) {
         const uint32_t sb = sb_of(it), sbn = sb_of(it + 1);
         const bool valid = sb < sb1, more = sbn < sb1;  // wave-uniform
@@ -441,7 +445,7 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
                             if constexpr (kMin) {
                                 float p = e == 0 ? 0.f : P[i][grp];
 #pragma unroll
-                                for (int k = 0; k < 8; ++k) p += float(av[i][k]);
+                                for (int k = 0; k < 8; ++k) p = __builtin_fmaf(float(av[i][k]), one, p);
                                 P[i][grp] = p;
                             }
 #pragma unroll

@@ -48,18 +48,46 @@ __device__ __forceinline__ void row_scale(float M, float &c24, float &inv_c, boo
 
 __device__ __forceinline__ half2_t splat(_Float16 v) { return half2_t{v, v}; }
 
+// The A and B factors of a Q4_K group pair (2p, 2p+1) in the two halves of one register, the odd
+// group's A times 2^-4, by packed fp16 operations from the packed scale and min bytes.  The high
+// nibbles then enter as 16q (the mask 0x00F000F0, no shift).  The tile values are those of the
+// formulas above bit for bit:
+//   - dc = d * 2^24 * c is an fp16 (a power of two times d) unless it is below 2^-14; then A < 2^-8,
+//     and |q * 2^-24 * A| < 2^-25 is under half a step of fp16 beside B, so F = B either way;
+//   - A * 2^-4 is exact unless A < 2^-10, where F = B again;
+//   - B = RNE16(mc * m) as one product of (mc * 2^22) and m * 2^-22; mc * 2^22 is an fp16 unless
+//     |mc| < 2^-36, where B = 0 either way.
+struct Q4Factors {
+    half2_t A, B;
+};
+// sc, m: four groups' bytes (q4_scales); h: the upper pair of them; dc, mc22: splat factors.
+__device__ __forceinline__ Q4Factors q4_factors(uint32_t sc, uint32_t m4, int h, half2_t dc, half2_t mc22) {
+    // bytes under the exponents 0x64 and 0x54 are the fp16 values 1024 + b and 64 + b/16
+    const uint32_t s = __builtin_amdgcn_perm(0x00005464u, sc, h ? 0x05030402u : 0x05010400u);
+    const uint32_t m = __builtin_amdgcn_perm(0u, m4, h ? 0x0C030C02u : 0x0C010C00u);  // 4m, an fp16 subnormal: m * 2^-22
+    Q4Factors f;
+    f.A = (__builtin_bit_cast(half2_t, s) + half2_t{_Float16(-1024.0f), _Float16(-64.0f)}) * dc;
+    f.B = __builtin_bit_cast(half2_t, m) * mc22;
+    return f;
+}
+// The splat factors of a block: header dword (d, dmin) and the row's c24 = c * 2^24.
+__device__ __forceinline__ half2_t q4_dc(uint32_t ddmin, float c24) { return splat(_Float16(lo_half(ddmin) * c24)); }
+__device__ __forceinline__ half2_t q4_mc22(uint32_t ddmin, float c24) {
+    return splat(_Float16(-hi_half(ddmin) * (c24 * 0.25f)));  // -dmin * c * 2^22
+}
+
 // One qs dword (elements l..l+3 of groups 2p (low nibbles) and 2p+1 (high)):
 // lo[0..1] = F of l..l+3 in group 2p, hi[0..1] the same in group 2p+1.
-__device__ __forceinline__ void q4_f16x8(uint32_t w, half2_t Alo, half2_t Blo, half2_t Ahi, half2_t Bhi,
-                                         uint32_t (&lo)[2], uint32_t (&hi)[2]) {
-    const uint32_t p = __builtin_amdgcn_perm(w, w, 0x03010200u);  // bytes [b0, b2, b1, b3]
+__device__ __forceinline__ void q4_f16x8(uint32_t w, const Q4Factors &g, uint32_t (&lo)[2], uint32_t (&hi)[2]) {
+    const uint32_t p = __builtin_amdgcn_perm(w, w, 0x03010200u), p8 = p >> 8;  // bytes [b0, b2, b1, b3]
+    const half2_t Al{g.A.x, g.A.x}, Bl{g.B.x, g.B.x}, Ah{g.A.y, g.A.y}, Bh{g.B.y, g.B.y};
     auto f = [](uint32_t q, half2_t A, half2_t B) {
         return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(half2_t, q), A, B));
     };
-    lo[0] = f(p & 0x000F000Fu, Alo, Blo);
-    lo[1] = f((p >> 8) & 0x000F000Fu, Alo, Blo);
-    hi[0] = f((p >> 4) & 0x000F000Fu, Ahi, Bhi);
-    hi[1] = f((p >> 12) & 0x000F000Fu, Ahi, Bhi);
+    lo[0] = f(p & 0x000F000Fu, Al, Bl);
+    lo[1] = f(p8 & 0x000F000Fu, Al, Bl);
+    hi[0] = f(p & 0x00F000F0u, Ah, Bh);
+    hi[1] = f(p8 & 0x00F000F0u, Ah, Bh);
 }
 
 // Four 6-bit Q6_K values, one per byte of v (elements l..l+3): F of l..l+3.
