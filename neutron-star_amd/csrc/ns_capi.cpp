@@ -201,9 +201,25 @@ int gemv(ns_ctx *ctx, const char *fn, int type, int layout, const void *w, const
     return e == hipSuccess ? NS_OK : hip_fail(e, fn);
 }
 
+// The few-token prefill GEMM (ns_gemm_skinny.hip) over 1-3 matrices that share x, FP32 mode.
+int gemm_skinny(ns_ctx *ctx, const char *fn, int type, int last_type, int layout, const void *const *w, const void *up,
+                const uint16_t *x, void *const *out, void *copy, const uint32_t *rows, int nseg, uint32_t cols,
+                uint32_t batch, hipStream_t s) {
+    size_t pf = 0, nc = 0;
+    gemm_skinny_workspace_need(type, cols, rows, nseg, batch, up != nullptr, ACC_FP32, ctx->ws.tune, &pf, &nc);
+    if (int rc = ensure_ws(ctx, pf, nc, s)) return rc;
+    const hipError_t e = launch_gemm_skinny(type, layout, ACC_FP32, reinterpret_cast<const uint8_t *const *>(w),
+                                            static_cast<const uint8_t *>(up), out, rows, nseg, x, cols, batch,
+                                            ctx->ws.partial, ctx->ws.counters, ctx->ws.tune, s, last_type, copy);
+    return e == hipSuccess ? NS_OK : hip_fail(e, fn);
+}
+
 // Batch 2-4: the weights stream once for every token (mm:273, mm:282).
 int gemv_mt(ns_ctx *ctx, const char *fn, int type, int layout, const void *w, const void *up, const void *x,
             bool xh, uint32_t batch, void *out, uint32_t cols, uint32_t rows, hipStream_t s) {
+    if (xh && !up && skinny_small_batch(type, layout, cols, rows, x, batch, false, ctx->ws.tune))
+        return gemm_skinny(ctx, fn, type, 0, layout, &w, nullptr, static_cast<const uint16_t *>(x), &out, nullptr, &rows, 1,
+                           cols, batch, s);
     size_t pf = 0, nc = 0;
     gemv_mt_workspace_need(type, layout, cols, rows, up != nullptr, batch, xh, ctx->ws.tune, &pf, &nc);
     if (int rc = ensure_ws(ctx, pf, nc, s)) return rc;
@@ -611,6 +627,20 @@ extern "C" int ns_qkv(ns_ctx *ctx, const void *wq, const void *wk, const void *w
     if (!x || !q || !k || !v) return fail(NS_ERR_ARG, "ns_qkv: null input/output");
     if (batch < 2) return fail(NS_ERR_UNSUPPORTED, "ns_qkv: the fused projection is the prefill path (batch >= 2)");
     const hipStream_t s = static_cast<hipStream_t>(stream);
+    // One launch for the three where the few-token GEMM takes them together
+    {
+        const void *const ws_[3] = {wq, wk, wv ? wv : wk};
+        void *const outs[3] = {q, k, v};
+        const uint32_t rows[3] = {q_rows, kv_rows, kv_rows};
+        const int nseg = wv ? 3 : 2;
+        const bool small_ok =
+            batch > 4 ||
+            (skinny_small_batch(Q4_K, layout, cols, q_rows, x, batch, true, ctx->ws.tune) &&
+             skinny_small_batch(wv ? v_type : Q4_K, layout, cols, kv_rows, x, batch, true, ctx->ws.tune));
+        if (small_ok && gemm_skinny_eligible(Q4_K, layout, ACC_FP32, cols, rows, nseg, batch, false, ctx->ws.tune))
+            return gemm_skinny(ctx, fn, Q4_K, wv ? v_type : 0, layout, ws_, nullptr, x, outs, wv ? nullptr : v, rows, nseg,
+                               cols, batch, s);
+    }
     // Q, K and V each stream their own weights once; x (fp16 [batch][cols]) is re-read
     // from the caches.  Batch 2-4 takes the small-batch kernels, larger batches the GEMM.
     auto proj = [&](const void *w, int type, uint32_t rows, float *out) {

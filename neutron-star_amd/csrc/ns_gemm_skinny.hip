@@ -56,6 +56,8 @@ struct Args {
     const uint8_t *w[kMaxSeg], *up;
     void *out[kMaxSeg];
     uint32_t rows[kMaxSeg], ct_end[kMaxSeg];
+    uint32_t q6_seg;  // the mixed kernel: the segment whose matrix is Q6_K
+    void *copy;       // a second output of the last segment (tied V), or nullptr
     const uint16_t *x;
     float *partial;
     uint32_t *counters;
@@ -116,9 +118,38 @@ struct RawQ6 {
     uint32_t x[7];  // ROW_MAJOR: the dword after each 16-byte piece (blocks are 2-byte aligned)
 };
 
+// A workgroup's work item and the LDS its kernel holds for it.
+struct Item {
+    uint32_t tt, kp, tile, seg, ct;
+};
+__device__ __forceinline__ Item work_item(const Args &a) {
+    // XCD-aware order: workgroup L runs on XCD L % 8, which takes a contiguous run of the work items
+    // q = (ct * kparts + kp) * ntok + tt, so the token tiles that share weights share an L2.
+    const uint32_t nwg = gridDim.x, w8 = nwg / 8, L = blockIdx.x;
+    const uint32_t q = L < 8 * w8 ? (L % 8) * w8 + L / 8 : L;
+    Item it;
+    it.tt = q % a.ntok;
+    const uint32_t g = q / a.ntok, ctg = g / a.kparts;
+    it.kp = g % a.kparts;
+    it.tile = ctg * a.ntok + it.tt;
+    it.seg = ctg < a.ct_end[0] ? 0u : ctg < a.ct_end[1] ? 1u : 2u;
+    it.ct = ctg - (it.seg == 0 ? 0u : a.ct_end[it.seg - 1]);
+    return it;
+}
+struct Shared {
+    float rmax[kWaves][NJ][32];
+    uint32_t last_flag;
+};
+// u32x4 of one x buffer: a stage for every wk group, and what the final sum of a token tile needs
+template <int MI, int WK>
+constexpr int buf_len() {
+    constexpr int x = WK * 32 * MI * (MI * WK <= 8 ? 128 : 64) / 8, red = kWaves * NJ * 16 * 64 / 4;
+    return x > red ? x : red;
+}
+
 // WC column groups x WK super-block groups of waves; MI 32-token tiles.
-template <int TYPE, int LAYOUT, int ACC, bool PAIR, int MI, int WK>
-__global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
+template <int TYPE, int LAYOUT, int ACC, bool PAIR, int MI, int WK, bool EX>
+__device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32x4 *X0, u32x4 *X1, Shared &sh) {
     constexpr bool Q4 = TYPE == Q4_K, F16 = ACC == ACC_FP16, ROW = LAYOUT == ROW_MAJOR;
     constexpr int WC = kWaves / WK, TT = 32 * MI;
     constexpr int KS = MI * WK <= 8 ? 128 : 64;      // columns of x per stage
@@ -128,23 +159,14 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
     constexpr int kXBuf = WK * TT * CR;               // u32x4 per buffer
     static_assert(TT % (RPI * WC) == 0 && 2 * kXBuf * 16 <= 131072, "x stages");
     using Raw = typename std::conditional<Q4, RawQ4, RawQ6>::type;
-    constexpr int kRedF4 = kWaves * NJ * 16 * 64 / 4;  // u32x4 the final sum of one token tile needs
-    // two LDS objects, so that the compiler does not take a DMA into one for a write to the other
-    __shared__ __attribute__((aligned(16))) u32x4 X0[kXBuf > kRedF4 ? kXBuf : kRedF4], X1[kXBuf > kRedF4 ? kXBuf : kRedF4];
-    __shared__ float rmax[kWaves][NJ][32];
-    __shared__ uint32_t last_flag;
+    static_assert(kXBuf <= buf_len<MI, WK>(), "x buffer");
+    // EX: sc*(v-32) in two exact fragments (see factors)
+    static_assert(!EX || (TYPE == Q6_K && ACC == ACC_FP32), "EX");
 
     const uint32_t tid = threadIdx.x, lane = tid & 63, hl = lane >> 5, ln = lane & 31;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wc = wave % WC, wk = wave / WC;
-    // XCD-aware order: workgroup L runs on XCD L % 8, which takes a contiguous run of the work items
-    // q = (ct * kparts + kp) * ntok + tt, so the token tiles that share weights share an L2.
-    const uint32_t nwg = gridDim.x, w8 = nwg / 8, L = blockIdx.x;
-    const uint32_t q = L < 8 * w8 ? (L % 8) * w8 + L / 8 : L;
-    const uint32_t tt = q % a.ntok, g = q / a.ntok, kp = g % a.kparts, ctg = g / a.kparts;
-    const uint32_t tile = ctg * a.ntok + tt;
-    const uint32_t seg = ctg < a.ct_end[0] ? 0u : ctg < a.ct_end[1] ? 1u : 2u;
-    const uint32_t ct = ctg - (seg == 0 ? 0u : a.ct_end[seg - 1]);
+    const uint32_t tt = item.tt, kp = item.kp, tile = item.tile, seg = item.seg, ct = item.ct;
     const uint32_t rows = a.rows[seg], cols = a.cols, batch = a.batch, t0 = tt * TT;
     const uint32_t nb = cols / kQK, kparts = a.kparts;
     const uint32_t sb0 = kp * nb / kparts, sb1 = (kp + 1) * nb / kparts;
@@ -217,11 +239,11 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
         if constexpr (!Q4 && ROW) {
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
-                const uint32_t sh = ((voff[j] + sb * kBlkStep) & 2u) * 8u;
+                const uint32_t by = ((voff[j] + sb * kBlkStep) & 2u) * 8u;
                 auto shift = [&](u32x4 &v, uint32_t hi) {
 #pragma unroll
-                    for (int i = 0; i < 3; ++i) v[i] = __builtin_amdgcn_alignbit(v[i + 1], v[i], sh);
-                    v[3] = __builtin_amdgcn_alignbit(hi, v[3], sh);
+                    for (int i = 0; i < 3; ++i) v[i] = __builtin_amdgcn_alignbit(v[i + 1], v[i], by);
+                    v[3] = __builtin_amdgcn_alignbit(hi, v[3], by);
                 };
 #pragma unroll
                 for (int c = 0; c < 4; ++c) shift(raw[j].ql[c], raw[j].x[c]);
@@ -295,14 +317,14 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             M[j] = __builtin_fmaxf(M[j], __shfl_xor(M[j], 32));
-            if (hl == 0) rmax[wave][j][ln] = M[j];
+            if (hl == 0) sh.rmax[wave][j][ln] = M[j];
         }
         lds_barrier();
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             float m = 0.f;
 #pragma unroll
-            for (int k = 0; k < WK; ++k) m = __builtin_fmaxf(m, rmax[uint32_t(k) * WC + wc][j][ln]);
+            for (int k = 0; k < WK; ++k) m = __builtin_fmaxf(m, sh.rmax[uint32_t(k) * WC + wc][j][ln]);
             row_scale(m, c24[j], inv_c[j], !Q4);
         }
     } else {
@@ -319,6 +341,7 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
 
     // ---- per super-block factors of column j, and its fragments (group grp, e)
     struct Factors {
+        half2_t A2[NJ][EX ? 8 : 1], B2[NJ][EX ? 8 : 1];  // EX: the odd unit of the scale
         half2_t A[NJ][8], B[NJ][8];  // per group; Q4_K FP32 mode: A alone; Q4_K FP16 mode: per group pair
     };
     auto factors = [&](const Raw (&r)[NJ], Factors &F) {
@@ -352,15 +375,21 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
                         F.A[j][gg] = splat(_Float16(dc * float(sc)));
                         F.B[j][gg] = splat(_Float16(dm * float(sc)));
                     } else {
-                        // v*2^-24 * sc*2^8 - sc*2^-11 = sc*(v-32)*2^-16
-                        F.A[j][gg] = splat(_Float16(float(sc) * 256.0f));
-                        F.B[j][gg] = splat(_Float16(float(sc) * -0.00048828125f));
+                        // v*2^-24 * sc*2^8 - sc*2^-11 = sc*(v-32)*2^-16, rounded once where |sc| > 64 makes
+                        // it 12 bits; EX takes sc without its lowest bit (11 bits) and that bit apart
+                        const int s1 = EX ? sc & ~1 : sc;
+                        F.A[j][gg] = splat(_Float16(float(s1) * 256.0f));
+                        F.B[j][gg] = splat(_Float16(float(s1) * -0.00048828125f));
+                        if constexpr (EX) {
+                            F.A2[j][gg] = splat(_Float16(float(sc & 1) * 256.0f));
+                            F.B2[j][gg] = splat(_Float16(float(sc & 1) * -0.00048828125f));
+                        }
                     }
                 }
             }
         }
     };
-    auto frag = [&](const Raw &r, const half2_t (&A)[8], const half2_t (&B)[8], int grp, int e) -> half8_t {
+    auto frag = [&](const Raw &r, const auto &A, const auto &B, int grp, int e) -> half8_t {
         u32x4 f;
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
@@ -435,11 +464,14 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
                     const int grp = st * (KS / 32) + gq;
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
-                        half8_t av[MI], fb[NJ];
+                        half8_t av[MI], fb[NJ], fb2[EX ? NJ : 1];
 #pragma unroll
                         for (int i = 0; i < MI; ++i) av[i] = load_a(st & 1, i, gq, e);
 #pragma unroll
-                        for (int j = 0; j < NJ; ++j) fb[j] = frag(raw[j], F.A[j], F.B[j], grp, e);
+                        for (int j = 0; j < NJ; ++j) {
+                            fb[j] = frag(raw[j], F.A[j], F.B[j], grp, e);
+                            if constexpr (EX) fb2[j] = frag(raw[j], F.A2[j], F.B2[j], grp, e);
+                        }
 #pragma unroll
                         for (int i = 0; i < MI; ++i) {
                             if constexpr (kMin) {
@@ -452,6 +484,7 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
                             for (int j = 0; j < NJ; ++j) {
                                 if constexpr (F16) acc[i][j] = mfma(av[i], fb[j], acc[i][j]);
                                 else S[i][j] = mfma(av[i], fb[j], grp == 0 && e == 0 ? float16_t{} : S[i][j]);
+                                if constexpr (EX) S[i][j] = mfma(av[i], fb2[j], S[i][j]);
                             }
                         }
                     }
@@ -554,6 +587,7 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
             }
     }
 
+    void *const copy = a.ct_end[seg] == a.ncol ? a.copy : nullptr;
     auto write_out = [&]() {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
@@ -570,8 +604,10 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
                         const uint32_t r = brow(j);
-                        if (r < rows)
-                            static_cast<float *>(a.out[seg])[size_t(t) * rows + r] = F16 ? round_f16p(fin[i][u][j]) : fin[i][u][j];
+                        if (r >= rows) continue;
+                        const float y = F16 ? round_f16p(fin[i][u][j]) : fin[i][u][j];
+                        static_cast<float *>(a.out[seg])[size_t(t) * rows + r] = y;
+                        if (copy) static_cast<float *>(copy)[size_t(t) * rows + r] = y;
                     }
                 }
             }
@@ -598,9 +634,9 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __syncthreads();
     if (tid == 0)
-        last_flag = __hip_atomic_fetch_add(&a.counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kparts - 1;
+        sh.last_flag = __hip_atomic_fetch_add(&a.counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kparts - 1;
     __syncthreads();
-    if (!last_flag) return;
+    if (!sh.last_flag) return;
     if (tid == 0) __hip_atomic_store(&a.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const float *parts = a.partial + size_t(tile) * kparts * kPart;
     for (uint32_t p0 = 0; p0 < kparts; p0 += 4) {  // four parts per round trip, added in part order
@@ -630,6 +666,30 @@ __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
                 }
     }
     write_out();
+}
+
+// The exact Q6_K form, where batch 2-4 runs here (its own kernels are exact): row-major tensors (9-13 us
+// against 14-15 us there) and V beside Q and K.  On the CDNA4 layout alone it loses (the down projection:
+// 17.0 us at 2-4 tokens against 16.5 on the small-batch kernel, and 17.4 against 15.0 rounded at 5).
+template <int TYPE, int LAYOUT, int ACC, int MI>
+constexpr bool kExact = TYPE == Q6_K && ACC == ACC_FP32 && LAYOUT == ROW_MAJOR && MI == 1;
+
+template <int TYPE, int LAYOUT, int ACC, bool PAIR, int MI, int WK>
+__global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
+    // two LDS objects, so that the compiler does not take a DMA into one for a write to the other
+    __shared__ __attribute__((aligned(16))) u32x4 X0[buf_len<MI, WK>()], X1[buf_len<MI, WK>()];
+    __shared__ Shared sh;
+    skinny_body<TYPE, LAYOUT, ACC, PAIR, MI, WK, kExact<TYPE, LAYOUT, ACC, MI>>(a, work_item(a), X0, X1, sh);
+}
+
+// Q, K and V in one launch where V is Q6_K (FP32 mode): a workgroup takes its matrix's form of the body.
+template <int LAYOUT, int MI, int WK>
+__global__ __launch_bounds__(kThreads) void gemm_skinny_mixed_kernel(const Args a) {
+    __shared__ __attribute__((aligned(16))) u32x4 X0[buf_len<MI, WK>()], X1[buf_len<MI, WK>()];
+    __shared__ Shared sh;
+    const Item item = work_item(a);
+    if (item.seg == a.q6_seg) skinny_body<Q6_K, LAYOUT, ACC_FP32, false, MI, WK, MI == 1>(a, item, X0, X1, sh);
+    else skinny_body<Q4_K, LAYOUT, ACC_FP32, false, MI, WK, false>(a, item, X0, X1, sh);
 }
 
 struct Plan {
@@ -709,6 +769,21 @@ hipError_t launch_mi(const Plan &p, const Args &a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+template <int LAYOUT>
+hipError_t launch_mixed(const Plan &p, const Args &a, hipStream_t stream) {
+    const dim3 grid(p.ntok * p.ncol * p.kparts), block(kThreads);
+    if (p.mi == 1) {
+        if (p.wk == 8) gemm_skinny_mixed_kernel<LAYOUT, 1, 8><<<grid, block, 0, stream>>>(a);
+        else gemm_skinny_mixed_kernel<LAYOUT, 1, 4><<<grid, block, 0, stream>>>(a);
+    } else if (p.mi == 2) {
+        if (p.wk == 8) gemm_skinny_mixed_kernel<LAYOUT, 2, 8><<<grid, block, 0, stream>>>(a);
+        else gemm_skinny_mixed_kernel<LAYOUT, 2, 4><<<grid, block, 0, stream>>>(a);
+    } else {
+        return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 }  // namespace
 
 // Whether this kernel is the faster one.  FP16 mode: by its plan's estimate against the tile kernel's
@@ -735,6 +810,14 @@ bool gemm_skinny_eligible(int type, int layout, int acc, uint32_t cols, const ui
     return cost <= (layout == ROW_MAJOR && type == Q6_K ? 2600u : 960u);
 }
 
+bool skinny_small_batch(int type, int layout, uint32_t cols, uint32_t rows, const void *x, uint32_t batch, bool mixed,
+                        const Tuning &t) {
+    if (type == Q6_K && layout == CDNA4 && !mixed) return false;  // not exact there (kExact)
+    if (batch < 2 || batch > 4 || reinterpret_cast<uintptr_t>(x) % 16) return false;
+    if (t.mt_mfma == 0 || t.mt_parts > 0 || t.mt_slabs > 0 || t.mt_spw > 0) return false;  // a small-batch kernel is asked for
+    return gemm_skinny_eligible(type, layout, ACC_FP32, cols, &rows, 1, batch, false, t);
+}
+
 void gemm_skinny_workspace_need(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair,
                                 int acc, const Tuning &t, size_t *part_floats, size_t *counters) {
     const Plan p = plan_skinny(type, cols, rows, nseg, batch, pair, acc == ACC_FP16, t);
@@ -745,9 +828,12 @@ void gemm_skinny_workspace_need(int type, uint32_t cols, const uint32_t *rows, i
 
 hipError_t launch_gemm_skinny(int type, int layout, int acc, const uint8_t *const *w, const uint8_t *up, void *const *out,
                               const uint32_t *rows, int nseg, const uint16_t *x, uint32_t cols, uint32_t batch,
-                              float *partial, uint32_t *counters, const Tuning &t, hipStream_t stream) {
+                              float *partial, uint32_t *counters, const Tuning &t, hipStream_t stream, int last_type,
+                              void *copy) {
     const bool pair = up != nullptr, f16 = acc == ACC_FP16;
+    const bool mixed = last_type != 0 && last_type != type;  // Q4_K matrices, then one of Q6_K
     if (nseg < 1 || nseg > kMaxSeg || (pair && nseg != 1)) return hipErrorInvalidValue;
+    if (mixed && (type != Q4_K || f16 || pair || nseg < 2)) return hipErrorInvalidValue;
     const Plan p = plan_skinny(type, cols, rows, nseg, batch, pair, f16, t);
     Args a{};
     uint32_t ct = 0;
@@ -760,6 +846,8 @@ hipError_t launch_gemm_skinny(int type, int layout, int acc, const uint8_t *cons
         a.ct_end[s] = ct;
     }
     a.up = up;
+    a.q6_seg = uint32_t(nseg - 1);
+    a.copy = copy;
     a.x = x;
     a.partial = partial;
     a.counters = counters;
@@ -768,6 +856,9 @@ hipError_t launch_gemm_skinny(int type, int layout, int acc, const uint8_t *cons
     a.ntok = p.ntok;
     a.ncol = p.ncol;
     a.kparts = p.kparts;
+    if (mixed)
+        return layout == CDNA4 ? launch_mixed<CDNA4>(p, a, stream)
+               : layout == ROW_MAJOR ? launch_mixed<ROW_MAJOR>(p, a, stream) : hipErrorInvalidValue;
     if (layout == CDNA4) {
         if (pair)
             return f16 ? launch_mi<Q4_K, CDNA4, ACC_FP16, true>(p, a, stream) : launch_mi<Q4_K, CDNA4, ACC_FP32, true>(p, a, stream);

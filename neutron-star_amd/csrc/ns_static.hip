@@ -19,6 +19,8 @@
 // word for bounded cross-workgroup waits that ran out, read by ns_noalloc_status.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include <mutex>
 #include <string>
 
@@ -126,6 +128,15 @@ extern "C" int ns_matmul_noalloc(const void *w, int type, int layout, uint32_t c
     ws.err = sm->err;
     ws.tune = t;
     const hipStream_t s = static_cast<hipStream_t>(stream);
+    // batch 2-4: the same choice of kernel as ns_matmul (its parts: at most one round of workgroups' tiles,
+    // 1 Mi floats, inside the scratch whatever the shape)
+    const bool skinny = batch <= 4 && half_input && skinny_small_batch(type, layout, cols, rows, in, batch, false, t);
+    if (skinny) {
+        size_t f = 0, c = 0;
+        gemm_skinny_workspace_need(type, cols, &rows, 1, batch, false, ACC_FP32, t, &f, &c);
+        if (f > kScratchFloats || c > kScratchCounters) return fail(NS_ERR_UNSUPPORTED, std::string(fn) + ": scratch");
+        need_c = std::max(need_c, c);
+    }
     if (need_c) {
         clear_counters<<<dim3(uint32_t((need_c + 255) / 256)), dim3(256), 0, s>>>(ws.counters, uint32_t(need_c));
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return fail(NS_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
@@ -133,7 +144,11 @@ extern "C" int ns_matmul_noalloc(const void *w, int type, int layout, uint32_t c
     hipError_t e;
     const auto *wb = static_cast<const uint8_t *>(w);
     if (batch == 1) e = launch_gemv(type, layout, wb, nullptr, static_cast<const float *>(in), out, cols, rows, ws, s);
-    else if (batch <= 4) e = launch_gemv_mt(type, layout, wb, nullptr, in, half_input != 0, batch, out, cols, rows, ws, s);
+    else if (skinny) {
+        void *o = out;
+        e = launch_gemm_skinny(type, layout, ACC_FP32, &wb, nullptr, &o, &rows, 1, static_cast<const uint16_t *>(in), cols,
+                               batch, ws.partial, ws.counters, t, s);
+    } else if (batch <= 4) e = launch_gemv_mt(type, layout, wb, nullptr, in, half_input != 0, batch, out, cols, rows, ws, s);
     else e = launch_gemm(type, layout, ACC_FP32, wb, nullptr, static_cast<const uint16_t *>(in), out, cols, rows, batch, ws, s);
     return e == hipSuccess ? NS_OK : fail(NS_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
 }

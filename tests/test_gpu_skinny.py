@@ -100,3 +100,60 @@ def test_skinny_exact_min_term_and_large_sums(ctx, tune):
     want = x.astype(np.float64) @ O.dequant_rows(N.Q4_K, O.ROW_MAJOR, host, cols, rows, 0, rows).astype(np.float64).T
     # 24 block groups of exact products, each sum and product rounded to 24 bits
     assert rel_err(y.cpu().numpy(), want) <= 64 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("batch", [2, 4, 31, 33, 70])
+@pytest.mark.parametrize("v", ["q4", "q6", "tied"])
+@pytest.mark.parametrize("layout", [N.ROW_MAJOR, N.CDNA4], ids=LNAME.get)
+def test_qkv_one_launch(ctx, tune, layout, v, batch):
+    """Q, K and V as column tiles of one launch equal the three projections by themselves up to the sum's
+    order (one launch may split K differently), ragged rows included; Q6_K scales span -128..127, where
+    batch 2-4 has to stay exact (24-bit sums), and the tied V is K bit for bit."""
+    cols, q_rows, kv_rows = 1280, 320, 192
+    if layout == N.ROW_MAJOR:
+        q_rows, kv_rows = 331, 135
+    vt = N.Q6_K if v == "q6" else N.Q4_K
+    host, dev = zip(*(weights(t, 0x57 + i, r, cols, N.ROW_MAJOR) for i, (t, r) in
+                      enumerate(((N.Q4_K, q_rows), (N.Q4_K, kv_rows), (vt, kv_rows)))))
+    if v == "q6":
+        host[2].reshape(-1, 210)[:, 192:208] = np.random.RandomState(3).randint(0, 256, (kv_rows * cols // 256, 16))
+    dev = [torch.from_numpy(np.ascontiguousarray(h if layout == N.ROW_MAJOR else
+                                                 N.retile(h, t, cols, r, N.ROW_MAJOR, layout))).cuda()
+           for h, (t, r) in zip(host, ((N.Q4_K, q_rows), (N.Q4_K, kv_rows), (vt, kv_rows)))]
+    bits, x = tokens(0x5A, batch, cols)
+    out = [torch.full((batch, r), float("nan"), dtype=torch.float32, device="cuda") for r in (q_rows, kv_rows, kv_rows)]
+    ctx.qkv(dev[0], dev[1], None if v == "tied" else dev[2], vt, layout, cols, q_rows, kv_rows, batch, x, *out)
+    torch.cuda.synchronize()
+    got = [o.cpu().numpy() for o in out]
+    xf = bits.view(np.float16).astype(np.float64)
+    for i, (t, r) in enumerate(((N.Q4_K, q_rows), (N.Q4_K, kv_rows), (vt, kv_rows))):
+        if i == 2 and v == "tied":
+            assert np.array_equal(got[2].view(np.uint32), got[1].view(np.uint32))
+            continue
+        want = xf @ O.dequant_rows(t, O.ROW_MAJOR, host[i], cols, r, 0, r).astype(np.float64).T
+        # sums of 24-bit roundings; Q6_K above 4 tokens may round sc*(v-32) to 11 bits
+        bar = 1e-3 if t == N.Q6_K and batch > 4 else 64 * 2.0 ** -24
+        assert rel_err(got[i], want) <= bar, i
+
+
+@pytest.mark.parametrize("batch", [2, 3, 4])
+@pytest.mark.parametrize("qtype,layout", [(N.Q4_K, N.CDNA4), (N.Q4_K, N.ROW_MAJOR), (N.Q6_K, N.ROW_MAJOR)],
+                         ids=["q4k-cdna4", "q4k-rowmajor", "q6k-rowmajor"])
+def test_small_batch_fp16_exact(ctx, qtype, layout, batch):
+    """Batch 2-4 with fp16 x where this kernel takes it: 24-bit sums of exact products, Q6_K scales over the
+    whole int8 range; an x that is not 16-byte aligned gives the same (by the small-batch kernels)."""
+    cols, rows = 2304, 192
+    host = N.synth_weights(qtype, 0x5B, rows, cols).copy()
+    if qtype == N.Q6_K:
+        host.reshape(-1, 210)[:, 192:208] = np.random.RandomState(4).randint(0, 256, (rows * cols // 256, 16))
+    img = host if layout == N.ROW_MAJOR else N.retile(host, qtype, cols, rows, N.ROW_MAJOR, layout)
+    w = torch.from_numpy(np.ascontiguousarray(img)).cuda()
+    bits, x = tokens(0x5C, batch, cols)
+    want = bits.view(np.float16).astype(np.float64) @ O.dequant_rows(qtype, O.ROW_MAJOR, host, cols, rows, 0, rows).astype(np.float64).T
+    shifted = torch.empty(batch * cols + 4, dtype=torch.int16, device="cuda")[4:]
+    shifted.copy_(x.reshape(-1))
+    for xin in (x, shifted):
+        y = torch.empty((batch, rows), dtype=torch.float32, device="cuda")
+        ctx.matmul(w, qtype, layout, cols, rows, batch, xin, y, half_input=True)
+        torch.cuda.synchronize()
+        assert rel_err(y.cpu().numpy(), want) <= 64 * 2.0 ** -24
