@@ -684,15 +684,6 @@ Kernel kernel_of(int type, bool pair) {
     return type == Q4_K ? &gemm_f16_kernel<Q4_K, false, MI> : &gemm_f16_kernel<Q6_K, false, MI>;
 }
 
-int device_cus() {
-    static int cache[64] = {};
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    int &n = cache[dev & 63];
-    if (n == 0 && (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)) n = 256;
-    return n;
-}
-
 // Workgroups of one instance the device holds at once, per device.
 uint64_t resident_wgs(Kernel kernel, int slot) {
     static int cache[64][6] = {};

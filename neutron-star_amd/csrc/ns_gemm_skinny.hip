@@ -697,15 +697,6 @@ struct Plan {
     uint32_t cost;  // the model's estimate, tenths of a microsecond
 };
 
-int device_cus() {
-    static int cache[64] = {};
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    int &n = cache[dev & 63];
-    if (n == 0 && (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)) n = 256;
-    return n;
-}
-
 uint32_t col_tiles(const uint32_t *rows, int nseg, bool pair, uint32_t wk) {
     const uint32_t per = (kWaves / wk) * (pair ? 32 : 64);
     uint32_t n = 0;

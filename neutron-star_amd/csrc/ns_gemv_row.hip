@@ -256,15 +256,6 @@ __global__ __launch_bounds__(64 * MW) void gemv_row_kernel(
     }
 }
 
-int device_cus() {
-    static int cache[64] = {};
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    int &n = cache[dev & 63];
-    if (n == 0 && (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)) n = 256;
-    return n;
-}
-
 }  // namespace
 
 // Rows of up to 256 super-blocks (16 waves of 16); the slab kernel where a test asks for one of its grids.

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <string>
 
@@ -40,6 +41,19 @@ struct Tuning {
 
 // Whether a launch may use a cross-workgroup wait at all (the GPU is not declared shared).
 inline bool waits_allowed(const Tuning &t) { return t.wait_free == 0; }
+
+// CUs of the current device (256 where the runtime cannot say), for the launch plans.
+inline int device_cus() {
+    static std::atomic<int> cache[64] = {};
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    int n = cache[dev & 63].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        cache[dev & 63].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
 
 // Kernels whose workgroups wait for each other (the split-K reduce-scatter of the prefill
 // GEMMs, the one-launch decode block, the multi-layer decode launch) bound every wait.  A

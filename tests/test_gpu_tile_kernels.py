@@ -1,8 +1,11 @@
 """The 128- and 256-token tile GEMMs at the batches that the few-token GEMM takes by default: the
 prefill tests of the other modules once more, on a context that never selects it (gemm_skinny 0)."""
+import numpy as np
 import pytest
 
+import ns_oracle as O
 import nsffn as N
+from helpers import rel_err
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -27,3 +30,25 @@ def ctx():
     yield c
     torch.cuda.synchronize()
     c.close()
+
+
+@pytest.mark.parametrize("qtype,cols,rows,batch", [(N.Q4_K, 2304, 2496, 1000), (N.Q4_K, 6400, 2496, 1020),
+                                                   (N.Q6_K, 4096, 3264, 1200), (N.Q6_K, 8192, 2752, 700)],
+                         ids=["q4k-3parts", "q4k-5parts", "q6k-3parts", "q6k-7parts"])
+def test_planned_odd_parts(ctx, tune, qtype, cols, rows, batch):
+    """FP32-mode splits of K that are no power of two, as the plan chooses them, on ragged tiles: the terms are
+    those of one part, so the two results differ by the order of 24-bit sums; and the repository's 1e-3 against
+    the dequantised weights."""
+    host = N.synth_weights(qtype, 0x61, rows, cols)
+    w = torch.from_numpy(np.ascontiguousarray(N.retile(host, qtype, cols, rows, N.ROW_MAJOR, N.CDNA4))).cuda()
+    bits = N.synth_normal_f16(0x62, batch * cols).reshape(batch, cols)
+    x = torch.from_numpy(bits.view(np.int16)).cuda()
+    y = [torch.full((batch, rows), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2)]
+    for kparts in (0, 1):
+        tune("gemm_kparts", kparts)
+        ctx.ffn_down(w, qtype, N.CDNA4, cols, rows, batch, x, y[kparts], half_input=True, fast_swa=False)
+    torch.cuda.synchronize()
+    planned, one = (t.cpu().numpy() for t in y)
+    assert rel_err(planned, one) <= 64 * 2.0 ** -24
+    want = bits.view(np.float16).astype(np.float32) @ O.dequant_rows(qtype, O.ROW_MAJOR, host, cols, rows, 0, rows).T
+    assert rel_err(planned, want) <= 1e-3
