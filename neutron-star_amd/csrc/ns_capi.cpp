@@ -177,7 +177,8 @@ void model_workspace_need(const Tuning &t, size_t *floats, size_t *counters) {
                     take(f, c);
                 }
             if (sh.rows > 16384) continue;  // the lm-head is a decode GEMV
-            for (uint32_t b = 5; b <= 2048; ++b) {
+            // the plans change at multiples of 16 tokens at most, and the need grows between them
+            for (uint32_t b = 16; b <= 2048; b += 16) {
                 gemm_workspace_need(sh.type, layout, sh.cols, sh.rows, b, sh.pair, t, &f, &c);
                 take(f, c);
             }
