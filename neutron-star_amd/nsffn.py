@@ -137,11 +137,20 @@ def _hptr(a):
     return a.ctypes.data
 
 
+_current_device = _raw_stream = None  # torch's, bound by the first call
+
+
 def _stream(stream):
-    if stream is None:
+    """The stream's handle, or that of torch's current stream on the current device.  Asked by its
+    handle rather than by a torch.cuda.Stream object: 0.4 us instead of 3.1, of 8.5 us that the host
+    spends on a call (a decode attention layer's four small products were bound by that)."""
+    if stream is not None:
+        return stream
+    global _current_device, _raw_stream
+    if _raw_stream is None:
         import torch
-        return torch.cuda.current_stream().cuda_stream
-    return stream
+        _current_device, _raw_stream = torch.cuda.current_device, torch._C._cuda_getCurrentRawStream
+    return _raw_stream(_current_device())
 
 
 def default_threads():
