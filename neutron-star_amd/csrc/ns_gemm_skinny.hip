@@ -28,9 +28,9 @@
 // mode: fragments are exact integers times a power of two (Q4_K sc*q*2^-14; Q6_K sc*(v-32)*2^-16,
 // one rounding past 11 bits as in ns_gemm.hip), summed per super-block in S, and y += d*S in fp32.
 // The Q4_K min term -dmin * sum_g m_g * (sum of x over group g) needs no pass over x ahead of the
-// GEMM: each lane adds up the 16 values per group that its own A fragments hold, in fp32, splits
-// the eight sums exactly into three bf16 pieces, and three bf16 MFMAs multiply them by the m_g
-// (exact in bf16) and add the two lane halves.
+// GEMM: each lane has the 16 values per group that its own A fragments hold added up in fp32 (by
+// 4x4x4 MFMAs), splits the eight sums exactly into three bf16 pieces, and three bf16 MFMAs multiply
+// them by the m_g (exact in bf16) and add the two lane halves.
 #include <algorithm>
 #include <type_traits>
 
@@ -41,8 +41,10 @@
 namespace ns {
 namespace {
 
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
@@ -257,9 +259,12 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
     // ---- x staging: instruction i of wave wc fills rows (wc*ND + i)*RPI .. of group wk's tile; lane l
     // writes position l%CR of row +l/CR and fetches the chunk that the swizzle puts there.
     auto swz = [](uint32_t R) { return CR == 16 ? (R & 15) : ((R >> 1) & 7); };
-    uint32_t xoff[ND];
+    // The swizzle repeats every 16 rows: where registers are short (Q4_K FP32 mode; spills else), the offsets
+    // of the first 16 / RPI instructions serve the others, at an add each.
+    constexpr int NX = Q4 && !F16 && 16 / RPI < ND ? 16 / RPI : ND;
+    uint32_t xoff[NX];
 #pragma unroll
-    for (int i = 0; i < ND; ++i) {
+    for (int i = 0; i < NX; ++i) {
         const uint32_t R = (wc * ND + uint32_t(i)) * RPI + lane / CR, c = (lane % CR) ^ swz(R);
         xoff[i] = ((t0 + R) * cols + 8 * c) * 2;
     }
@@ -267,9 +272,15 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
     auto dma_x = [&](uint32_t sb, bool live, int st) {
         const uint32_t so = (sb * kQK + uint32_t(st) * KS) * 2;
         const rsrc_t xsrc = make_rsrc(a.x, live ? xbytes : 0);
+        uint32_t xo[NX];
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {
+            xo[i] = xoff[i];
+            if constexpr (NX < ND) asm volatile("" : "+v"(xo[i]));  // the sums below are formed here, not kept in registers
+        }
 #pragma unroll
         for (int i = 0; i < ND; ++i)
-            dma16(xsrc, xbuf(st & 1) + wk * (TT * CR) + (wc * ND + uint32_t(i)) * 64, xoff[i], so);
+            dma16(xsrc, xbuf(st & 1) + wk * (TT * CR) + (wc * ND + uint32_t(i)) * 64, xo[i % NX] + uint32_t(i / NX) * 32 * cols, so);
     };
     // A fragment of token tile i: row 32i + ln, chunk 4*gq + 2*hl + e of the stage
     const uint32_t a0 = wk * (TT * CR) + ln * CR, asw = (2 * hl) ^ swz(ln);
@@ -429,14 +440,25 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
     // registers, filled one super-block earlier, changed nothing: 20.3 us either way for the FP16 pair
     // at 5 tokens, and the FP32 pair took 23.0 instead of 21.5.)
     constexpr bool kMin = Q4 && !F16;
-    float one = 1.0f;  // opaque, so that x * one + p stays one mixed-precision FMA (else a convert and an add)
-    asm volatile("" : "+s"(one));
+    auto group_sum = [](int s, half4_t sel, half4_t xv, float4_t c) {  // s is a constant once unrolled
+        return s == 0   ? __builtin_amdgcn_mfma_f32_4x4x4f16(sel, xv, c, 4, 0, 0)
+               : s == 1 ? __builtin_amdgcn_mfma_f32_4x4x4f16(sel, xv, c, 4, 1, 0)
+               : s == 2 ? __builtin_amdgcn_mfma_f32_4x4x4f16(sel, xv, c, 4, 2, 0)
+                        : __builtin_amdgcn_mfma_f32_4x4x4f16(sel, xv, c, 4, 3, 0);
+    };
+    // The group sums of x by 4x4x4 MFMAs (16 independent 4x4 blocks): a lane's four x values are one column
+    // and its column of D stays with the lane, so D's row s takes group 4h + s where A is ones in row s alone.
+    // A's block s (lanes 4s..) holds that selector, broadcast to all blocks.  (As mixed-precision FMAs they
+    // were 256 of the 680 VALU instructions per super-block at 64 tokens, and as many wait states: row-major
+    // projections at 384 tokens 27.6 us then, 26.7 now, Q4_K downs at 64-512 tokens 21.0-91.7 us, 20.0-87.0.)
+    const _Float16 one = lane >> 2 == (lane & 3) ? _Float16(1.0f) : _Float16(0.0f);
+    const half4_t ones{one, one, one, one};
     for (uint32_t it = 0; it < iters; ++it) {
         const uint32_t sb = sb_of(it), sbn = sb_of(it + 1);
         const bool valid = sb < sb1, more = sbn < sb1;  // wave-uniform
         Factors F;
         float16_t S[F16 ? 1 : MI][NJ];
-        float P[kMin ? MI : 1][8];
+        float4_t P[kMin ? MI : 1][2];  // group sums of this lane half's x: groups 4h + slot
 #pragma unroll
         for (int st = 0; st < NS; ++st) {
             __builtin_amdgcn_sched_barrier(0);
@@ -475,10 +497,9 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
 #pragma unroll
                         for (int i = 0; i < MI; ++i) {
                             if constexpr (kMin) {
-                                float p = e == 0 ? 0.f : P[i][grp];
-#pragma unroll
-                                for (int k = 0; k < 8; ++k) p = __builtin_fmaf(float(av[i][k]), one, p);
-                                P[i][grp] = p;
+                                float4_t p = grp % 4 == 0 && e == 0 ? float4_t{} : P[i][grp / 4];
+                                p = group_sum(grp % 4, ones, __builtin_shufflevector(av[i], av[i], 0, 1, 2, 3), p);
+                                P[i][grp / 4] = group_sum(grp % 4, ones, __builtin_shufflevector(av[i], av[i], 4, 5, 6, 7), p);
                             }
 #pragma unroll
                             for (int j = 0; j < NJ; ++j) {
@@ -536,7 +557,7 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
                             uint32_t pb[3][2];
 #pragma unroll
                             for (int u = 0; u < 2; ++u) {
-                                float r = P[i][2 * k + u];
+                                float r = P[i][k / 2][2 * (k & 1) + u];
 #pragma unroll
                                 for (int z = 0; z < 3; ++z) {
                                     pb[z][u] = __builtin_bit_cast(uint32_t, r) & 0xffff0000u;

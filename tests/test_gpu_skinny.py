@@ -157,3 +157,26 @@ def test_small_batch_fp16_exact(ctx, qtype, layout, batch):
         ctx.matmul(w, qtype, layout, cols, rows, batch, xin, y, half_input=True)
         torch.cuda.synchronize()
         assert rel_err(y.cpu().numpy(), want) <= 64 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")], ids=str)
+@pytest.mark.parametrize("layout", [N.CDNA4, N.ROW_MAJOR], ids=LNAME.get)
+@pytest.mark.parametrize("batch", [32, 50])
+def test_group_sums_keep_tokens_apart(ctx, layout, batch, value):
+    """Q4_K, FP32 mode: x values that are not finite reach their own token's outputs alone, though the group
+    sums of a wave's tokens share MFMA instructions; the others are bit for bit what they are without them."""
+    cols, rows = 1280, 192
+    _, w = weights(N.Q4_K, 0x5D, rows, cols, layout)
+    _, x = tokens(0x5E, batch, cols)
+    bad = x.clone()
+    for t, c in ((3, 17), (batch - 1, cols - 1)):
+        bad.view(torch.float16)[t, c] = value
+    y = [torch.empty((batch, rows), dtype=torch.float32, device="cuda") for _ in range(2)]
+    for xin, out in zip((x, bad), y):
+        ctx.ffn_down(w, N.Q4_K, layout, cols, rows, batch, xin, out, half_input=True, fast_swa=False)
+    torch.cuda.synchronize()
+    clean, got = (t.cpu().numpy() for t in y)
+    hit = np.zeros(batch, bool)
+    hit[[3, batch - 1]] = True
+    assert np.array_equal(got[~hit].view(np.uint32), clean[~hit].view(np.uint32))
+    assert not np.isfinite(got[hit]).any()
