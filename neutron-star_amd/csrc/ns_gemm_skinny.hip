@@ -195,10 +195,13 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
     // byte offset, past voff + the super-block's uniform part, of chunk c
     auto chunk = [](uint32_t c) { return c * (ROW ? 16u : 1024u); };
     constexpr uint32_t kBlkStep = ROW ? block_bytes(TYPE) : kRegion;
-    // live = 0: a range of no bytes, so the loads read zeros and touch no memory (past the last block)
+    // live = 0 (past the last block): the range is the tensor's first block step, from uniform offset 0, so all
+    // but the first rows' loads read zeros and touch no memory.  No instruction's uniform offset passes the
+    // range: the check compares with their difference.
     auto load_raw = [&](uint32_t sb, bool live, Raw (&raw)[NJ]) {
-        const uint32_t so = sb * kBlkStep;
-        const rsrc_t wsrc0 = make_rsrc(w0, live ? wbytes : 0), wsrc1 = make_rsrc(w1, live ? wbytes : 0);
+        const uint32_t so = live ? sb * kBlkStep : 0;
+        const rsrc_t wsrc0 = make_rsrc(w0, live ? wbytes : kBlkStep),
+                     wsrc1 = make_rsrc(w1, live ? wbytes : kBlkStep);
         auto wsrc = [&](int j) { return (PAIR && j == 1) ? wsrc1 : wsrc0; };
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
@@ -270,7 +273,7 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
     }
     auto xbuf = [&](int b) -> u32x4 * { return b ? X1 : X0; };
     auto dma_x = [&](uint32_t sb, bool live, int st) {
-        const uint32_t so = (sb * kQK + uint32_t(st) * KS) * 2;
+        const uint32_t so = live ? (sb * kQK + uint32_t(st) * KS) * 2 : 0;
         const rsrc_t xsrc = make_rsrc(a.x, live ? xbytes : 0);
         uint32_t xo[NX];
 #pragma unroll
