@@ -143,7 +143,10 @@ struct Plan {
     uint32_t S, M, P, KP;
 };
 
-template <int TYPE, bool PAIR, bool XH>
+// STREAM: a wave takes slab after slab of its column group, a whole grid apart, against the x staged once; its
+// prefetch runs on into the next slab (stream_grid).  What bounds it then is the double buffer: a wave has one
+// super-block (13 KB) in flight while it unpacks the other, ~5.6 TB/s over the lm-head.
+template <int TYPE, bool PAIR, bool XH, bool STREAM>
 __global__ __launch_bounds__(kMaxWaves * 64) void gemv_mfma_kernel(
     const uint8_t *__restrict__ w0, const uint8_t *__restrict__ w1, const void *__restrict__ x, uint32_t batch,
     void *__restrict__ out, uint32_t rows, uint32_t nb, Plan pl, float *__restrict__ partial,
@@ -176,12 +179,9 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_mfma_kernel(
     // lane part of the weight offsets: 8 bytes at chunk (o >> 1) of row n, half (o & 1)
     const uint32_t vq = ((o >> 1) * kRowTile + n) * 16 + 8 * (o & 1);
     const uint32_t vrow = n * 16;  // 16-byte piece of row n in a chunk
-    auto region = [&](uint32_t sb) {
-        const uint32_t s = __builtin_elementwise_min(slab, slabs - 1);
-        return uint32_t(region_offset(TYPE, s, sb, nb));
-    };
-    auto load = [&](uint32_t sb, RawOf<TYPE> &r) {
-        const uint32_t base = __builtin_amdgcn_readfirstlane(region(sb));
+    auto load_at = [&](uint32_t sl, uint32_t sb, RawOf<TYPE> &r) {
+        const uint32_t s = __builtin_elementwise_min(sl, slabs - 1);
+        const uint32_t base = __builtin_amdgcn_readfirstlane(uint32_t(region_offset(TYPE, s, sb, nb)));
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const uint32_t tb = base + 256 * t;  // rows 16t.. of the slab
@@ -199,6 +199,8 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_mfma_kernel(
             }
         }
     };
+
+    auto load = [&](uint32_t sb, RawOf<TYPE> &r) { load_at(slab, sb, r); };
 
     // ---- prologue: the first super-block's weights in flight, then x staged in LDS -------
     RawOf<TYPE> ra, rb;
@@ -465,8 +467,42 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_mfma_kernel(
         }
     };
 
+    // ---- combine: the four D quarters (planes, groups) of each row, then the token scale -------
+    float mine[NT];
+    auto combine = [&]() {
+        float tot[4][4];  // [tile][token] for row 16*tile + n
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                float s = acc[t][v];
+                s += __shfl_xor(s, 16);
+                s += __shfl_xor(s, 32);
+                tot[t][v] = s * oscale[v];
+            }
+        // lane l takes row l of the slab (tile l >> 4): choices between values, not between array elements
+        // (which the compiler makes an address in scratch, or branches over the lanes)
+#pragma unroll
+        for (int v = 0; v < NT; ++v) {
+            const float t0 = tot[0][v], t1 = tot[1][v], t2 = tot[2][v], t3 = tot[3][v];
+            const float lo = lane & 16 ? t1 : t0, hi = lane & 16 ? t3 : t2;
+            mine[v] = lane & 32 ? hi : lo;
+        }
+    };
+    auto store_out = [&](uint32_t sl, const float (&gv)[NT], const float (&uv)[NT]) {
+        const uint32_t row = sl * kRowTile + lane;
+#pragma unroll
+        for (int v = 0; v < NT; ++v) {
+            if (uint32_t(v) >= batch) break;
+            if constexpr (PAIR)
+                static_cast<_Float16 *>(out)[size_t(v) * rows + row] = _Float16(gelu_tanh(gv[v]) * uv[v]);
+            else
+                static_cast<float *>(out)[size_t(v) * rows + row] = gv[v];
+        }
+    };
+
     // ---- main loop: compute one super-block while the next one's weights load ---------------
-    // Two buffers alternate.  The first iteration is peeled: its prefetch is unconditional
+    // (one slab per wave; STREAM's is the first below)  Two buffers alternate.  The first iteration is peeled: its prefetch is unconditional
     // (clamped into the tensor; a wave with one super-block drops it) and pinned by a signal
     // fence, so it leaves right after the staging barrier.  Entering the loop with the
     // prologue's buffer instead made the compiler copy that buffer into the loop's registers,
@@ -476,6 +512,37 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_mfma_kernel(
     // which serialises load and compute.  The scheduling barrier keeps the prefetch ahead of the
     // compute.  Every wave runs it (one past the last slab on the clamped last slab, its results
     // dropped), and every wave has at least one super-block (the plan keeps P <= nsb).
+    if constexpr (STREAM) {  // P = KP = 1, nb >= 2: no barrier follows, so waves leave on their own
+        if (!active) return;
+        const uint32_t stride = gridDim.x * pl.S;
+        uint32_t sl = slab, sb = 0;  // the unit being computed
+        auto finish = [&]() {
+            combine();
+            store_out(sl, mine, mine);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+        };
+        // one unit: the next one's weights requested first (behind the wave's last unit its own again, from
+        // the caches and unused: a copy of the code without the request cost registers, and spilled)
+        auto unit = [&](const RawOf<TYPE> &cur, RawOf<TYPE> &next) -> bool {
+            const bool end = sb + 1 == nb, last = end && sl + stride >= slabs;
+            load_at(end && !last ? sl + stride : sl, last ? sb : end ? 0 : sb + 1, next);
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(cur, sb);
+            __builtin_amdgcn_sched_barrier(0);
+            ++sb;
+            if (end) {
+                finish();
+                sl += stride;
+                sb = 0;
+            }
+            return !last;
+        };
+        while (unit(ra, rb) && unit(rb, ra)) {
+        }
+        return;
+    }
     {
         uint32_t sb = wsb0;
         const bool more = sb + 1 != wsb1;
@@ -504,37 +571,9 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_mfma_kernel(
         }
     }
 
-    // ---- combine: the four D quarters (planes, groups) of each row, then the token scale -------
-    float tot[4][4];  // [tile][token] for row 16*tile + n
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            float s = acc[t][v];
-            s += __shfl_xor(s, 16);
-            s += __shfl_xor(s, 32);
-            tot[t][v] = s * oscale[v];
-        }
-    // lane l takes row l of the slab (tile l >> 4)
-    float mine[NT];
-#pragma unroll
-    for (int v = 0; v < NT; ++v) {
-        const uint32_t t = lane >> 4;
-        mine[v] = t == 0 ? tot[0][v] : t == 1 ? tot[1][v] : t == 2 ? tot[2][v] : tot[3][v];
-    }
-    const uint32_t row = slab * kRowTile + lane;
-    auto store_out = [&](const float (&gv)[NT], const float (&uv)[NT]) {
-#pragma unroll
-        for (int v = 0; v < NT; ++v) {
-            if (uint32_t(v) >= batch) break;
-            if constexpr (PAIR)
-                static_cast<_Float16 *>(out)[size_t(v) * rows + row] = _Float16(gelu_tanh(gv[v]) * uv[v]);
-            else
-                static_cast<float *>(out)[size_t(v) * rows + row] = gv[v];
-        }
-    };
+    combine();
     if (pl.P == 1 && M == 1 && pl.KP == 1) {
-        if (active) store_out(mine, mine);
+        if (active) store_out(slab, mine, mine);
         return;
     }
 
@@ -586,12 +625,12 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_mfma_kernel(
                                                  __HIP_MEMORY_SCOPE_AGENT);
         if (lane == 0) __hip_atomic_store(&counters[slab], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    store_out(r[0], r[M - 1]);
+    store_out(slab, r[0], r[M - 1]);
 }
 
-template <int TYPE, bool PAIR, bool XH>
+template <int TYPE, bool PAIR, bool XH, bool STREAM = false>
 constexpr auto mfma_kernel() {
-    return &gemv_mfma_kernel<TYPE, PAIR, XH>;
+    return &gemv_mfma_kernel<TYPE, PAIR, XH, STREAM>;
 }
 
 // Plan: workgroups of four waves, so that two fill a CU (the kernel's ~250 VGPRs allow two waves
@@ -628,9 +667,23 @@ Plan plan_mfma(uint32_t rows, uint32_t nb, bool pair, const Tuning &t) {
     return p;
 }
 
+// Workgroups of the streaming form, or 0 for one slab per wave: where the plan's grid takes more than one
+// round of two workgroups per CU, whose later workgroups would stage x again with little in flight.  MI355X,
+// the 262,144-row Q6_K lm-head (1,024 workgroups, 512 streaming) at 3 fp32 tokens: 148.1 us before, 146.4 now.
+uint32_t stream_grid(const Plan &p, uint32_t nwg, uint32_t nb) {
+    const uint32_t room = 2 * uint32_t(device_cus());
+    if (p.M != 1 || p.P != 1 || p.KP != 1 || nb < 2 || nwg <= room) return 0;
+    const uint32_t steps = (nwg + room - 1) / room;
+    return (nwg + steps - 1) / steps;
+}
+
 template <class Fn>
-auto dispatch_mfma(int type, bool pair, bool xh, Fn &&fn) {
+auto dispatch_mfma(int type, bool pair, bool xh, bool stream, Fn &&fn) {
     if (pair) return fn(mfma_kernel<Q4_K, true, true>());
+    if (stream) {
+        if (type == Q4_K) return xh ? fn(mfma_kernel<Q4_K, false, true, true>()) : fn(mfma_kernel<Q4_K, false, false, true>());
+        return xh ? fn(mfma_kernel<Q6_K, false, true, true>()) : fn(mfma_kernel<Q6_K, false, false, true>());
+    }
     if (type == Q4_K) return xh ? fn(mfma_kernel<Q4_K, false, true>()) : fn(mfma_kernel<Q4_K, false, false>());
     return xh ? fn(mfma_kernel<Q6_K, false, true>()) : fn(mfma_kernel<Q6_K, false, false>());
 }
@@ -664,8 +717,9 @@ hipError_t launch_gemv_mfma(int type, const uint8_t *w, const uint8_t *up, const
     if (p.KP > 1 && (ws.partial_floats < size_t(slabs) * p.KP * p.M * NT * 64 || ws.counter_count < slabs))
         return hipErrorInvalidValue;
     const uint32_t nwg = (slabs + p.S - 1) / p.S * p.KP;
-    return dispatch_mfma(type, pair, xh, [&](auto k) {
-        k<<<dim3(nwg), dim3(p.S * p.M * p.P * 64), 0, stream>>>(w, up, x, batch, out, rows, nb, p, ws.partial,
+    const uint32_t sgrid = stream_grid(p, nwg, nb);
+    return dispatch_mfma(type, pair, xh, sgrid != 0, [&](auto k) {
+        k<<<dim3(sgrid ? sgrid : nwg), dim3(p.S * p.M * p.P * 64), 0, stream>>>(w, up, x, batch, out, rows, nb, p, ws.partial,
                                                                  ws.counters);
         return hipGetLastError();
     });
