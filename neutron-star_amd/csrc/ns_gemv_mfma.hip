@@ -480,13 +480,19 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_mfma_kernel(
                 s += __shfl_xor(s, 32);
                 tot[t][v] = s * oscale[v];
             }
-        // lane l takes row l of the slab (tile l >> 4): choices between values, not between array elements
-        // (which the compiler makes an address in scratch, or branches over the lanes)
+        // lane l takes row l of the slab (tile l >> 4).  In the loop of STREAM the choice is between values and
+        // not between array elements, which the compiler made branches over the lanes or an address in
+        // scratch; elsewhere that form changed nothing (FFN block at 3 tokens 40.3-41.0 us against 40.6).
 #pragma unroll
         for (int v = 0; v < NT; ++v) {
-            const float t0 = tot[0][v], t1 = tot[1][v], t2 = tot[2][v], t3 = tot[3][v];
-            const float lo = lane & 16 ? t1 : t0, hi = lane & 16 ? t3 : t2;
-            mine[v] = lane & 32 ? hi : lo;
+            if constexpr (STREAM) {
+                const float t0 = tot[0][v], t1 = tot[1][v], t2 = tot[2][v], t3 = tot[3][v];
+                const float lo = lane & 16 ? t1 : t0, hi = lane & 16 ? t3 : t2;
+                mine[v] = lane & 32 ? hi : lo;
+            } else {
+                const uint32_t t = lane >> 4;
+                mine[v] = t == 0 ? tot[0][v] : t == 1 ? tot[1][v] : t == 2 ? tot[2][v] : tot[3][v];
+            }
         }
     };
     auto store_out = [&](uint32_t sl, const float (&gv)[NT], const float (&uv)[NT]) {
