@@ -443,6 +443,10 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
     // registers, filled one super-block earlier, changed nothing: 20.3 us either way for the FP16 pair
     // at 5 tokens, and the FP32 pair took 23.0 instead of 21.5.)
     constexpr bool kMin = Q4 && !F16;
+    // The 32-token tile (which also takes batch 2-4) has the registers for two chains of sums, one per half of
+    // the super-block: error against 64 bits of Q4_K projections at 2-4 tokens 1.55e-7 in one chain, 1.28e-7 in
+    // two (the small-batch kernels: 1.45e-7 on matrix cores, 1.19e-7 on the VALU), at the same times.
+    constexpr bool kTwo = !F16 && MI == 1 && !EX;
     auto group_sum = [](int s, half4_t sel, half4_t xv, float4_t c) {  // s is a constant once unrolled
         return s == 0   ? __builtin_amdgcn_mfma_f32_4x4x4f16(sel, xv, c, 4, 0, 0)
                : s == 1 ? __builtin_amdgcn_mfma_f32_4x4x4f16(sel, xv, c, 4, 1, 0)
@@ -460,7 +464,7 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
         const uint32_t sb = sb_of(it), sbn = sb_of(it + 1);
         const bool valid = sb < sb1, more = sbn < sb1;  // wave-uniform
         Factors F;
-        float16_t S[F16 ? 1 : MI][NJ];
+        float16_t S[F16 ? 1 : MI][NJ], S2[kTwo ? NJ : 1];
         float4_t P[kMin ? MI : 1][2];  // group sums of this lane half's x: groups 4h + slot
 #pragma unroll
         for (int st = 0; st < NS; ++st) {
@@ -507,6 +511,7 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
 #pragma unroll
                             for (int j = 0; j < NJ; ++j) {
                                 if constexpr (F16) acc[i][j] = mfma(av[i], fb[j], acc[i][j]);
+                                else if (kTwo && grp >= 4) S2[kTwo ? j : 0] = mfma(av[i], fb[j], grp == 4 && e == 0 ? float16_t{} : S2[kTwo ? j : 0]);
                                 else S[i][j] = mfma(av[i], fb[j], grp == 0 && e == 0 ? float16_t{} : S[i][j]);
                                 if constexpr (EX) S[i][j] = mfma(av[i], fb2[j], S[i][j]);
                             }
@@ -551,7 +556,7 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
 #pragma unroll
                     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_fmaf(d[j], S[i][j][v], acc[i][j][v]);
+                        for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_fmaf(d[j], kTwo ? S[i][j][v] + S2[kTwo ? j : 0][v] : S[i][j][v], acc[i][j][v]);
                     if constexpr (kMin) {
                         // P = hi + mid + lo, each exact in bf16 (8 of the 24 bits at a time)
                         u32x4 pc[3];
