@@ -11,7 +11,7 @@
 // Work split.  A workgroup is 8 waves = WC column groups x WK groups of super-blocks.  Each wave
 // owns 64 columns (2 MFMA tiles; for the gate/up pair 32 gate rows and the same 32 up rows) and
 // walks every WK-th super-block of the workgroup's K range alone; the WK partial sums meet in LDS
-// at the end, in wk order.  So 64 * WC columns keep all eight waves streaming weights, and the
+// at the end, in a fixed order.  So 64 * WC columns keep all eight waves streaming weights, and the
 // gate/up pair needs no reduction between workgroups.  A shape with too few columns to fill the
 // device splits K over kparts workgroups as well; the last of them to arrive adds the parts in
 // part order (no workgroup ever waits for another).
@@ -443,10 +443,12 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
     // registers, filled one super-block earlier, changed nothing: 20.3 us either way for the FP16 pair
     // at 5 tokens, and the FP32 pair took 23.0 instead of 21.5.)
     constexpr bool kMin = Q4 && !F16;
-    // The 32-token tile (which also takes batch 2-4) has the registers for two chains of sums, one per half of
-    // the super-block: error against 64 bits of Q4_K projections at 2-4 tokens 1.55e-7 in one chain, 1.28e-7 in
-    // two (the small-batch kernels: 1.45e-7 on matrix cores, 1.19e-7 on the VALU), at the same times.
-    constexpr bool kTwo = !F16 && MI == 1 && !EX;
+    // The 32-token tile (which also takes batch 2-4) has the registers for short chains of sums: one per quarter
+    // of the super-block, added up in T, and one for EX's small second fragments.  Together with the pairwise sum
+    // over the waves and the min term's small pieces first, error against 64 bits of row-major projections
+    // (3840 x 4096, 3 tokens): Q4_K 1.55e-7 in one chain per super-block, 1.28e-7 in two, 1.09e-7 now; Q6_K
+    // 1.42e-7 in one, 0.93e-7 now (the small-batch VALU kernel: 1.12e-7 and 1.04e-7), at the same times.
+    constexpr bool kShort = !F16 && MI == 1;
     auto group_sum = [](int s, half4_t sel, half4_t xv, float4_t c) {  // s is a constant once unrolled
         return s == 0   ? __builtin_amdgcn_mfma_f32_4x4x4f16(sel, xv, c, 4, 0, 0)
                : s == 1 ? __builtin_amdgcn_mfma_f32_4x4x4f16(sel, xv, c, 4, 1, 0)
@@ -464,7 +466,7 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
         const uint32_t sb = sb_of(it), sbn = sb_of(it + 1);
         const bool valid = sb < sb1, more = sbn < sb1;  // wave-uniform
         Factors F;
-        float16_t S[F16 ? 1 : MI][NJ], S2[kTwo ? NJ : 1];
+        float16_t S[F16 ? 1 : MI][NJ], S2[EX ? NJ : 1], T[kShort ? NJ : 1];
         float4_t P[kMin ? MI : 1][2];  // group sums of this lane half's x: groups 4h + slot
 #pragma unroll
         for (int st = 0; st < NS; ++st) {
@@ -511,9 +513,11 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
 #pragma unroll
                             for (int j = 0; j < NJ; ++j) {
                                 if constexpr (F16) acc[i][j] = mfma(av[i], fb[j], acc[i][j]);
-                                else if (kTwo && grp >= 4) S2[kTwo ? j : 0] = mfma(av[i], fb[j], grp == 4 && e == 0 ? float16_t{} : S2[kTwo ? j : 0]);
-                                else S[i][j] = mfma(av[i], fb[j], grp == 0 && e == 0 ? float16_t{} : S[i][j]);
-                                if constexpr (EX) S[i][j] = mfma(av[i], fb2[j], S[i][j]);
+                                else S[i][j] = mfma(av[i], fb[j], grp % (kShort ? 2 : 8) == 0 && e == 0 ? float16_t{} : S[i][j]);
+                                if constexpr (EX) S2[j] = mfma(av[i], fb2[j], grp == 0 && e == 0 ? float16_t{} : S2[j]);
+                                if constexpr (kShort) {
+                                    if (grp % 2 == 1 && e == 1) T[j] = grp == 1 ? S[i][j] : T[j] + S[i][j];
+                                }
                             }
                         }
                     }
@@ -556,7 +560,10 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
 #pragma unroll
                     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_fmaf(d[j], kTwo ? S[i][j][v] + S2[kTwo ? j : 0][v] : S[i][j][v], acc[i][j][v]);
+                        for (int v = 0; v < 16; ++v) {
+                            const float sum = !kShort ? S[i][j][v] : EX ? T[kShort ? j : 0][v] + S2[EX ? j : 0][v] : T[kShort ? j : 0][v];
+                            acc[i][j][v] = __builtin_fmaf(d[j], sum, acc[i][j][v]);
+                        }
                     if constexpr (kMin) {
                         // P = hi + mid + lo, each exact in bf16 (8 of the 24 bits at a time)
                         u32x4 pc[3];
@@ -579,8 +586,9 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
                         for (int j = 0; j < NJ; ++j) {
                             float16_t mn{};
 #pragma unroll
-                            for (int z = 0; z < 3; ++z)
-                                mn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8_t, pc[z]), mb[j], mn, 0, 0, 0);
+                            for (int z = 0; z < 3; ++z)  // MI 1: the smallest piece first (MI 2 has no register to spare)
+                                mn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8_t, pc[kShort ? 2 - z : z]), mb[j],
+                                                                             mn, 0, 0, 0);
 #pragma unroll
                             for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_fmaf(-dmin[j], mn[v], acc[i][j][v]);
                         }
@@ -609,10 +617,19 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
         for (int u = 0; u < VP; ++u)
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
-                float s = 0.f;
+                float s[WK];
 #pragma unroll
-                for (int k = 0; k < WK; ++k) s += red[(((uint32_t(k) * WC + wc) * 16 + wk * VP + u) * NJ + j) * 64 + lane];
-                fin[i][u][j] = F16 ? s * inv_c[j] : s;
+                for (int k = 0; k < WK; ++k) s[k] = red[(((uint32_t(k) * WC + wc) * 16 + wk * VP + u) * NJ + j) * 64 + lane];
+                if constexpr (kShort) {  // pairwise
+#pragma unroll
+                    for (int m = 1; m < WK; m *= 2)
+#pragma unroll
+                        for (int k = 0; k < WK; k += 2 * m) s[k] += s[k + m];
+                } else {
+#pragma unroll
+                    for (int k = 1; k < WK; ++k) s[0] += s[k];
+                }
+                fin[i][u][j] = F16 ? s[0] * inv_c[j] : s[0];
             }
     }
 

@@ -180,3 +180,33 @@ def test_group_sums_keep_tokens_apart(ctx, layout, batch, value):
     hit[[3, batch - 1]] = True
     assert np.array_equal(got[~hit].view(np.uint32), clean[~hit].view(np.uint32))
     assert not np.isfinite(got[hit]).any()
+
+
+def sum_error(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("batch", [2, 3, 4])
+@pytest.mark.parametrize("qtype,layout", [(N.Q4_K, N.CDNA4), (N.Q4_K, N.ROW_MAJOR), (N.Q6_K, N.ROW_MAJOR)],
+                         ids=["q4k-cdna4", "q4k-rowmajor", "q6k-rowmajor"])
+@pytest.mark.parametrize("rows,cols", [(2048, 3840), (1024, 15360)])
+def test_small_batch_sums_no_worse(ctx, tune, qtype, layout, rows, cols, batch):
+    """Batch 2-4 with fp16 x: the sums are no further from 64 bits than the small-batch kernels', for one matrix
+    and for Q, K and V in one launch.  5% above them is the spread of a 2-norm over 12,288 roundings and more."""
+    host, w = weights(qtype, 0x5F, rows, cols, layout)
+    dense = torch.empty((rows, cols), dtype=torch.float32, device="cuda")
+    ctx.dequant(w, qtype, layout, cols, rows, 0, rows, out_f32=dense)
+    wt = dense.double().t().contiguous()
+    _, q4 = (host, w) if qtype == N.Q4_K else weights(N.Q4_K, 0x60, rows, cols, layout)
+    err = {}
+    for skinny in (-1, 0):
+        tune("gemm_skinny", skinny)
+        err[skinny] = np.zeros(2)
+        for seed in range(6):
+            _, x = tokens(0x61 + seed, batch, cols)
+            want = x.view(torch.float16).double() @ wt
+            y, q, k, v = (torch.empty((batch, rows), dtype=torch.float32, device="cuda") for _ in range(4))
+            ctx.matmul(w, qtype, layout, cols, rows, batch, x, y, half_input=True)
+            ctx.qkv(q4, q4, w, qtype, layout, cols, rows, rows, batch, x, q, k, v)
+            err[skinny] += [sum_error(y, want), sum_error(v, want)]
+    assert (err[-1] <= 1.05 * err[0]).all(), err
