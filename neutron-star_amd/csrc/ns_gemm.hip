@@ -872,12 +872,11 @@ struct GemmPlan {
     uint32_t ntok, ncol, kparts;
 };
 
-// Output tiles and split of K (the 3840-row down projection has only 4 x 15 tiles at batch 1024).  Up
-// to the power of two that covers most of the CUs, the split with the least estimate, in tenths of a
-// microsecond fitted to MI355X timings of the down projections (one workgroup per CU): a round costs 30 us
-// and 4.9 per super-block, and a last arrival reads the parts (2 us each) where the reduce-scatter
-// cannot run.  What it avoids is a second round that is nearly empty: Q6_K downs at 513-768 tokens
-// (45 tiles) in 8 parts 168-189 us, in 4 parts 114-118; at 1300 (90 tiles) in 4 parts 260, in 2 parts 212.
+// Output tiles and split of K: enough workgroups to cover most of the 256 CUs
+// (the 3840-row down projection has only 4 x 15 tiles at batch 1024).  Fewer parts would take less time
+// where they leave no nearly empty second round (Q6_K downs at 600 tokens, 45 tiles: 8 parts 168-189 us,
+// 4 parts 114-118), but a part is one chain of fp32 sums: against 64 bits those outputs are 2.85e-7 off in
+// 8 parts, 4.05e-7 in 4 (scales of 5 bits; with larger ones the tile's rounding, 1.4e-4, hides it).
 GemmPlan plan_gemm(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t) {
     GemmPlan p;
     p.ntok = (batch + TT - 1) / TT;
@@ -885,17 +884,7 @@ GemmPlan plan_gemm(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, cons
     p.ncol = (rows + rows_per_tile - 1) / rows_per_tile;
     const uint32_t nb = cols / kQK, tiles = p.ntok * p.ncol;
     p.kparts = 1;
-    uint32_t most = 1, best = ~0u;
-    while (tiles * most < 200 && most * 2 <= nb / 4) most *= 2;
-    const uint32_t cus = uint32_t(device_cus());
-    for (uint32_t kp = 1; kp <= most; ++kp) {
-        const bool scatter = MI % kp == 0 && tiles * kp <= cus;
-        const uint32_t cost = (tiles * kp + cus - 1) / cus * (300 + (nb + kp - 1) / kp * 49) + (scatter ? 0 : kp * 20);
-        if (cost < best) {
-            best = cost;
-            p.kparts = kp;
-        }
-    }
+    while (tiles * p.kparts < 200 && p.kparts * 2 <= nb / 4) p.kparts *= 2;
     if (t.gemm_kparts >= 1 && uint32_t(t.gemm_kparts) <= nb) p.kparts = uint32_t(t.gemm_kparts);
     // one split-K part (padded to whole tiles) must stay under 4 GiB: 32-bit offsets in the kernel
     if (uint64_t(pair ? 2 : 1) * p.ntok * TT * p.ncol * rows_per_tile * 4 >= (uint64_t(1) << 32)) p.kparts = 1;

@@ -574,26 +574,15 @@ RegPlan plan_reg(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const 
     p.ncol = (rows + rows_per_tile - 1) / rows_per_tile;
     const uint32_t nb = cols / kQK, tiles = p.ntok * p.ncol;
     p.kparts = 1;
-    // Two workgroups per CU: up to the power of two that covers most of them, the split of K with the least
-    // estimate, in tenths of a microsecond fitted to MI355X timings of the gate/up pair and the down
-    // projections.  A super-block costs 5.3 us while every CU has one workgroup at most, 7.3 to 9.3 above; a
-    // round 3 us more; a last arrival reads every part where the reduce-scatter cannot run.  The power of two
-    // alone (before / now): downs at 520-640 tokens (75 tiles) 8 parts 148 us / 6 parts 113, 700-768 (90
-    // tiles) 8 parts 167 / 5 parts 128, 1300 (165 tiles) 4 parts 232 / 3 parts 199; the pair at 257-384 (360
-    // tiles) 2 parts 139 / 1 part 122.
-    uint32_t most = 1, best = ~0u;
-    while (tiles * most < 400 && most * 2 <= nb / 2) most *= 2;
-    const uint32_t cus = uint32_t(device_cus()), slots = 2 * cus;
-    for (uint32_t kp = 1; kp <= most; ++kp) {
-        const uint32_t n = tiles * kp, sb = (nb + kp - 1) / kp, rest = n % slots;
-        uint32_t cost = n / slots * (30 + sb * 93);
-        if (rest > 0) cost += 30 + sb * (rest <= cus ? 53 : 73 + 20 * (rest - cus) / cus);
-        if (kp > 1) cost += kp == uint32_t(MI) && n <= slots ? 40 : 40 + 25 * kp;
-        if (cost < best) {
-            best = cost;
-            p.kparts = kp;
-        }
-    }
+    // two workgroups per CU on 256 CUs: split K until the grid covers most of them.  Plain outputs keep that
+    // many parts although fewer would leave no nearly empty second round (downs at 520-640 tokens, 75 tiles:
+    // 8 parts 148 us, 6 parts 113): a part is one chain of fp32 sums, and fewer parts are further from 64 bits.
+    while (tiles * p.kparts < 400 && p.kparts * 2 <= nb / 2) p.kparts *= 2;
+    // The pair's h is rounded to fp16 (2.1e-4), which no order of the sums shows in.  From 256 tiles on, two
+    // parts are a second round and one is not; one part is the faster up to 15 super-blocks (3,840 x 15,360 at
+    // 257-384 tokens, 360 tiles: 122 us against 139; 256-399 tiles: 0.54-1.00 of the time up to 15 super-blocks,
+    // 0.96-1.05 at 16, 1.03-1.37 at 60).
+    if (pair && p.kparts == 2 && tiles >= 256 && nb <= 15) p.kparts = 1;
     if (t.gemm_kparts >= 1 && uint32_t(t.gemm_kparts) <= nb) p.kparts = uint32_t(t.gemm_kparts);
     // one split-K part (padded to whole tiles) must stay under 4 GiB: 32-bit offsets in the kernel
     if (uint64_t(pair ? 2 : 1) * p.ntok * TT * p.ncol * rows_per_tile * 4 >= (uint64_t(1) << 32)) p.kparts = 1;

@@ -32,23 +32,43 @@ def ctx():
     c.close()
 
 
-@pytest.mark.parametrize("qtype,cols,rows,batch", [(N.Q4_K, 2304, 2496, 1000), (N.Q4_K, 6400, 2496, 1020),
-                                                   (N.Q6_K, 4096, 3264, 1200), (N.Q6_K, 8192, 2752, 700)],
+@pytest.mark.parametrize("qtype,cols,rows,batch,kparts", [(N.Q4_K, 2304, 2496, 1000, 3), (N.Q4_K, 6400, 2496, 1020, 5),
+                                                          (N.Q6_K, 4096, 3264, 1200, 3), (N.Q6_K, 8192, 2752, 700, 7)],
                          ids=["q4k-3parts", "q4k-5parts", "q6k-3parts", "q6k-7parts"])
-def test_planned_odd_parts(ctx, tune, qtype, cols, rows, batch):
-    """FP32-mode splits of K that are no power of two, as the plan chooses them, on ragged tiles: the terms are
-    those of one part, so the two results differ by the order of 24-bit sums; and the repository's 1e-3 against
-    the dequantised weights."""
+def test_odd_parts(ctx, tune, qtype, cols, rows, batch, kparts):
+    """FP32-mode splits of K that are no power of two, on ragged tiles: the terms are those of one part, so the
+    two results differ by the order of 24-bit sums; and the repository's 1e-3 against the dequantised weights."""
     host = N.synth_weights(qtype, 0x61, rows, cols)
     w = torch.from_numpy(np.ascontiguousarray(N.retile(host, qtype, cols, rows, N.ROW_MAJOR, N.CDNA4))).cuda()
     bits = N.synth_normal_f16(0x62, batch * cols).reshape(batch, cols)
     x = torch.from_numpy(bits.view(np.int16)).cuda()
     y = [torch.full((batch, rows), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2)]
-    for kparts in (0, 1):
-        tune("gemm_kparts", kparts)
-        ctx.ffn_down(w, qtype, N.CDNA4, cols, rows, batch, x, y[kparts], half_input=True, fast_swa=False)
+    for out, parts in zip(y, (kparts, 1)):
+        tune("gemm_kparts", parts)
+        ctx.ffn_down(w, qtype, N.CDNA4, cols, rows, batch, x, out, half_input=True, fast_swa=False)
     torch.cuda.synchronize()
-    planned, one = (t.cpu().numpy() for t in y)
-    assert rel_err(planned, one) <= 64 * 2.0 ** -24
+    split, one = (t.cpu().numpy() for t in y)
+    assert rel_err(split, one) <= 64 * 2.0 ** -24
     want = bits.view(np.float16).astype(np.float32) @ O.dequant_rows(qtype, O.ROW_MAJOR, host, cols, rows, 0, rows).T
-    assert rel_err(planned, want) <= 1e-3
+    assert rel_err(split, want) <= 1e-3
+
+
+@pytest.mark.parametrize("batch,kparts", [(600, 8), (1300, 4)])
+@pytest.mark.parametrize("qtype,layout", [(N.Q6_K, N.CDNA4), (N.Q4_K, N.CDNA4), (N.Q4_K, N.ROW_MAJOR), (N.Q6_K, N.NSMFFN)],
+                         ids=["q6k-cdna4", "q4k-cdna4", "q4k-rowmajor", "q6k-nsmffn"])
+def test_down_parts_keep_their_chains(ctx, tune, qtype, layout, batch, kparts):
+    """FP32 mode, 3840 x 15360: no fewer K parts than the power of two that fills the device, so no longer chains
+    of fp32 sums (against 64 bits a Q6_K down in 4 parts is 1.42 times as far off as in 8): the planned result is
+    that of 8 parts (3 x 15 tiles of 256 tokens, 5 x 15 of 128) and of 4 parts (6 x 15, 11 x 15) bit for bit."""
+    cols, rows = 15360, 3840
+    host = N.synth_weights(qtype, 0x63, rows, cols)
+    img = host if layout == N.ROW_MAJOR else N.retile(host, qtype, cols, rows, N.ROW_MAJOR, layout)
+    w = torch.from_numpy(np.ascontiguousarray(img)).cuda()
+    x = torch.from_numpy(N.synth_normal_f16(0x64, batch * cols).reshape(batch, cols).view(np.int16)).cuda()
+    y = [torch.full((batch, rows), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2)]
+    for out, parts in zip(y, (0, kparts)):
+        tune("gemm_kparts", parts)
+        ctx.ffn_down(w, qtype, layout, cols, rows, batch, x, out, half_input=True, fast_swa=False)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y[0]).all()
+    assert torch.equal(y[0].view(torch.int32), y[1].view(torch.int32))
