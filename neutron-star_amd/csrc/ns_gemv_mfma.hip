@@ -674,11 +674,16 @@ Plan plan_mfma(uint32_t rows, uint32_t nb, bool pair, const Tuning &t) {
 }
 
 // Workgroups of the streaming form, or 0 for one slab per wave: where the plan's grid takes more than one
-// round of two workgroups per CU, whose later workgroups would stage x again with little in flight.  MI355X,
-// the 262,144-row Q6_K lm-head (1,024 workgroups, 512 streaming) at 3 fp32 tokens: 148.1 us before, 146.4 now.
+// round of two workgroups per CU, whose later workgroups would stage x again with little in flight, and its last
+// round is more than half full: streaming spreads the slabs evenly, so a last round of few workgroups leaves
+// fewer waves in flight over the whole call.  MI355X, 3 fp32 tokens of 3,840 columns, one slab per wave /
+// streaming (us): the 262,144-row Q6_K lm-head (2 rounds of 512 workgroups) 148.1 / 146.4, 212,992 rows (1.63)
+// 135 / 129, 196,608 rows (1.5) 109 / 126, 163,840 rows (1.25) 102 / 123, 278,528 rows (2.13) 168 / 181; Q4_K
+// 262,144 rows 113 / 106, 163,840 rows 80 / 92.
 uint32_t stream_grid(const Plan &p, uint32_t nwg, uint32_t nb) {
     const uint32_t room = 2 * uint32_t(device_cus());
     if (p.M != 1 || p.P != 1 || p.KP != 1 || nb < 2 || nwg <= room) return 0;
+    if (nwg % room != 0 && nwg % room <= room / 2) return 0;
     const uint32_t steps = (nwg + room - 1) / room;
     return (nwg + steps - 1) / steps;
 }
