@@ -1929,7 +1929,7 @@ hipError_t launch_gemv(int type, int layout, const uint8_t *w, const uint8_t *up
                        const NormPrologue *np) {
     if (up) return launch_typed<Q4_K, true>(layout, w, up, x, out, cols, rows, ws, stream, np);
     if (np) return hipErrorInvalidValue;  // the prologue exists for the gate/up pair only
-    if (gemv_row_eligible(layout, cols, ws.tune)) return launch_gemv_row(type, w, x, out, cols, rows, stream);
+    if (gemv_row_eligible(type, layout, cols, rows, ws.tune)) return launch_gemv_row(type, w, x, out, cols, rows, stream);
     if (type == Q4_K) return launch_typed<Q4_K, false>(layout, w, nullptr, x, out, cols, rows, ws, stream, nullptr);
     return launch_typed<Q6_K, false>(layout, w, nullptr, x, out, cols, rows, ws, stream, nullptr);
 }

@@ -258,10 +258,27 @@ __global__ __launch_bounds__(64 * MW) void gemv_row_kernel(
 
 }  // namespace
 
-// Rows of up to 256 super-blocks (16 waves of 16); the slab kernel where a test asks for one of its grids.
-bool gemv_row_eligible(int layout, uint32_t cols, const Tuning &t) {
-    return layout == ROW_MAJOR && t.gemv_row != 0 && cols / kQK <= 16 * kSpan && t.gemv_pf < 0 && t.gemv_waves == 0 &&
-           t.gemv_whole != 0 && t.gemv_qslab != 0;
+// Where this kernel is the faster one: rows of up to 256 super-blocks (16 waves of 16); the slab kernel where a
+// test asks for one of its grids.  While the rows do not fill the device the ramp and the round trip decide, and
+// this kernel takes 0.3-1.0 of the slab kernel's time at every length.  Beyond, a row costs a wave the same
+// whatever its length, so the lanes have to be in use; the slab kernel's time follows the super-blocks.  MI355X,
+// this kernel's time over the slab kernel's:
+//   Q4_K  32,768 rows: 2.07 at 1 super-block, 1.20 at 4, 0.81 at 5, 0.40 at 16, 0.68 at 17, 1.17 at 65, 0.93 at
+//         80, 0.58 at 128;  8,192 rows: 0.87 at 1 and at 4, 1.09 at 65, 0.93 at 72
+//   Q6_K  98,304 rows: 4.87 at 1, 1.23 at 8, 1.00 at 9, 0.71 at 16, 1.12 at 17, 0.84 at 28;  49,152 rows: 1.07 at
+//         36, 0.89 at 48, 1.60 at 72;  16,384 rows: 1.30 at 6, 0.86 at 9, 0.93 at 17, 1.04 at 112, 0.82 at 128;
+//         8,192 rows: 1.13 at 4, 0.99 at 5, 1.41 at 72
+// (rows of 5 to 7 waves run few waves per CU, the one workgroup's)
+bool gemv_row_eligible(int type, int layout, uint32_t cols, uint32_t rows, const Tuning &t) {
+    const uint32_t nb = cols / kQK, kw = (nb + kSpan - 1) / kSpan;
+    if (layout != ROW_MAJOR || t.gemv_row == 0 || nb > 16 * kSpan || t.gemv_pf >= 0 || t.gemv_waves != 0 ||
+        t.gemv_whole == 0 || t.gemv_qslab == 0)
+        return false;
+    if (rows <= 4096) return true;
+    if (type == Q4_K) return kw > 4 ? nb > 80 : nb >= 5 || rows <= 8192;
+    if (kw > 4) return nb >= 128;
+    if (rows <= 21504) return nb >= (rows <= 8192 ? 5 : 9);
+    return kw == 1 ? nb >= 9 : nb * 5 >= kw * kSpan * 4;  // a second wave's lanes mostly in use
 }
 
 hipError_t launch_gemv_row(int type, const uint8_t *w, const float *x, float *out, uint32_t cols, uint32_t rows,

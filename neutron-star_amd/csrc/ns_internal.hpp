@@ -100,7 +100,7 @@ hipError_t launch_gemv(int type, int layout, const uint8_t *w, const uint8_t *up
 
 // Decode GEMV on ROW_MAJOR tensors with a row's blocks across the lanes (ns_gemv_row.hip);
 // launch_gemv routes there (plain, no NormPrologue) when eligible.
-bool gemv_row_eligible(int layout, uint32_t cols, const Tuning &t);
+bool gemv_row_eligible(int type, int layout, uint32_t cols, uint32_t rows, const Tuning &t);
 hipError_t launch_gemv_row(int type, const uint8_t *w, const float *x, float *out, uint32_t cols, uint32_t rows,
                            hipStream_t stream);
 

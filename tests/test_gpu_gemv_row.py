@@ -22,7 +22,7 @@ def ctx():
 
 
 @pytest.mark.parametrize("rows,nb", [(1, 1), (7, 15), (9, 16), (64, 17), (33, 33), (130, 47), (5, 60), (66, 65),
-                                     (3, 256), (8199, 3)])
+                                     (3, 256), (8199, 3), (8199, 9), (4097, 130)])
 @pytest.mark.parametrize("qtype", [N.Q4_K, N.Q6_K], ids=["q4k", "q6k"])
 def test_gemv_row(ctx, tune, qtype, rows, nb):
     cols = nb * 256
@@ -42,3 +42,22 @@ def test_gemv_row(ctx, tune, qtype, rows, nb):
     ctx.matmul(w, qtype, N.ROW_MAJOR, cols, rows, 1, xd, z)
     torch.cuda.synchronize()
     assert rel_err(got[:rows], z.cpu().numpy()) <= 2.0 ** -24 * 8 * np.sqrt(cols)
+
+
+@pytest.mark.parametrize("qtype,rows,nb,same", [
+    (N.Q4_K, 32768, 1, True), (N.Q4_K, 32768, 4, True), (N.Q4_K, 32768, 5, False), (N.Q4_K, 8193, 65, True),
+    (N.Q4_K, 8192, 1, False), (N.Q4_K, 4096, 65, False), (N.Q6_K, 32768, 8, True), (N.Q6_K, 32768, 9, False),
+    (N.Q6_K, 32768, 17, True), (N.Q6_K, 32768, 28, False), (N.Q6_K, 8193, 8, True), (N.Q6_K, 4097, 4, True),
+    (N.Q6_K, 4096, 1, False), (N.Q6_K, 4097, 127, True), (N.Q6_K, 4097, 128, False)])
+def test_short_rows_on_the_slab_kernel(ctx, tune, qtype, rows, nb, same):
+    """Which kernel many rows of few super-blocks run on (the row kernel took up to 6 times as long there): the
+    two sum in different orders, so the slab kernel's bits tell it."""
+    cols = nb * 256
+    w = torch.from_numpy(N.synth_weights(qtype, 0x62, rows, cols)).cuda()
+    x = torch.from_numpy(N.synth_normal_f32(0x63, cols)).cuda()
+    y = [torch.empty(rows, dtype=torch.float32, device="cuda") for _ in range(2)]
+    ctx.matmul(w, qtype, N.ROW_MAJOR, cols, rows, 1, x, y[0])
+    tune("gemv_row", 0)
+    ctx.matmul(w, qtype, N.ROW_MAJOR, cols, rows, 1, x, y[1])
+    torch.cuda.synchronize()
+    assert torch.equal(y[0], y[1]) == same
