@@ -218,7 +218,7 @@ int gemm_skinny(ns_ctx *ctx, const char *fn, int type, int last_type, int layout
 // Batch 2-4: the weights stream once for every token (mm:273, mm:282).
 int gemv_mt(ns_ctx *ctx, const char *fn, int type, int layout, const void *w, const void *up, const void *x,
             bool xh, uint32_t batch, void *out, uint32_t cols, uint32_t rows, hipStream_t s) {
-    if (xh && !up && skinny_small_batch(type, layout, cols, rows, x, batch, false, ctx->ws.tune))
+    if (xh && !up && skinny_small_batch(type, layout, cols, rows, x, batch, ctx->ws.tune))
         return gemm_skinny(ctx, fn, type, 0, layout, &w, nullptr, static_cast<const uint16_t *>(x), &out, nullptr, &rows, 1,
                            cols, batch, s);
     size_t pf = 0, nc = 0;
@@ -634,11 +634,7 @@ extern "C" int ns_qkv(ns_ctx *ctx, const void *wq, const void *wk, const void *w
         void *const outs[3] = {q, k, v};
         const uint32_t rows[3] = {q_rows, kv_rows, kv_rows};
         const int nseg = wv ? 3 : 2;
-        const bool small_ok =
-            batch > 4 ||
-            (skinny_small_batch(Q4_K, layout, cols, q_rows, x, batch, true, ctx->ws.tune) &&
-             skinny_small_batch(wv ? v_type : Q4_K, layout, cols, kv_rows, x, batch, true, ctx->ws.tune));
-        if (small_ok && gemm_skinny_eligible(Q4_K, layout, ACC_FP32, cols, rows, nseg, batch, false, ctx->ws.tune))
+        if (skinny_qkv_eligible(layout, cols, rows, nseg, wv ? v_type : 0, x, batch, ctx->ws.tune))
             return gemm_skinny(ctx, fn, Q4_K, wv ? v_type : 0, layout, ws_, nullptr, x, outs, wv ? nullptr : v, rows, nseg,
                                cols, batch, s);
     }

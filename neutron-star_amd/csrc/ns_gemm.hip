@@ -952,6 +952,11 @@ hipError_t launch_layout(int layout, int acc, const uint8_t *w, const uint8_t *u
 
 }  // namespace
 
+TileGrid gemm_grid(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t) {
+    const GemmPlan p = plan_gemm(cols, rows, batch, pair, t);
+    return {p.ntok * p.ncol, p.kparts, TT};
+}
+
 // Workspace layout: [Q4_K: the XsLayout block (group sums of x, token factors, the
 // rescaled copy of x)] [split-K parts: kparts x planes x tokens x rows, both padded to
 // whole tiles].
@@ -978,7 +983,7 @@ void gemm_workspace_need(int type, int layout, uint32_t cols, uint32_t rows, uin
     *floats = std::max(f16_floats, f32_floats);
     *counters = std::max(f16_counters, f32_counters);
     for (int acc : {ACC_FP32, ACC_FP16})
-        if (gemm_skinny_eligible(type, layout, acc, cols, &rows, 1, batch, pair, t)) {
+        if (gemm_skinny_eligible(type, layout, acc, cols, rows, batch, pair, t)) {
             size_t f = 0, c = 0;
             gemm_skinny_workspace_need(type, cols, &rows, 1, batch, pair, acc, t, &f, &c);
             *floats = std::max(*floats, f);
@@ -1003,7 +1008,7 @@ static void gemm_fp32_workspace_need(int type, int layout, uint32_t cols, uint32
 hipError_t launch_gemm(int type, int layout, int acc, const uint8_t *w, const uint8_t *up, const uint16_t *x,
                        void *out, uint32_t cols, uint32_t rows, uint32_t batch, const Workspace &ws,
                        hipStream_t stream) {
-    if (gemm_skinny_eligible(type, layout, acc, cols, &rows, 1, batch, up != nullptr, ws.tune))
+    if (gemm_skinny_eligible(type, layout, acc, cols, rows, batch, up != nullptr, ws.tune))
         return launch_gemm_skinny(type, layout, acc, &w, up, &out, &rows, 1, x, cols, batch, ws.partial, ws.counters,
                                   ws.tune, stream);
     if (layout == CDNA4 && acc == ACC_FP16)

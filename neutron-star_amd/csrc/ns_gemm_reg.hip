@@ -591,6 +591,11 @@ RegPlan plan_reg(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const 
 
 }  // namespace
 
+TileGrid gemm_reg_grid(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t) {
+    const RegPlan p = plan_reg(cols, rows, batch, pair, t);
+    return {p.ntok * p.ncol, p.kparts, TT};
+}
+
 void gemm_reg_workspace_need(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t,
                              size_t *part_floats, size_t *counters) {
     const RegPlan p = plan_reg(cols, rows, batch, pair, t);

@@ -790,6 +790,54 @@ Plan plan_skinny(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32
     return best;
 }
 
+// What a call takes, in microseconds, here and on the FP32-mode tile kernel that would run instead
+// (ns_gemm_reg.hip for Q4_K on CDNA4, else ns_gemm.hip): least squares of the logarithms over 7,000 timings of
+// random shapes each, weighted to where the two are close (there within 17% in 90 of 100).
+//   here   call + rounds * (wg + super-blocks a wave walks * sb[32- or 64-token tile]) + part per K part and
+//          32 tokens + mb per MB of output; rounds of one workgroup per CU, past the first by size plus `over`
+//   tile   call + rounds * (wg + super-blocks * sb) + part_mb per MB of K parts (padded to tiles) + x_mb per MB
+//          of x + col per super-block of columns (the group sums ahead) + last per K part that a last arrival
+//          reads + mb; ns_gemm_reg.hip runs two workgroups per CU, from sb[0] alone to sb[1] together
+struct Route {
+    double call, wg, sb[2], part, over, mb;
+    struct {
+        double call, wg, sb[2], over, part_mb, x_mb, col, last, mb;
+    } tile;
+};
+const Route &route_of(int type, int layout, bool pair) {
+    static constexpr Route kPair{3.73, 1.71, {3.9, 6.01}, 0.29, 0.07, 0.4, {8.73, 0, {5.71, 7.75}, 0.22, 0.32, 0.18, 0.21, 1.19, 0.65}};
+    static constexpr Route kQ4{2.7, 1.05, {3.83, 5.82}, 0.52, 0.24, 0.38, {9.91, 0, {5.16, 7.88}, 0.26, 0.33, 0.16, 0.24, 0.77, 0.15}};
+    static constexpr Route kQ6{1.9, 1.81, {4.06, 5.25}, 0.62, 0.36, 0.3, {3.3, 0.71, {6.79, 6.79}, 0.68, 0.28, 0.05, 0.36, 1.02, 0.19}};
+    static constexpr Route kQ4Row{3.16, 0.55, {4.68, 6.26}, 0.54, 0.24, 0.36, {8.3, 0, {8.78, 8.78}, 0.61, 0.31, 0.02, 0.33, 1.45, 0.19}};
+    static constexpr Route kQ6Row{2.69, 0, {9.21, 9.01}, 0.62, 0.28, 0.08, {7.56, 3.17, {29.52, 29.52}, 0.54, 1.23, 0, 0.28, 1.23, 0.19}};
+    if (layout == ROW_MAJOR) return type == Q4_K ? kQ4Row : kQ6Row;
+    return pair ? kPair : type == Q4_K ? kQ4 : kQ6;
+}
+double out_mb(const uint32_t *rows, int nseg, uint32_t batch, bool pair) {
+    double n = 0;
+    for (int s = 0; s < nseg; ++s) n += rows[s];
+    return n * batch * (pair ? 2 : 4) * 1e-6;
+}
+double skinny_us(const Route &r, const Plan &p, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair) {
+    const uint32_t nb = cols / kQK, iters = ((nb + p.kparts - 1) / p.kparts + p.wk - 1) / p.wk;
+    const double q = double(p.ntok * p.ncol) * p.kparts / device_cus();
+    return r.call + (q <= 1 ? 1 : q + r.over) * (r.wg + iters * r.sb[p.mi == 1 ? 0 : 1]) +
+           (p.kparts > 1 ? r.part * p.kparts * p.mi : 0) + r.mb * out_mb(rows, nseg, batch, pair);
+}
+double tile_us(const Route &r, int type, int layout, uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t) {
+    const auto &c = r.tile;
+    const bool reg = layout == CDNA4 && type == Q4_K;
+    const TileGrid g = reg ? gemm_reg_grid(cols, rows, batch, pair, t) : gemm_grid(cols, rows, batch, pair, t);
+    const double n = double(g.tiles) * g.kparts, q = n / device_cus();
+    const uint32_t nb = cols / kQK, sb = (nb + g.kparts - 1) / g.kparts;
+    const double rounds = reg ? (q <= 2 ? 1 : q / 2 + c.over) : (q <= 1 ? 1 : q + c.over);
+    const double step = c.sb[0] + (c.sb[1] - c.sb[0]) * std::min(std::max(q - 1, 0.0), 1.0);
+    const bool scatter = (g.tokens / 32) % g.kparts == 0 && q <= (reg ? 2 : 1);
+    return c.call + rounds * (c.wg + sb * step) + (g.kparts > 1 ? c.part_mb * n * g.tokens * 256 * 4e-6 : 0) +
+           c.x_mb * batch * cols * 2e-6 + c.col * nb + (g.kparts > 1 && !scatter ? c.last * g.kparts : 0) +
+           c.mb * out_mb(&rows, 1, batch, pair);
+}
+
 template <int TYPE, int LAYOUT, int ACC, bool PAIR>
 hipError_t launch_mi(const Plan &p, const Args &a, hipStream_t stream) {
     const dim3 grid(p.ntok * p.ncol * p.kparts), block(kThreads);
@@ -825,34 +873,90 @@ hipError_t launch_mixed(const Plan &p, const Args &a, hipStream_t stream) {
 
 // Whether this kernel is the faster one.  FP16 mode: by its plan's estimate against the tile kernel's
 // (gate/up 128 tokens: 44 us here, 50 there; 225: 75 / 65; downs 225: 43-46 / 48-55; 320: 63-67 / 63).
-// FP32 mode: a bound on the estimate, because the 128- and 256-token tile kernels need many output
-// tiles to fill the device and then cost ~90-115 us; below that they take as long.  MI355X, this
-// kernel against them (us), each bound from both sides:
-//   gate/up        192 tokens: 81 / 94,               225: 106 / 95
-//   downs          512: 78-96 / 114-127,              775: 157-180 / 134-145
-//   4096 x 3840    1536: 89 / 114, row-major 93 / 95;   2048: 121 / 103, row-major 125 / 106
-// A row-major Q6_K tensor runs at 260-273 us at any batch there (2-byte loads) and at 42-80 us here
-// for 2,048 rows at 1,024-2,048 tokens.
-bool gemm_skinny_eligible(int type, int layout, int acc, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch,
-                          bool pair, const Tuning &t) {
+// FP32 mode: by the two estimates of Route, 5% for their error.  Over 37,000 random shapes (256 to 32,768
+// columns, 64 to 262,144 rows, 5 to 2,048 tokens) the choice is more than 5% slower than the tile kernels in
+// 0.2% of them and more than 5% slower than this kernel in 1%; it takes 0.362 of the tile kernels' time
+// (geometric mean), the better one of each two 0.361.  MI355X, this kernel against them (us):
+//   gate/up 192 tokens: 81 / 94, 225: 106 / 95;  downs 512: 78-96 / 114-127, 775: 157-180 / 134-145
+//   4096 x 3840, 1536 tokens: 89 / 114, row-major 93 / 95;  2048: 121 / 103, row-major 125 / 106
+//   256 columns: 65,536 rows at 71 tokens 55 / 23 (the pair), Q6_K at 217 62 / 20
+bool gemm_skinny_eligible(int type, int layout, int acc, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
+                          const Tuning &t) {
     if (t.gemm_skinny == 0) return false;
     if (layout == NSMFFN || (layout == ROW_MAJOR && (acc == ACC_FP16 || pair))) return false;
     if (t.gemm_skinny > 0) return batch <= uint32_t(t.gemm_skinny);
     if (t.gemm_q4_reg == 0 && type == Q4_K && acc == ACC_FP32) return false;  // the LDS-tile kernel is asked for
     if (batch > 2048) return false;  // beyond what was measured
-    const uint32_t cost = plan_skinny(type, cols, rows, nseg, batch, pair, acc == ACC_FP16, t).cost;
+    Tuning plain = t;  // a forced number of K parts does not change the kernel
+    plain.gemm_kparts = 0;
+    const Plan p = plan_skinny(type, cols, &rows, 1, batch, pair, acc == ACC_FP16, plain);
     // (and a bound: past two rounds the weights are read once per token tile from beyond L2, which the
     // estimate leaves out: downs at 600 tokens 124-130 us here, 109 there)
-    if (acc == ACC_FP16) return cost <= std::min(800u, gemm_f16_cost(cols, rows[0], batch, pair, t));
-    return cost <= (layout == ROW_MAJOR && type == Q6_K ? 2600u : 960u);
+    if (acc == ACC_FP16) return p.cost <= std::min(800u, gemm_f16_cost(cols, rows, batch, pair, plain));
+    const Route &r = route_of(type, layout, pair);
+    return skinny_us(r, p, cols, &rows, 1, batch, pair) <= 0.95 * tile_us(r, type, layout, cols, rows, batch, pair, plain);
 }
 
-bool skinny_small_batch(int type, int layout, uint32_t cols, uint32_t rows, const void *x, uint32_t batch, bool mixed,
-                        const Tuning &t) {
-    if (type == Q6_K && layout == CDNA4 && !mixed) return false;  // not exact there (kExact)
-    if (batch < 2 || batch > 4 || reinterpret_cast<uintptr_t>(x) % 16) return false;
-    if (t.mt_mfma == 0 || t.mt_parts > 0 || t.mt_slabs > 0 || t.mt_spw > 0) return false;  // a small-batch kernel is asked for
-    return gemm_skinny_eligible(type, layout, ACC_FP32, cols, &rows, 1, batch, false, t);
+namespace {
+
+// Batch 2-4: x comes by 16-byte DMA, and no small-batch kernel is asked for.
+bool small_batch_possible(int type, const void *x, uint32_t batch, const Tuning &t) {
+    return batch >= 2 && batch <= 4 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && t.gemm_skinny != 0 &&
+           (t.gemm_q4_reg != 0 || type != Q4_K) && t.mt_mfma != 0 && t.mt_parts <= 0 && t.mt_slabs <= 0 && t.mt_spw <= 0;
+}
+
+// What the small-batch kernels take at 2 and at 3-4 fp16 tokens, in microseconds: call, per super-block of columns
+// (its serial part) and per 1,024 super-blocks (fitted as Route; within 20%).
+double small_us(int type, int layout, uint32_t cols, uint32_t rows, uint32_t batch) {
+    static constexpr double k[2][2][2][3] = {{{{7.0, 0.082, 0.0908}, {8.0, 0.11, 0.098}}, {{8.7, 0.103, 0.0928}, {8.1, 0.098, 0.1086}}},
+                                             {{{10.0, 0.087, 0.0285}, {10.0, 0.087, 0.0285}}, {{8.2, 0.097, 0.0358}, {8.2, 0.097, 0.0358}}}};
+    const double *c = k[layout == CDNA4][type == Q6_K][batch > 2];
+    const uint32_t nb = cols / kQK;
+    return c[0] + c[1] * nb + c[2] * (double(rows) * nb / 1024);
+}
+
+}  // namespace
+
+// Row-major tensors by the two estimates, 5% for their error; short rows, whose estimates are loose, stay there.
+// Over 8,900 random shapes the choice is more than 5% slower than the small-batch kernels in 0.3% of them (2,048 x
+// 3,840 at 3 tokens 9.4 us here, 12.4 there; Q6_K 64 x 3,840 13 / 10, 65,536 x 2,304 55 / 76).  Q4_K on CDNA4:
+// here but for tall matrices of up to 15 super-blocks, which the small-batch kernel walks with a wave per slab and
+// no hand-off (at up to two slabs per CU 0.58-1.00 of its time, at 65,536-262,144 rows 1.1-2.0 of it).  Q6_K on
+// CDNA4: not exact here (kExact).
+bool skinny_small_batch(int type, int layout, uint32_t cols, uint32_t rows, const void *x, uint32_t batch, const Tuning &t) {
+    if (layout == NSMFFN || (type == Q6_K && layout == CDNA4) || !small_batch_possible(type, x, batch, t)) return false;
+    if (t.gemm_skinny > 0) return batch <= uint32_t(t.gemm_skinny);
+    const uint32_t nb = cols / kQK;
+    if (layout == CDNA4) return nb > 15 || rows <= 2 * uint32_t(device_cus()) * kRowTile;
+    if (nb < (type == Q4_K ? 2u : 6u)) return false;
+    Tuning plain = t;
+    plain.gemm_kparts = 0;
+    return skinny_us(route_of(type, layout, false), plan_skinny(type, cols, &rows, 1, batch, false, false, plain), cols, &rows, 1,
+                     batch, false) <= 0.95 * small_us(type, layout, cols, rows, batch);
+}
+
+// Q, K and V (or Q and a K that is V too) in one launch: against the launches of their own that they would take.
+bool skinny_qkv_eligible(int layout, uint32_t cols, const uint32_t *rows, int nseg, int last_type, const void *x,
+                         uint32_t batch, const Tuning &t) {
+    if (t.gemm_skinny == 0 || layout == NSMFFN || t.gemm_q4_reg == 0 || batch > 2048) return false;
+    const bool small = batch <= 4;
+    if (small && !small_batch_possible(Q4_K, x, batch, t)) return false;
+    if (t.gemm_skinny > 0) return batch <= uint32_t(t.gemm_skinny);
+    Tuning plain = t;
+    plain.gemm_kparts = 0;
+    double q6 = 0, total = 0, apart = last_type ? 0 : 4;  // a tied V is a copy of K
+    for (int s = 0; s < nseg; ++s) {
+        const int type = s == nseg - 1 && last_type ? last_type : Q4_K;
+        const Route &r = route_of(type, layout, false);
+        const double own = skinny_us(r, plan_skinny(type, cols, rows + s, 1, batch, false, false, plain), cols, rows + s, 1, batch, false);
+        if (!small) apart += std::min(own, tile_us(r, type, layout, cols, rows[s], batch, false, plain));
+        else apart += skinny_small_batch(type, layout, cols, rows[s], x, batch, t) ? own : small_us(type, layout, cols, rows[s], batch);
+        total += rows[s];
+        if (type == Q6_K) q6 += rows[s];
+    }
+    Route mix = route_of(Q4_K, layout, false);  // by the share of the column tiles that are Q6_K
+    for (int m = 0; m < 2; ++m) mix.sb[m] += (route_of(Q6_K, layout, false).sb[m] - mix.sb[m]) * (q6 / total);
+    return skinny_us(mix, plan_skinny(Q4_K, cols, rows, nseg, batch, false, false, plain), cols, rows, nseg, batch, false) <= apart;
 }
 
 void gemm_skinny_workspace_need(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair,

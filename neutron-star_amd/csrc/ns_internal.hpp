@@ -203,19 +203,27 @@ hipError_t launch_gemm_f16(int type, const uint8_t *w, const uint8_t *up, const 
                            uint32_t rows, uint32_t batch, float *partial, uint32_t *counters, uint32_t *err,
                            const Tuning &t, hipStream_t stream);
 
+// The output tiles, K parts and tokens per tile that the FP32-mode tile kernels would run with.
+struct TileGrid {
+    uint32_t tiles, kparts, tokens;
+};
+TileGrid gemm_reg_grid(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t);
+TileGrid gemm_grid(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t);
+
 // The prefill GEMM for few tokens (ns_gemm_skinny.hip): CDNA4 in both modes, ROW_MAJOR in the FP32
 // mode without the pair.  Up to three matrices that share x (rows, w and out arrays of nseg
 // entries) in one launch, the last of last_type if that is not 0 (Q6_K behind Q4_K, FP32 mode);
 // copy: a second output of the last one.  With `up` the gate/up pair (nseg 1).
-bool gemm_skinny_eligible(int type, int layout, int acc, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch,
-                          bool pair, const Tuning &t);
-// Batch 2-4 with fp16 x: whether it takes this kernel, the faster one that keeps the small-batch
-// kernels' precision (every product exact).  It reads x by 16-byte DMA, so x has to be aligned.  mixed: the
-// matrix is one of several in a launch (ns_qkv), where Q6_K is exact on every layout.  Not for the gate/up
+bool gemm_skinny_eligible(int type, int layout, int acc, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
+                          const Tuning &t);
+// The same for Q, K and V together (batch 2 and above).
+bool skinny_qkv_eligible(int layout, uint32_t cols, const uint32_t *rows, int nseg, int last_type, const void *x,
+                         uint32_t batch, const Tuning &t);
+// Batch 2-4 with fp16 x: whether it takes this kernel, where it is the faster one; it keeps the small-batch
+// kernels' precision (every product exact).  It reads x by 16-byte DMA, so x has to be aligned.  Not for the gate/up
 // pair: 19.9 us here against 21.2, but of the two it had the larger error against 64 bits (its gate and up
 // round to fp16 h on other sides).
-bool skinny_small_batch(int type, int layout, uint32_t cols, uint32_t rows, const void *x, uint32_t batch, bool mixed,
-                        const Tuning &t);
+bool skinny_small_batch(int type, int layout, uint32_t cols, uint32_t rows, const void *x, uint32_t batch, const Tuning &t);
 void gemm_skinny_workspace_need(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair,
                                 int acc, const Tuning &t, size_t *part_floats, size_t *counters);
 hipError_t launch_gemm_skinny(int type, int layout, int acc, const uint8_t *const *w, const uint8_t *up, void *const *out,

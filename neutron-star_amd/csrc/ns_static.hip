@@ -130,7 +130,7 @@ extern "C" int ns_matmul_noalloc(const void *w, int type, int layout, uint32_t c
     const hipStream_t s = static_cast<hipStream_t>(stream);
     // batch 2-4: the same choice of kernel as ns_matmul (its parts: at most one round of workgroups' tiles,
     // 1 Mi floats, inside the scratch whatever the shape)
-    const bool skinny = batch <= 4 && half_input && skinny_small_batch(type, layout, cols, rows, in, batch, false, t);
+    const bool skinny = batch <= 4 && half_input && skinny_small_batch(type, layout, cols, rows, in, batch, t);
     if (skinny) {
         size_t f = 0, c = 0;
         gemm_skinny_workspace_need(type, cols, &rows, 1, batch, false, ACC_FP32, t, &f, &c);

@@ -210,3 +210,25 @@ def test_small_batch_sums_no_worse(ctx, tune, qtype, layout, rows, cols, batch):
             ctx.qkv(q4, q4, w, qtype, layout, cols, rows, rows, batch, x, q, k, v)
             err[skinny] += [sum_error(y, want), sum_error(v, want)]
     assert (err[-1] <= 1.05 * err[0]).all(), err
+
+
+@pytest.mark.parametrize("qtype,layout,rows,nb,batch,tile", [
+    (N.Q6_K, N.CDNA4, 65536, 1, 217, True), (N.Q4_K, N.CDNA4, 131072, 1, 65, True), (N.Q4_K, N.ROW_MAJOR, 15360, 1, 933, True),
+    (N.Q6_K, N.ROW_MAJOR, 32768, 1, 1023, True), (N.Q6_K, N.CDNA4, 4096, 16, 1687, True), (N.Q4_K, N.CDNA4, 15360, 15, 1024, True),
+    (N.Q4_K, N.CDNA4, 4096, 15, 157, False), (N.Q4_K, N.ROW_MAJOR, 2048, 15, 1024, False), (N.Q6_K, N.ROW_MAJOR, 2048, 15, 500, False),
+    (N.Q6_K, N.CDNA4, 3840, 60, 64, False),
+    (N.Q4_K, N.CDNA4, 262144, 2, 3, True), (N.Q4_K, N.CDNA4, 65536, 15, 2, True), (N.Q4_K, N.ROW_MAJOR, 64, 16, 2, True),
+    (N.Q6_K, N.ROW_MAJOR, 2048, 4, 4, True), (N.Q6_K, N.ROW_MAJOR, 64, 15, 3, True), (N.Q4_K, N.CDNA4, 32768, 15, 3, False),
+    (N.Q4_K, N.ROW_MAJOR, 4096, 15, 3, False), (N.Q6_K, N.ROW_MAJOR, 3840, 60, 3, False)])
+def test_route_by_the_faster_kernel(ctx, tune, qtype, layout, rows, nb, batch, tile):
+    """FP32 mode: which of the two kernels runs, on shapes where one of them takes 1.1 to 3 times as long.  They sum
+    in different orders, so the tile or small-batch kernel's bits tell it."""
+    cols = nb * 256
+    _, w = weights(qtype, 0x65, rows, cols, layout)
+    _, x = tokens(0x66, batch, cols)
+    y = [torch.empty((batch, rows), dtype=torch.float32, device="cuda") for _ in range(2)]
+    for out, skinny in zip(y, (-1, 0)):
+        tune("gemm_skinny", skinny)
+        ctx.matmul(w, qtype, layout, cols, rows, batch, x, out, half_input=True)
+    torch.cuda.synchronize()
+    assert torch.equal(y[0], y[1]) == tile
