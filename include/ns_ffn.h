@@ -150,13 +150,14 @@ int ns_matmul(ns_ctx *ctx, const void *w, int type, int layout, uint32_t cols, u
  * (code under HIP graph capture, serving loops and harnesses that forbid hipMalloc).  The same
  * regimes and kernels as ns_matmul with the default tuning, without a context: the split
  * reductions use a static device scratch array of 16 MiB of parts and 65,536 counters that
- * each GPU holds until the process ends (whether or not it ever calls this function).  A
- * prefill GEMM (batch > 4) whose default split-K plan needs more parts than the array holds
- * runs with one K part (the gemm_kparts 1 tuning of ns_matmul: same kernels, one part per
- * tile, each output within the FP32 tolerance of ns_matmul's); a shape that still needs more
- * fails with NS_ERR_UNSUPPORTED (a Q4_K GEMM needs ~0.53 floats of scratch per input value:
- * up to ~2,000 tokens of the 3840-wide gate/up input, ~500 of the 15360-wide down input; Q6_K
- * none).  fp32 input above batch 4 is refused (its fp16 copy would need a buffer).  Calls
+ * each GPU holds until the process ends (whether or not it ever calls this function).  Where
+ * ns_matmul takes the few-token GEMM its parts fit and the results are ns_matmul's bit for
+ * bit.  A prefill GEMM (batch > 4) on the tile kernels whose default split-K plan needs more
+ * parts than the array holds runs with one K part (the gemm_kparts 1 tuning of ns_matmul: same
+ * kernels, one part per tile, each output within the FP32 tolerance of ns_matmul's); a shape
+ * that still needs more fails with NS_ERR_UNSUPPORTED (a Q4_K tile GEMM needs ~0.53 floats of
+ * scratch per input value: up to ~2,000 tokens of a 3840-wide input, ~500 of a 15360-wide
+ * one; Q6_K none).  fp32 input above batch 4 is refused (its fp16 copy would need a buffer).  Calls
  * that overlap on one GPU share the array and race: order them (one stream).  Allocates
  * nothing, never synchronises, and may be captured into a graph. */
 int ns_matmul_noalloc(const void *w, int type, int layout, uint32_t cols, uint32_t rows, uint32_t batch,

@@ -178,10 +178,14 @@ void model_workspace_need(const Tuning &t, size_t *floats, size_t *counters) {
                 }
             if (sh.rows > 16384) continue;  // the lm-head is a decode GEMV
             // the plans change at multiples of 16 tokens at most, and the need grows between them
-            for (uint32_t b = 16; b <= 2048; b += 16) {
-                gemm_workspace_need(sh.type, layout, sh.cols, sh.rows, b, sh.pair, t, &f, &c);
-                take(f, c);
-            }
+            // (which kernel runs may change anywhere: both kernels' needs)
+            for (uint32_t b = 16; b <= 2048; b += 16)
+                for (int acc : {ACC_FP32, ACC_FP16}) {
+                    gemm_tile_workspace_need(sh.type, layout, acc, sh.cols, sh.rows, b, sh.pair, t, &f, &c);
+                    take(f, c);
+                    gemm_skinny_workspace_need(sh.type, sh.cols, &sh.rows, 1, b, sh.pair, acc, t, &f, &c);
+                    take(f, c);
+                }
         }
     size_t f = 0, c = 0;
     block_decode_workspace_need(3840, 15360, &f, &c);
@@ -203,15 +207,14 @@ int gemv(ns_ctx *ctx, const char *fn, int type, int layout, const void *w, const
 }
 
 // The few-token prefill GEMM (ns_gemm_skinny.hip) over 1-3 matrices that share x, FP32 mode.
-int gemm_skinny(ns_ctx *ctx, const char *fn, int type, int last_type, int layout, const void *const *w, const void *up,
-                const uint16_t *x, void *const *out, void *copy, const uint32_t *rows, int nseg, uint32_t cols,
-                uint32_t batch, hipStream_t s) {
+int gemm_skinny(ns_ctx *ctx, const char *fn, int type, int last_type, int layout, const void *const *w, const uint16_t *x,
+                void *const *out, void *copy, const uint32_t *rows, int nseg, uint32_t cols, uint32_t batch, hipStream_t s) {
     size_t pf = 0, nc = 0;
-    gemm_skinny_workspace_need(type, cols, rows, nseg, batch, up != nullptr, ACC_FP32, ctx->ws.tune, &pf, &nc);
+    gemm_skinny_workspace_need(type, cols, rows, nseg, batch, false, ACC_FP32, ctx->ws.tune, &pf, &nc);
     if (int rc = ensure_ws(ctx, pf, nc, s)) return rc;
     const hipError_t e = launch_gemm_skinny(type, layout, ACC_FP32, reinterpret_cast<const uint8_t *const *>(w),
-                                            static_cast<const uint8_t *>(up), out, rows, nseg, x, cols, batch,
-                                            ctx->ws.partial, ctx->ws.counters, ctx->ws.tune, s, last_type, copy);
+                                            nullptr, out, rows, nseg, x, cols, batch, ctx->ws.partial,
+                                            ctx->ws.counters, ctx->ws.tune, s, last_type, copy);
     return e == hipSuccess ? NS_OK : hip_fail(e, fn);
 }
 
@@ -219,8 +222,7 @@ int gemm_skinny(ns_ctx *ctx, const char *fn, int type, int last_type, int layout
 int gemv_mt(ns_ctx *ctx, const char *fn, int type, int layout, const void *w, const void *up, const void *x,
             bool xh, uint32_t batch, void *out, uint32_t cols, uint32_t rows, hipStream_t s) {
     if (xh && !up && skinny_small_batch(type, layout, cols, rows, x, batch, ctx->ws.tune))
-        return gemm_skinny(ctx, fn, type, 0, layout, &w, nullptr, static_cast<const uint16_t *>(x), &out, nullptr, &rows, 1,
-                           cols, batch, s);
+        return gemm_skinny(ctx, fn, type, 0, layout, &w, static_cast<const uint16_t *>(x), &out, nullptr, &rows, 1, cols, batch, s);
     size_t pf = 0, nc = 0;
     gemv_mt_workspace_need(type, layout, cols, rows, up != nullptr, batch, xh, ctx->ws.tune, &pf, &nc);
     if (int rc = ensure_ws(ctx, pf, nc, s)) return rc;
@@ -232,7 +234,7 @@ int gemv_mt(ns_ctx *ctx, const char *fn, int type, int layout, const void *w, co
 int gemm(ns_ctx *ctx, const char *fn, int type, int layout, int acc, const void *w, const void *up,
          const uint16_t *x, void *out, uint32_t cols, uint32_t rows, uint32_t batch, hipStream_t s) {
     size_t wf = 0, wc = 0;
-    gemm_workspace_need(type, layout, cols, rows, batch, up != nullptr, ctx->ws.tune, &wf, &wc);
+    gemm_workspace_need(type, layout, acc, cols, rows, batch, up != nullptr, ctx->ws.tune, &wf, &wc);
     if (int rc = ensure_ws(ctx, wf, wc, s)) return rc;
     const hipError_t e = launch_gemm(type, layout, acc, static_cast<const uint8_t *>(w),
                                      static_cast<const uint8_t *>(up), x, out, cols, rows, batch, ctx->ws, s);
@@ -635,8 +637,8 @@ extern "C" int ns_qkv(ns_ctx *ctx, const void *wq, const void *wk, const void *w
         const uint32_t rows[3] = {q_rows, kv_rows, kv_rows};
         const int nseg = wv ? 3 : 2;
         if (skinny_qkv_eligible(layout, cols, rows, nseg, wv ? v_type : 0, x, batch, ctx->ws.tune))
-            return gemm_skinny(ctx, fn, Q4_K, wv ? v_type : 0, layout, ws_, nullptr, x, outs, wv ? nullptr : v, rows, nseg,
-                               cols, batch, s);
+            return gemm_skinny(ctx, fn, Q4_K, wv ? v_type : 0, layout, ws_, x, outs, wv ? nullptr : v, rows, nseg, cols,
+                               batch, s);
     }
     // Q, K and V each stream their own weights once; x (fp16 [batch][cols]) is re-read
     // from the caches.  Batch 2-4 takes the small-batch kernels, larger batches the GEMM.

@@ -973,22 +973,20 @@ static bool use_gemm_reg(int type, int layout, const Tuning &t) {
     return layout == CDNA4 && type == Q4_K && t.gemm_q4_reg != 0;
 }
 
-void gemm_workspace_need(int type, int layout, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
+// What the kernel that launch_gemm runs needs (the same choices in the same order).
+void gemm_workspace_need(int type, int layout, int acc, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
                          const Tuning &t, size_t *floats, size_t *counters) {
-    // FP16 mode on CDNA4 runs ns_gemm_f16.hip; the need covers both modes
-    size_t f16_floats = 0, f16_counters = 0;
-    if (layout == CDNA4) gemm_f16_workspace_need(cols, rows, batch, pair, t, &f16_floats, &f16_counters);
-    size_t f32_floats = 0, f32_counters = 0;
-    gemm_fp32_workspace_need(type, layout, cols, rows, batch, pair, t, &f32_floats, &f32_counters);
-    *floats = std::max(f16_floats, f32_floats);
-    *counters = std::max(f16_counters, f32_counters);
-    for (int acc : {ACC_FP32, ACC_FP16})
-        if (gemm_skinny_eligible(type, layout, acc, cols, rows, batch, pair, t)) {
-            size_t f = 0, c = 0;
-            gemm_skinny_workspace_need(type, cols, &rows, 1, batch, pair, acc, t, &f, &c);
-            *floats = std::max(*floats, f);
-            *counters = std::max(*counters, c);
-        }
+    if (gemm_skinny_eligible(type, layout, acc, cols, rows, batch, pair, t))
+        gemm_skinny_workspace_need(type, cols, &rows, 1, batch, pair, acc, t, floats, counters);
+    else
+        gemm_tile_workspace_need(type, layout, acc, cols, rows, batch, pair, t, floats, counters);
+}
+
+// The tile kernels' part of it.
+void gemm_tile_workspace_need(int type, int layout, int acc, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
+                              const Tuning &t, size_t *floats, size_t *counters) {
+    if (layout == CDNA4 && acc == ACC_FP16) gemm_f16_workspace_need(cols, rows, batch, pair, t, floats, counters);
+    else gemm_fp32_workspace_need(type, layout, cols, rows, batch, pair, t, floats, counters);
 }
 
 static void gemm_fp32_workspace_need(int type, int layout, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,

@@ -155,9 +155,12 @@ hipError_t launch_gemv_mfma(int type, const uint8_t *w, const uint8_t *up, const
 void gemv_mt_workspace_need(int type, int layout, uint32_t cols, uint32_t rows, bool pair, uint32_t batch, bool xh,
                             const Tuning &t, size_t *partial_floats, size_t *counters);
 
-// Workspace the prefill GEMM needs: Q4_K group sums of x, split-K parts, tile counters.
-void gemm_workspace_need(int type, int layout, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
+// Workspace that launch_gemm needs for these arguments: Q4_K group sums of x, split-K parts, tile counters.
+void gemm_workspace_need(int type, int layout, int acc, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
                          const Tuning &t, size_t *floats, size_t *counters);
+// The same without the few-token GEMM.
+void gemm_tile_workspace_need(int type, int layout, int acc, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
+                              const Tuning &t, size_t *floats, size_t *counters);
 
 // What the FP32-mode Q4_K prefill GEMMs read beside x, written by the group-sums
 // kernel, at float offsets from one base (each part starts on a 256-byte boundary):

@@ -13,13 +13,11 @@
 // streams, or two threads) race; callers order them.  The counters must start
 // at zero: each call clears the ones it uses with a small kernel before the
 // matmul (stream-ordered, no hipMemsetAsync, so the call can be captured).
-// A prefill GEMM whose default plan (split-K parts padded to whole tiles) does not
-// fit runs with one K part instead (no parts; only the Q4_K group sums of x), as
-// ns_matmul does with the gemm_kparts 1 tuning.  The array also holds a status
+// A prefill GEMM on the tile kernels whose default plan (split-K parts padded to whole
+// tiles) does not fit runs with one K part instead (no parts; only the Q4_K group sums of
+// x), as ns_matmul does with the gemm_kparts 1 tuning; the few-token GEMM's parts always fit.  The array also holds a status
 // word for bounded cross-workgroup waits that ran out, read by ns_noalloc_status.
 #include <hip/hip_runtime.h>
-
-#include <algorithm>
 
 #include <mutex>
 #include <string>
@@ -105,13 +103,15 @@ extern "C" int ns_matmul_noalloc(const void *w, int type, int layout, uint32_t c
     Tuning t;
     size_t need_f = 0, need_c = 0;
     const auto fits = [&] { return need_f <= kScratchFloats && need_c <= kScratchCounters; };
-    if (batch == 1) gemv_workspace_need(type, layout, cols, rows, false, t, &need_f, &need_c);
+    const bool skinny = batch <= 4 && half_input && skinny_small_batch(type, layout, cols, rows, in, batch, t);
+    if (skinny) gemm_skinny_workspace_need(type, cols, &rows, 1, batch, false, ACC_FP32, t, &need_f, &need_c);
+    else if (batch == 1) gemv_workspace_need(type, layout, cols, rows, false, t, &need_f, &need_c);
     else if (batch <= 4) gemv_mt_workspace_need(type, layout, cols, rows, false, batch, half_input != 0, t, &need_f, &need_c);
     else {
-        gemm_workspace_need(type, layout, cols, rows, batch, false, t, &need_f, &need_c);
+        gemm_workspace_need(type, layout, ACC_FP32, cols, rows, batch, false, t, &need_f, &need_c);
         if (!fits()) {  // no split-K parts: the GEMM keeps its whole K range per tile
             t.gemm_kparts = 1;
-            gemm_workspace_need(type, layout, cols, rows, batch, false, t, &need_f, &need_c);
+            gemm_workspace_need(type, layout, ACC_FP32, cols, rows, batch, false, t, &need_f, &need_c);
         }
     }
     if (!fits())
@@ -128,15 +128,6 @@ extern "C" int ns_matmul_noalloc(const void *w, int type, int layout, uint32_t c
     ws.err = sm->err;
     ws.tune = t;
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    // batch 2-4: the same choice of kernel as ns_matmul (its parts: at most one round of workgroups' tiles,
-    // 1 Mi floats, inside the scratch whatever the shape)
-    const bool skinny = batch <= 4 && half_input && skinny_small_batch(type, layout, cols, rows, in, batch, t);
-    if (skinny) {
-        size_t f = 0, c = 0;
-        gemm_skinny_workspace_need(type, cols, &rows, 1, batch, false, ACC_FP32, t, &f, &c);
-        if (f > kScratchFloats || c > kScratchCounters) return fail(NS_ERR_UNSUPPORTED, std::string(fn) + ": scratch");
-        need_c = std::max(need_c, c);
-    }
     if (need_c) {
         clear_counters<<<dim3(uint32_t((need_c + 255) / 256)), dim3(256), 0, s>>>(ws.counters, uint32_t(need_c));
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return fail(NS_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));

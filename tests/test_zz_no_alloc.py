@@ -52,14 +52,13 @@ def test_noalloc_matches_matmul(ctx, first, second):
 
 
 PREFILL_CASES = [  # (first call, second call on a smaller input): (qtype, rows, cols, batch)
-    ((N.Q6_K, 3840, 15360, 1024), (N.Q4_K, 15360, 3840, 300)),
-    ((N.Q4_K, 3840, 15360, 256), (N.Q6_K, 3840, 15360, 5)),
+    ((N.Q6_K, 3840, 15360, 1024), (N.Q4_K, 4096, 3840, 1800)),
 ]
 
 
-@pytest.mark.parametrize("first,second", PREFILL_CASES, ids=["q6down1024-q4gate300", "q4down256-q6down5"])
+@pytest.mark.parametrize("first,second", PREFILL_CASES, ids=["q6down1024-q4proj1800"])
 def test_noalloc_prefill_matches_matmul_with_one_k_part(ctx, first, second):
-    """Above batch 4 the static scratch cannot hold the default plan's split-K parts (a
+    """The static scratch cannot hold the parts that the tile kernels split K into by default (a
     batch-1024 Q6_K down needs ~63 MB): the GEMM runs with one K part, as ns_matmul does with
     the gemm_kparts 1 tuning, and equals it bit for bit; the status stays clear."""
     for k, (qtype, rows, cols, batch) in enumerate((first, second)):
@@ -76,6 +75,26 @@ def test_noalloc_prefill_matches_matmul_with_one_k_part(ctx, first, second):
         N.noalloc_status()
         assert not torch.isnan(ref).any()
         assert torch.equal(got, ref), (k, qtype, rows, cols, batch)
+
+
+@pytest.mark.parametrize("qtype,layout,rows,cols,batch", [
+    (N.Q6_K, N.CDNA4, 3840, 15360, 5), (N.Q4_K, N.CDNA4, 3840, 15360, 5), (N.Q6_K, N.CDNA4, 3840, 15360, 32),
+    (N.Q4_K, N.CDNA4, 3840, 15360, 256), (N.Q4_K, N.CDNA4, 15360, 3840, 300), (N.Q4_K, N.ROW_MAJOR, 2048, 3840, 64),
+    (N.Q4_K, N.CDNA4, 3840, 15360, 600), (N.Q6_K, N.ROW_MAJOR, 2048, 15360, 3)])
+def test_noalloc_few_tokens_match_matmul(ctx, qtype, layout, rows, cols, batch):
+    """Where ns_matmul takes the few-token GEMM, whose parts fit the scratch, the call runs the same plan: equal
+    bit for bit with nothing tuned, whatever the tile kernels would have needed (at 600 tokens of a 15,360-column
+    Q4_K down more than the scratch even with one K part)."""
+    host = N.synth_weights(qtype, 340, rows, cols)
+    img = host if layout == N.ROW_MAJOR else N.retile(host, qtype, cols, rows, N.ROW_MAJOR, layout)
+    w = torch.from_numpy(np.ascontiguousarray(img)).cuda()
+    x = torch.from_numpy(N.synth_normal_f16(341, batch * cols).view(np.int16)).cuda()
+    ref, got = (torch.full((batch, rows), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2))
+    ctx.matmul(w, qtype, layout, cols, rows, batch, x, ref, half_input=True)
+    N.matmul_noalloc(w, qtype, layout, cols, rows, batch, x, got, half_input=True)
+    N.noalloc_status()
+    assert not torch.isnan(ref).any()
+    assert torch.equal(got, ref)
 
 
 def test_noalloc_refuses_shapes_past_the_scratch():
