@@ -719,7 +719,7 @@ F16Plan plan_f16(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const 
     F16Plan best{};
     uint32_t best_cost = ~0u;
     for (uint32_t mi : {8u, 4u}) {
-        if (t.f16_mi > 0 && uint32_t(t.f16_mi) != mi) continue;
+        if ((t.f16_mi == 4 || t.f16_mi == 8) && uint32_t(t.f16_mi) != mi) continue;  // other values force nothing
         F16Plan p{mi, (batch + 32 * mi - 1) / (32 * mi), ncol, 1, 0};
         const uint32_t tiles = p.ntok * ncol, sb = mi == 8 ? 70 : 38;
         for (uint32_t kp = 1; kp == 1 || (kp <= 2 * mi && kp * 2 <= nb && tiles * kp <= cus); kp *= 2) {

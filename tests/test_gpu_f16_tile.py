@@ -69,3 +69,17 @@ def test_f16_tile128_gate_up(ctx, tune, batch, kparts):
         out.append(h.cpu().numpy())
     assert rel_err(f16_value(out[0].view(np.uint16)), O.gate_up_geglu_prefill(O.ROW_MAJOR, hg, hu, cols, rows, batch, bits, 1)) <= 5e-3
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("value", [1, 5, 16])
+def test_f16_unknown_tile_forces_nothing(ctx, tune, value):
+    """Values of f16_mi that name no tile leave the plan's: the same bits."""
+    cols, rows, batch = 1024, 192, 140
+    _, w = weights(N.Q4_K, 0x76, rows, cols)
+    x = torch.from_numpy(N.synth_normal_f16(0x77, batch * cols).view(np.int16)).cuda()
+    y = [torch.full((batch, rows), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2)]
+    for out, mi in zip(y, (0, value)):
+        tune("f16_mi", mi)
+        ctx.ffn_down(w, N.Q4_K, N.CDNA4, cols, rows, batch, x, out, half_input=True, fast_swa=True)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y[0]).all() and torch.equal(y[0], y[1])
