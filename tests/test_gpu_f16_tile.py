@@ -1,7 +1,7 @@
 """The FP16-mode prefill GEMM's 128-token tile (f16_mi 4, csrc/ns_gemm_f16.hip): against the oracle at
 ragged batches around its tiles, and bit for bit against the 256-token tile (the same parts in the same
 order), with the split-K finished by the reduce-scatter, also where a part owns half an MFMA tile
-(8 parts), and by the last arrival."""
+(8 parts, and 16 of the 256-token tile), and by the last arrival."""
 import numpy as np
 import pytest
 
@@ -83,3 +83,23 @@ def test_f16_unknown_tile_forces_nothing(ctx, tune, value):
         ctx.ffn_down(w, N.Q4_K, N.CDNA4, cols, rows, batch, x, out, half_input=True, fast_swa=True)
     torch.cuda.synchronize()
     assert torch.isfinite(y[0]).all() and torch.equal(y[0], y[1])
+
+
+@pytest.mark.parametrize("qtype", [N.Q4_K, N.Q6_K], ids=["q4k", "q6k"])
+def test_f16_tile256_sixteen_parts(ctx, tune, qtype):
+    """16 K parts of the 256-token tile, the most that the plan takes: each part finishes one 16-token unit of the
+    reduce-scatter, bit for bit what the last arrival adds up; a ragged second token tile and column tile."""
+    cols, rows, batch = 8192, 320, 300
+    host, w = weights(qtype, 0x78, rows, cols)
+    bits = N.synth_normal_f16(0x79, batch * cols).reshape(batch, cols)
+    x = torch.from_numpy(bits.view(np.int16)).cuda()
+    tune("f16_mi", 8)
+    tune("gemm_kparts", 16)
+    y = [torch.full((batch, rows), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2)]
+    for rs, out in enumerate(y):
+        tune("gemm_rs", rs)
+        ctx.ffn_down(w, qtype, N.CDNA4, cols, rows, batch, x, out, half_input=True, fast_swa=True)
+    torch.cuda.synchronize()
+    last, scatter = (t.cpu().numpy() for t in y)
+    assert np.array_equal(last.view(np.uint32), scatter.view(np.uint32))
+    assert rel_err(scatter, O.gemm(qtype, O.ROW_MAJOR, host, cols, rows, batch, bits, 1)) <= 1e-3

@@ -428,9 +428,9 @@ def test_prefill_q4k_down_full_size(ctx, acc):
 @pytest.mark.parametrize("acc", [N.ACC_FP32, N.ACC_FP16], ids=["fp32acc", "fp16acc"])
 @pytest.mark.parametrize("batch", [512, 256])
 def test_prefill_q6k_down_many_parts(ctx, batch, acc):
-    """The down projection below batch 1024 splits K into 8 parts (fewer token tiles): the
-    last workgroup adds them four at a time.  128-row samples against the oracle in the same
-    mode, and the values do not depend on the part count beyond fp32 rounding (kparts 4)."""
+    """The down projection below batch 1024 splits K into many parts (fewer token tiles): the tile
+    kernels, which test_gpu_tile_kernels.py runs this on, into 8, at 256 tokens in the FP16 mode into 16,
+    added four at a time.  128-row samples against the oracle in the same mode."""
     D, F = 3840, 15360
     hd, wd = weights(N.Q6_K, 67, D, F, N.CDNA4)
     x = N.synth_normal_f16(68, batch * F).reshape(batch, F)

@@ -118,7 +118,9 @@ def test_lm_head_batch4(ctx):
 # ---- the MFMA form (ns_gemv_mfma.hip, CDNA4 layout; mt_mfma = 0 selects the VALU kernel) ----
 
 def _both_kernels(ctx, tune, fn):
-    """fn() run on the MFMA kernel and on the VALU kernel (host copies)."""
+    """fn() run on the MFMA kernel and on the VALU kernel (host copies); fp16 Q4_K would take the few-token
+    GEMM instead."""
+    tune("gemm_skinny", 0)
     a = fn()
     tune("mt_mfma", 0)
     b = fn()

@@ -1,5 +1,6 @@
-"""The 128- and 256-token tile GEMMs at the batches that the few-token GEMM takes by default: the
-prefill tests of the other modules once more, on a context that never selects it (gemm_skinny 0)."""
+"""The 128- and 256-token tile GEMMs and the small-batch kernels at the batches that the few-token GEMM takes
+by default: the prefill and small-batch tests of the other modules once more, on a context that never selects
+it (gemm_skinny 0)."""
 import numpy as np
 import pytest
 
@@ -19,7 +20,8 @@ from test_gpu_parity import (test_prefill_down_small, test_prefill_gate_up_small
                              test_prefill_q6k_down_many_parts, test_prefill_split_k)
 from test_gpu_q6k_scales import (test_prefill_down_full_range_scales,  # noqa: E402,F401
                                  test_prefill_down_full_range_scales_power_of_two_d)
-from test_gpu_shape_sweep import test_gate_up_sweep, test_prefill_sweep  # noqa: E402,F401
+from test_gpu_shape_sweep import test_gate_up_sweep, test_prefill_sweep, test_small_batch_sweep  # noqa: E402,F401
+from test_gpu_small_batch import test_ffn_down_small_batch_half_input, test_matmul_small_batch  # noqa: E402,F401
 
 
 @pytest.fixture(scope="module")
