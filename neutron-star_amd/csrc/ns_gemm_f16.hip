@@ -711,6 +711,9 @@ struct F16Plan {
 // tile decodes each weight fragment for half the matrix work (3.8 us per super-block against 7.0), so
 // it pays where it fills a round better: gate/up pair at 225 tokens 82 -> 65 us (240 workgroups
 // without split K instead of 120 tiles in two K parts), downs at 225 61-70 -> 49-55, at 320 78-81 -> 64.
+// Where 256-token tiles make more than two rounds, 128-token ones have to cost less with their rounds not
+// rounded up too (workgroups start as others end): 163,840 x 4,096 at 138 tokens 298 us in 256-token tiles, 347
+// in 128-token ones; 30,720 x 4,096 at 1,203 tokens 324 / 345; over 38 random shapes 0.86-1.04 of their time.
 // K is split only while all parts run in one round (downs at 600 tokens: 45 tiles in 8 parts, 360
 // workgroups, took 173-195 us; in 4 parts 102).
 F16Plan plan_f16(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t) {
@@ -721,6 +724,7 @@ F16Plan plan_f16(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const 
     for (uint32_t mi : {8u, 4u}) {
         if ((t.f16_mi == 4 || t.f16_mi == 8) && uint32_t(t.f16_mi) != mi) continue;  // other values force nothing
         F16Plan p{mi, (batch + 32 * mi - 1) / (32 * mi), ncol, 1, 0};
+        if (mi == 4 && best.mi == 8 && best.ntok * ncol > 2 * cus && p.ntok * 38 > best.ntok * 70) continue;
         const uint32_t tiles = p.ntok * ncol, sb = mi == 8 ? 70 : 38;
         for (uint32_t kp = 1; kp == 1 || (kp <= 2 * mi && kp * 2 <= nb && tiles * kp <= cus); kp *= 2) {
             const uint32_t cost = (tiles * kp + cus - 1) / cus * (60 + (nb + kp - 1) / kp * sb) + (kp > 1 ? 100 : 0);
