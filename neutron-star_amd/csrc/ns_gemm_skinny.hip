@@ -443,12 +443,14 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
     // registers, filled one super-block earlier, changed nothing: 20.3 us either way for the FP16 pair
     // at 5 tokens, and the FP32 pair took 23.0 instead of 21.5.)
     constexpr bool kMin = Q4 && !F16;
-    // The 32-token tile (which also takes batch 2-4) has the registers for short chains of sums: one per quarter
-    // of the super-block, added up in T, and one for EX's small second fragments.  Together with the pairwise sum
-    // over the waves and the min term's small pieces first, error against 64 bits of row-major projections
-    // (3840 x 4096, 3 tokens): Q4_K 1.55e-7 in one chain per super-block, 1.28e-7 in two, 1.09e-7 now; Q6_K
-    // 1.42e-7 in one, 0.93e-7 now (the small-batch VALU kernel: 1.12e-7 and 1.04e-7), at the same times.
+    // The 32-token tile (which also takes batch 2-4) has the registers for short chains of sums: one per half of
+    // the super-block, per quarter for row-major Q4_K, added up in T (each once the next is under way, the last
+    // after the loads), and one for EX's small second fragments.  Together with the pairwise sum over the waves and
+    // the min term's small pieces first, error against 64 bits at 3 tokens of 3840 x 4096, in brackets that of the
+    // small-batch kernel: row-major Q4_K 1.09e-7 (1.12e-7; in halves 1.18e-7, in one chain 1.55e-7), Q6_K
+    // 1.01e-7 (1.04e-7; in one chain 1.42e-7), CDNA4 Q4_K 1.18e-7 (1.40e-7).  Quarters everywhere took 0.5-2% more time.
     constexpr bool kShort = !F16 && MI == 1;
+    constexpr int kChain = !kShort ? 8 : Q4 && ROW ? 2 : 4;  // in groups of 32
     auto group_sum = [](int s, half4_t sel, half4_t xv, float4_t c) {  // s is a constant once unrolled
         return s == 0   ? __builtin_amdgcn_mfma_f32_4x4x4f16(sel, xv, c, 4, 0, 0)
                : s == 1 ? __builtin_amdgcn_mfma_f32_4x4x4f16(sel, xv, c, 4, 1, 0)
@@ -513,10 +515,10 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
 #pragma unroll
                             for (int j = 0; j < NJ; ++j) {
                                 if constexpr (F16) acc[i][j] = mfma(av[i], fb[j], acc[i][j]);
-                                else S[i][j] = mfma(av[i], fb[j], grp % (kShort ? 2 : 8) == 0 && e == 0 ? float16_t{} : S[i][j]);
+                                else S[i][j] = mfma(av[i], fb[j], grp % kChain == 0 && e == 0 ? float16_t{} : S[i][j]);
                                 if constexpr (EX) S2[j] = mfma(av[i], fb2[j], grp == 0 && e == 0 ? float16_t{} : S2[j]);
                                 if constexpr (kShort) {
-                                    if (grp % 2 == 1 && e == 1) T[j] = grp == 1 ? S[i][j] : T[j] + S[i][j];
+                                    if (grp % kChain == kChain - 1 && grp < 7 && e == 1) T[j] = grp < kChain ? S[i][j] : T[j] + S[i][j];
                                 }
                             }
                         }
@@ -561,7 +563,9 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
                     for (int j = 0; j < NJ; ++j)
 #pragma unroll
                         for (int v = 0; v < 16; ++v) {
-                            const float sum = !kShort ? S[i][j][v] : EX ? T[kShort ? j : 0][v] + S2[EX ? j : 0][v] : T[kShort ? j : 0][v];
+                            float sum = S[i][j][v];
+                            if constexpr (kShort) sum = T[j][v] + sum;
+                            if constexpr (EX) sum += S2[j][v];
                             acc[i][j][v] = __builtin_fmaf(d[j], sum, acc[i][j][v]);
                         }
                     if constexpr (kMin) {
@@ -772,8 +776,11 @@ Plan plan_skinny(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32
             if (wk == 8 && mi == 4) continue;  // no room for its x stages
             if (t.skinny_wk > 0 && uint32_t(t.skinny_wk) != wk && mi < 4) continue;
             const uint32_t ncol = col_tiles(rows, nseg, pair, wk), tiles = ncol * ntok;
-            for (uint32_t kp = forced ? forced : 1; kp <= nb && (forced ? kp == forced : kp == 1 || tiles * kp <= cus); ++kp) {
-                const uint32_t rounds = (tiles * kp + cus - 1) / cus, iters = ((nb + kp - 1) / kp + wk - 1) / wk;
+            // of the parts that leave a wave as many super-blocks, the fewest
+            for (uint32_t kp = forced ? forced : 1, iters = 0; kp <= nb && (forced || kp == 1 || tiles * kp <= cus);
+                 kp = iters > 1 && !forced ? (nb + (iters - 1) * wk - 1) / ((iters - 1) * wk) : nb + 1) {
+                const uint32_t rounds = (tiles * kp + cus - 1) / cus;
+                iters = (nb + kp * wk - 1) / (kp * wk);
                 const uint32_t cost = 60 + rounds * (60 + iters * iter_cost[m]) + (kp > 1 ? 10 + 4 * kp * mi : 0);
                 if (cost < best_cost) {
                     best_cost = cost;
@@ -917,8 +924,9 @@ double small_us(int type, int layout, uint32_t cols, uint32_t rows, uint32_t bat
 
 }  // namespace
 
-// Row-major tensors by the two estimates, 5% for their error; short rows, whose estimates are loose, stay there.
-// Over 8,900 random shapes the choice is more than 5% slower than the small-batch kernels in 0.3% of them (2,048 x
+// Row-major tensors by the two estimates (Q4_K at 3-4 tokens, where that of the small-batch kernel is low, by 5%
+// more); short rows, whose estimates are loose, stay there.  Over 8,900 random shapes the choice is more than 5%
+// slower than the small-batch kernels in 0.7% of them, and more than 5% slower than this one in 3% (2,048 x
 // 3,840 at 3 tokens 9.4 us here, 12.4 there; Q6_K 64 x 3,840 13 / 10, 65,536 x 2,304 55 / 76).  Q4_K on CDNA4:
 // here but for tall matrices of up to 15 super-blocks, which the small-batch kernel walks with a wave per slab and
 // no hand-off (at up to two slabs per CU 0.58-1.00 of its time, at 65,536-262,144 rows 1.1-2.0 of it).  Q6_K on
@@ -932,7 +940,7 @@ bool skinny_small_batch(int type, int layout, uint32_t cols, uint32_t rows, cons
     Tuning plain = t;
     plain.gemm_kparts = 0;
     return skinny_us(route_of(type, layout, false), plan_skinny(type, cols, &rows, 1, batch, false, false, plain), cols, &rows, 1,
-                     batch, false) <= 0.95 * small_us(type, layout, cols, rows, batch);
+                     batch, false) <= (type == Q4_K && batch > 2 ? 1.05 : 1.0) * small_us(type, layout, cols, rows, batch);
 }
 
 // Q, K and V (or Q and a K that is V too) in one launch: against the launches of their own that they would take.
@@ -944,19 +952,23 @@ bool skinny_qkv_eligible(int layout, uint32_t cols, const uint32_t *rows, int ns
     if (t.gemm_skinny > 0) return batch <= uint32_t(t.gemm_skinny);
     Tuning plain = t;
     plain.gemm_kparts = 0;
-    double q6 = 0, total = 0, apart = last_type ? 0 : 4;  // a tied V is a copy of K
+    double total = 0;
+    for (int s = 0; s < nseg; ++s) total += rows[s];
+    Route mix = route_of(Q4_K, layout, false);
+    if (last_type == Q6_K)  // by the share of the column tiles that are Q6_K
+        for (int m = 0; m < 2; ++m) mix.sb[m] += (route_of(Q6_K, layout, false).sb[m] - mix.sb[m]) * (rows[nseg - 1] / total);
+    const double together =
+        skinny_us(mix, plan_skinny(Q4_K, cols, rows, nseg, batch, false, false, plain), cols, rows, nseg, batch, false);
+    if (together <= 18) return true;  // less than the launches alone, and the host would take longer to find out
+    double apart = last_type ? 0 : 4;  // a tied V is a copy of K
     for (int s = 0; s < nseg; ++s) {
         const int type = s == nseg - 1 && last_type ? last_type : Q4_K;
         const Route &r = route_of(type, layout, false);
         const double own = skinny_us(r, plan_skinny(type, cols, rows + s, 1, batch, false, false, plain), cols, rows + s, 1, batch, false);
         if (!small) apart += std::min(own, tile_us(r, type, layout, cols, rows[s], batch, false, plain));
         else apart += skinny_small_batch(type, layout, cols, rows[s], x, batch, t) ? own : small_us(type, layout, cols, rows[s], batch);
-        total += rows[s];
-        if (type == Q6_K) q6 += rows[s];
     }
-    Route mix = route_of(Q4_K, layout, false);  // by the share of the column tiles that are Q6_K
-    for (int m = 0; m < 2; ++m) mix.sb[m] += (route_of(Q6_K, layout, false).sb[m] - mix.sb[m]) * (q6 / total);
-    return skinny_us(mix, plan_skinny(Q4_K, cols, rows, nseg, batch, false, false, plain), cols, rows, nseg, batch, false) <= apart;
+    return together <= apart;
 }
 
 void gemm_skinny_workspace_need(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair,
