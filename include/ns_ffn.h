@@ -134,9 +134,14 @@ int ns_ctx_set_tuning(ns_ctx *ctx, const char *key, int value);
  *   batch 2-4, fp32 or fp16     -> small-batch GEMV streaming the weights once for all tokens
  *                                  (gemma_q4k/q6k_mm_fast[_f16][_metal], metal:125-177, mm:273);
  *                                  on the matrix cores for the CDNA4 layout, FP32 accumulation.
- *   batch  > 4, half_input != 0 -> dequant-into-LDS MFMA GEMM, FP32 accumulation (any layout:
- *                                  the reference's swizzled row-major kernels, metal:263-301,
- *                                  432-478, serve attention tensors that stay row-major).
+ *                                  fp16 input that is 16-byte aligned takes the few-token GEMM
+ *                                  instead where that is estimated the faster (Q4_K on CDNA4 and
+ *                                  ROW_MAJOR, Q6_K on ROW_MAJOR): as exact, but the sums' order and
+ *                                  so the last bits depend on the input's alignment.
+ *   batch  > 4, half_input != 0 -> MFMA GEMM, FP32 accumulation (any layout: the reference's
+ *                                  swizzled row-major kernels, metal:263-301, 432-478, serve
+ *                                  attention tensors that stay row-major): the few-token GEMM or
+ *                                  the 128- and 256-token tile kernels, by the faster estimate.
  *   batch  > 4, fp32 input      -> the same GEMM on x rounded to fp16 (round to nearest even),
  *                                  as the reference's tile loader converts fp32 x to half
  *                                  (metal:235, gemma_q{4,6}k_mma_swizzled, mm:274); the fp16
@@ -274,9 +279,10 @@ int ns_embedding(ns_ctx *ctx, const void *w, int type, int layout, uint32_t cols
 /* qkv (mm:311; gemma_qkv_q4_f16 / _q6v_f16 / _tied_v_f16, metal:442-454): the attention
  * projections of one layer in prefill.  x fp16 bits [batch][cols]; q fp32 [batch][q_rows];
  * k, v fp32 [batch][kv_rows].  wq, wk Q4_K; wv of v_type (Q4_K or Q6_K), or NULL for tied V
- * (V = K).  FP32 accumulation.  batch >= 2 (batch 2-4: the small-batch kernels; larger: the
- * prefill GEMM); any layout, ROW_MAJOR being the reference's (attention weights are not
- * re-laid by .nsmffn). */
+ * (V = K).  FP32 accumulation.  batch >= 2; any layout, ROW_MAJOR being the reference's (attention
+ * weights are not re-laid by .nsmffn).  One launch of the few-token GEMM where that is estimated the
+ * faster (batch 2-4: with x 16-byte aligned), else each matrix as ns_matmul (batch 2-4: the
+ * small-batch kernels; larger: the prefill GEMM). */
 int ns_qkv(ns_ctx *ctx, const void *wq, const void *wk, const void *wv, int v_type, int layout, uint32_t cols,
            uint32_t q_rows, uint32_t kv_rows, uint32_t batch, const uint16_t *x, float *q, float *k, float *v,
            void *stream);

@@ -724,6 +724,9 @@ __device__ __forceinline__ void skinny_body(const Args &a, const Item &item, u32
 template <int TYPE, int LAYOUT, int ACC, int MI>
 constexpr bool kExact = TYPE == Q6_K && ACC == ACC_FP32 && LAYOUT == ROW_MAJOR && MI == 1;
 
+// (Two instances spill: Q6_K in the FP16 mode with 128-token tiles 12 bytes per lane, the row-major mixed kernel
+// with 64-token tiles and WK 8 8 bytes.  Scratch accesses count as vector memory instructions too, in order, so
+// they can only make the counted waits of the main loop stricter.)
 template <int TYPE, int LAYOUT, int ACC, bool PAIR, int MI, int WK>
 __global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(const Args a) {
     // two LDS objects, so that the compiler does not take a DMA into one for a write to the other

@@ -224,8 +224,8 @@ bool skinny_qkv_eligible(int layout, uint32_t cols, const uint32_t *rows, int ns
                          uint32_t batch, const Tuning &t);
 // Batch 2-4 with fp16 x: whether it takes this kernel, where it is the faster one; it keeps the small-batch
 // kernels' precision (every product exact).  It reads x by 16-byte DMA, so x has to be aligned.  Not for the gate/up
-// pair: 19.9 us here against 21.2, but of the two it had the larger error against 64 bits (its gate and up
-// round to fp16 h on other sides).
+// pair, where neither is ahead: 21.8-22.1 us here at 2-4 tokens, 21.9-22.3 there, h 2.12e-4 from 64 bits (its
+// fp16 rounding) in both.
 bool skinny_small_batch(int type, int layout, uint32_t cols, uint32_t rows, const void *x, uint32_t batch, const Tuning &t);
 void gemm_skinny_workspace_need(int type, uint32_t cols, const uint32_t *rows, int nseg, uint32_t batch, bool pair,
                                 int acc, const Tuning &t, size_t *part_floats, size_t *counters);

@@ -111,9 +111,10 @@ public:
     FfnPath(const FfnPath &) = delete;
     FfnPath &operator=(const FfnPath &) = delete;
 
-    // mm:269-275: batch 1 -> dequant-fused GEMV; batch 2-4 -> the small-batch kernels (the
-    // weights streamed once for every token, fp32 or fp16 input); batch > 4 -> MFMA GEMM (FP32
-    // accumulation; fp32 input rounded to fp16 first, as the reference's tile loader does).
+    // mm:269-275: batch 1 -> dequant-fused GEMV; batch 2-4 -> the weights streamed once for
+    // every token (the small-batch kernels; 16-byte aligned fp16 input mostly the few-token
+    // GEMM); batch > 4 -> MFMA GEMM (FP32 accumulation; fp32 input rounded to fp16 first, as the
+    // reference's tile loader does).
     void matmul(hipStream_t e, const Tensor &w, const void *in, float *out, uint32_t batch,
                 bool half_input = false) const {
         check(ns_matmul(ctx_, w_.data(w), int(w.type), int(w_.layout(w)), cols(w), rows(w), batch, in,
