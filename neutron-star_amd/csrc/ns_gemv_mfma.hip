@@ -707,6 +707,11 @@ bool gemv_mfma_eligible(int layout, bool pair, bool xh, uint32_t batch, const Tu
     return layout == CDNA4 && t.mt_mfma != 0 && (!pair || (xh && batch >= 2));
 }
 
+uint32_t gemv_mfma_stream_grid(uint32_t cols, uint32_t rows, const Tuning &t) {
+    const Plan p = plan_mfma(rows, cols / kQK, false, t);
+    return stream_grid(p, (rows / kRowTile + p.S - 1) / p.S * p.KP, cols / kQK);
+}
+
 void gemv_mfma_workspace_need(uint32_t cols, uint32_t rows, bool pair, const Tuning &t, size_t *partial_floats,
                               size_t *counters) {
     const Plan p = plan_mfma(rows, cols / kQK, pair, t);
@@ -728,7 +733,7 @@ hipError_t launch_gemv_mfma(int type, const uint8_t *w, const uint8_t *up, const
     if (p.KP > 1 && (ws.partial_floats < size_t(slabs) * p.KP * p.M * NT * 64 || ws.counter_count < slabs))
         return hipErrorInvalidValue;
     const uint32_t nwg = (slabs + p.S - 1) / p.S * p.KP;
-    const uint32_t sgrid = stream_grid(p, nwg, nb);
+    const uint32_t sgrid = pair ? 0 : gemv_mfma_stream_grid(cols, rows, ws.tune);
     return dispatch_mfma(type, pair, xh, sgrid != 0, [&](auto k) {
         k<<<dim3(sgrid ? sgrid : nwg), dim3(p.S * p.M * p.P * 64), 0, stream>>>(w, up, x, batch, out, rows, nb, p, ws.partial,
                                                                  ws.counters);

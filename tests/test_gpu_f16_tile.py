@@ -103,23 +103,3 @@ def test_f16_tile256_sixteen_parts(ctx, tune, qtype):
     last, scatter = (t.cpu().numpy() for t in y)
     assert np.array_equal(last.view(np.uint32), scatter.view(np.uint32))
     assert rel_err(scatter, O.gemm(qtype, O.ROW_MAJOR, host, cols, rows, batch, bits, 1)) <= 1e-3
-
-
-def test_f16_many_rounds_take_the_larger_tile(ctx, tune):
-    """640 tiles of 256 tokens hold 138 tokens of 163,840 rows; 1,280 of 128 tokens take 1.16 times as long."""
-    cols, rows, batch = 4096, 163840, 138
-    w = torch.randint(0, 256, (rows * 16 * 210,), dtype=torch.uint8, device="cuda")
-    x = torch.randn(batch, cols, device="cuda").half()
-    y = torch.empty((batch, rows), dtype=torch.float32, device="cuda")
-    best = {}
-    for mi in (0, 8, 0, 8):
-        tune("f16_mi", mi)
-        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-        for n in (2, 12):
-            a.record()
-            for _ in range(n):
-                ctx.ffn_down(w, N.Q6_K, N.CDNA4, cols, rows, batch, x, y, half_input=True, fast_swa=True)
-            b.record()
-            b.synchronize()
-        best[mi] = min(best.get(mi, float("inf")), a.elapsed_time(b))
-    assert best[0] <= 1.08 * best[8], best

@@ -1,7 +1,7 @@
 """Batch 2-4 on tensors of more slabs than one round of workgroups holds (csrc/ns_gemv_mfma.hip, the
 streaming form): the same numbers as from calls on 65,536-row pieces, which give every wave one slab.
 Slab counts just past one round and just past a half-full last one, that leave waves of the last step without
-a slab, and of three steps; one, two, three and fifteen super-blocks per row.  And which slab counts stream."""
+a slab, and of three steps; one, two, three and fifteen super-blocks per row."""
 import pytest
 
 import nsffn as N
@@ -40,28 +40,3 @@ def test_streaming_matches_pieces(qtype, half, rows, nb, batch):
         else:
             assert torch.allclose(y[:, r0:r0 + n], z, rtol=0, atol=2.0 ** -24 * 8 * cols ** 0.5 * float(z.abs().max())), r0
     ctx.close()
-
-
-def time_us(call):
-    a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-    best = float("inf")
-    for _ in range(5):
-        a.record()
-        for _ in range(10):
-            call()
-        b.record()
-        b.synchronize()
-        best = min(best, a.elapsed_time(b) * 100)
-    return best
-
-
-def test_short_last_round_does_not_stream():
-    """163,840 rows are 1.25 rounds of workgroups: they take 1.25 times as long as the one round of 131,072 rows,
-    and some 1.3 with the second staging of x (measured 1.31-1.38); streamed by fewer waves they took 1.6."""
-    ctx = N.Context(0)
-    cols = 3840
-    w = torch.randint(0, 256, (163840 * 15 * 210,), dtype=torch.uint8, device="cuda")
-    x, y = torch.randn(3, cols, device="cuda"), torch.empty(3, 163840, device="cuda")
-    t = [time_us(lambda: ctx.matmul(w, N.Q6_K, N.CDNA4, cols, rows, 3, x, y)) for rows in (131072, 163840)]
-    ctx.close()
-    assert t[1] <= 1.47 * t[0], t

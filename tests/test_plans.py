@@ -1,0 +1,69 @@
+"""Which kernel form the launch plans choose, on the CPU: the plans' C++ functions (csrc/ns_internal.hpp) called in
+the built library, with 256 CUs where there is no GPU.  For rules whose two sides give the same bits."""
+import ctypes
+import os
+import re
+
+import pytest
+
+import nsffn as N
+
+U32, SIZE = ctypes.c_uint32, ctypes.c_size_t
+
+
+def tuning(**overrides):
+    """struct Tuning with its defaults, read from the header."""
+    text = open(os.path.join(N.PKG, "csrc", "ns_internal.hpp")).read()
+    body = re.search(r"struct Tuning \{(.*?)\n\};", text, re.S).group(1)
+    fields = {k: int(v) for k, v in re.findall(r"^\s*int (\w+) = (-?\d+);", body, re.M)}
+    assert set(overrides) <= set(fields)
+    fields.update(overrides)
+    return (ctypes.c_int * len(fields))(*fields.values())
+
+
+def function(mangled, restype):
+    f = getattr(N.lib(), mangled)
+    f.restype = restype
+    return f
+
+
+@pytest.mark.parametrize("rows,grid", [(131072, 0), (139264, 0), (163840, 0), (196608, 0), (212992, 416), (262144, 512),
+                                       (278528, 0), (327680, 0), (360448, 470), (393216, 512)])
+def test_stream_only_with_a_full_last_round(rows, grid):
+    """The batch 2-4 kernel streams where its last round of 512 workgroups is more than half full (rows / 256 of them):
+    163,840 rows of 3,840 columns, 1.25 rounds, took 1.15-1.2 times as long streamed."""
+    f = function("_ZN2ns21gemv_mfma_stream_gridEjjRKNS_6TuningE", U32)
+    assert f(U32(3840), U32(rows), tuning()) == grid
+
+
+@pytest.mark.parametrize("cols,rows,batch,tile", [
+    (4096, 163840, 138, 8), (4096, 30720, 1203, 8), (8192, 30720, 1548, 8), (3840, 30720, 1713, 8),
+    (3840, 15360, 300, 4), (3840, 3840, 225, 4), (3840, 163840, 300, 4)])
+def test_f16_tile_over_many_rounds(cols, rows, batch, tile):
+    """The FP16-mode GEMM's tile: of 256 tokens (8) where that makes more than two rounds and 128-token tiles (4) only
+    look cheaper by their rounds rounded up; 128-token ones where they fill a round better or pad less."""
+    f = function("_ZN2ns13gemm_f16_costEjjjbRKNS_6TuningE", U32)
+    cost = {mi: f(U32(cols), U32(rows), U32(batch), ctypes.c_bool(False), tuning(f16_mi=mi)) for mi in (0, 4, 8)}
+    assert cost[4] != cost[8]
+    assert cost[0] == cost[tile]
+
+
+def test_context_need_covers_every_batch():
+    """A context is sized at multiples of 16 tokens: no batch between them needs more, on either kind of kernel."""
+    tile = function("_ZN2ns24gemm_tile_workspace_needEiiijjjbRKNS_6TuningEPmS3_", None)
+    skinny = function("_ZN2ns26gemm_skinny_workspace_needEijPKjijbiRKNS_6TuningEPmS5_", None)
+    t, top = tuning(), {}
+    for step in (1, 16):
+        most = [0, 0]
+        for qtype, cols, rows, pair in ((N.Q4_K, 3840, 15360, True), (N.Q4_K, 15360, 3840, False), (N.Q6_K, 15360, 3840, False)):
+            for batch in range(16 if step == 16 else 5, 2049, step):
+                for acc in (N.ACC_FP32, N.ACC_FP16):
+                    f, c = SIZE(), SIZE()
+                    for call in (lambda: tile(qtype, N.CDNA4, acc, U32(cols), U32(rows), U32(batch), ctypes.c_bool(pair), t,
+                                              ctypes.byref(f), ctypes.byref(c)),
+                                 lambda: skinny(qtype, U32(cols), (U32 * 1)(rows), 1, U32(batch), ctypes.c_bool(pair), acc, t,
+                                                ctypes.byref(f), ctypes.byref(c))):
+                        call()
+                        most = [max(most[0], f.value), max(most[1], c.value)]
+        top[step] = most
+    assert top[1] == top[16]
