@@ -104,6 +104,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_reg_kernel(
     uint32_t ncol_tiles, uint32_t kparts, uint32_t wbytes, uint32_t rs_spin, uint32_t *__restrict__ err) {
     __shared__ __attribute__((aligned(16))) u32x4 Xs[XBUF][TT * 8];
     __shared__ uint32_t last_flag, late_flag;
+    constexpr float kResidue = PAIR ? 1.0f : 0.015625f;  // of the hi sums, in the min term's second fragment
 
     const uint32_t tid = threadIdx.x, lane = tid & 63, hl = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -228,14 +229,17 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_reg_kernel(
                     // Min term B fragments.  b_g = fp16(m_g * (-dmin / E)) sits in k 0-7 (against
                     // the hi sums) and again in k 8-15 (against the lo sums); its rounding residue
                     // fp16(m_g * (-dmin / E) - b_g) is a second fragment, k 0-7 only, against the
-                    // hi sums, so the min term keeps ~22 significant bits (b_g alone: 11).
+                    // hi sums, so the min term keeps ~22 significant bits (b_g alone: 11).  Plain outputs:
+                    // the residue times 64 meets the hi sums times 1/64, as at around 2^-17 it would be an
+                    // fp16 subnormal and lose most of its bits (outputs 1.08e-6 off in any number of K parts,
+                    // 2.4e-7 to 8.7e-7 now).  The pair's h is rounded to fp16, which hides both.
                     const float f = -dmin * re * 0.00006103515625f;
                     half8_t bh, bl;
 #pragma unroll
                     for (int gg = 0; gg < 8; ++gg) {
                         const float v = f * float(q4_m(sc, gg));
                         bh[gg] = _Float16(v);
-                        bl[gg] = hl == 0 ? _Float16(v - float(bh[gg])) : _Float16(0.0f);
+                        bl[gg] = hl == 0 ? _Float16((v - float(bh[gg])) * (1.0f / kResidue)) : _Float16(0.0f);
                     }
                     bmin[j] = bh;
                     bmin_lo[j] = bl;
@@ -286,12 +290,24 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_reg_kernel(
 #pragma unroll
                 for (int i = 0; i < MI; ++i)
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                            __builtin_bit_cast(half8_t, xsf[i]), bmin_lo[j],
-                            __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, xsf[i]), bmin[j],
-                                                                   acc[i][j], 0, 0, 0),
-                            0, 0, 0);
+                    for (int j = 0; j < NJ; ++j) {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, xsf[i]), bmin[j],
+                                                                           acc[i][j], 0, 0, 0);
+                        if constexpr (PAIR)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, xsf[i]),
+                                                                               bmin_lo[j], acc[i][j], 0, 0, 0);
+                    }
+                if constexpr (!PAIR)
+#pragma unroll
+                    for (int i = 0; i < MI; ++i) {
+                        // not to be multiplied before this point: earlier, the step would wait for the loads of
+                        // the sums (3 us of a call of 30)
+                        asm volatile("" : "+v"(xsf[i]));
+                        const half8_t xs = __builtin_bit_cast(half8_t, xsf[i]) * _Float16(kResidue);
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs, bmin_lo[j], acc[i][j], 0, 0, 0);
+                    }
             }
             // x(s+1) must be in LDS for every wave: wait for its DMA (issued one step
             // ago; the loads issued after it -- raw(s+1), x(s+2), raw(s+2) -- may stay
@@ -573,16 +589,31 @@ RegPlan plan_reg(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const 
     const uint32_t rows_per_tile = pair ? TC / 2 : TC;
     p.ncol = (rows + rows_per_tile - 1) / rows_per_tile;
     const uint32_t nb = cols / kQK, tiles = p.ntok * p.ncol;
-    p.kparts = 1;
-    // two workgroups per CU on 256 CUs: split K until the grid covers most of them.  Plain outputs keep that
-    // many parts although fewer would leave no nearly empty second round (downs at 520-640 tokens, 75 tiles:
-    // 8 parts 148 us, 6 parts 113): a part is one chain of fp32 sums, and fewer parts are further from 64 bits.
-    while (tiles * p.kparts < 400 && p.kparts * 2 <= nb / 2) p.kparts *= 2;
-    // The pair's h is rounded to fp16 (2.1e-4), which no order of the sums shows in.  From 256 tiles on, two
-    // parts are a second round and one is not; one part is the faster up to 15 super-blocks (3,840 x 15,360 at
-    // 257-384 tokens, 360 tiles: 122 us against 139; 256-399 tiles: 0.54-1.00 of the time up to 15 super-blocks,
-    // 0.96-1.05 at 16, 1.03-1.37 at 60).
-    if (pair && p.kparts == 2 && tiles >= 256 && nb <= 15) p.kparts = 1;
+    // Two workgroups per CU on 256 CUs: split K until the grid covers most of them.  Fewer parts than that power
+    // of two where they leave no nearly empty second round, by an estimate in tenths of a microsecond (least
+    // squares over MI355X timings of the gate/up pair and the down projections): a super-block costs 5.3 us while
+    // every CU has one workgroup at most, 7.3 to 9.3 above; a round 3 us more; a last arrival reads every part
+    // where the reduce-scatter cannot run.  The power of two / the estimate: downs at 520-640 tokens (75 tiles) 8
+    // parts 148 us / 6 parts 113, 700-768 (90 tiles) 167 / 5 parts 128, 1300 (165 tiles) 4 parts 232 / 3 parts
+    // 199; the pair at 257-384 (360 tiles) 2 parts 139 / 1 part 122.  Over 8,840 random shapes 0.914 of the time
+    // (the best number of parts: 0.899), more than 5% above it in 2% of them, at most 1.16.  A part is one chain
+    // of fp32 sums: plain outputs are 1.03e-6 off against 64 bits where one chain walks 84 super-blocks, and no
+    // fewer parts than that are taken.
+    uint32_t most = 1, best = ~0u;
+    while (tiles * most < 400 && most * 2 <= nb / 2) most *= 2;
+    const uint32_t cus = uint32_t(device_cus()), slots = 2 * cus;
+    const auto cost = [&](uint32_t kp) {
+        const uint32_t n = tiles * kp, sb = (nb + kp - 1) / kp, rest = n % slots;
+        uint32_t c = n / slots * (30 + sb * 93);
+        if (rest > 0) c += 30 + sb * (rest <= cus ? 53 : 73 + 20 * (rest - cus) / cus);
+        if (kp > 1) c += kp == uint32_t(MI) && n <= slots ? 40 : 40 + 25 * kp;
+        return c;
+    };
+    for (uint32_t kp = std::min(most, (nb + 83) / 84); kp <= most; ++kp)
+        if (cost(kp) < best) {
+            best = cost(kp);
+            p.kparts = kp;
+        }
     if (t.gemm_kparts >= 1 && uint32_t(t.gemm_kparts) <= nb) p.kparts = uint32_t(t.gemm_kparts);
     // one split-K part (padded to whole tiles) must stay under 4 GiB: 32-bit offsets in the kernel
     if (uint64_t(pair ? 2 : 1) * p.ntok * TT * p.ncol * rows_per_tile * 4 >= (uint64_t(1) << 32)) p.kparts = 1;

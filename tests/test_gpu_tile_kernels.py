@@ -56,12 +56,13 @@ def test_odd_parts(ctx, tune, qtype, cols, rows, batch, kparts):
 
 
 @pytest.mark.parametrize("batch,kparts", [(600, 8), (1300, 4)])
-@pytest.mark.parametrize("qtype,layout", [(N.Q6_K, N.CDNA4), (N.Q4_K, N.CDNA4), (N.Q4_K, N.ROW_MAJOR), (N.Q6_K, N.NSMFFN)],
-                         ids=["q6k-cdna4", "q4k-cdna4", "q4k-rowmajor", "q6k-nsmffn"])
+@pytest.mark.parametrize("qtype,layout", [(N.Q6_K, N.CDNA4), (N.Q4_K, N.ROW_MAJOR), (N.Q6_K, N.NSMFFN)],
+                         ids=["q6k-cdna4", "q4k-rowmajor", "q6k-nsmffn"])
 def test_down_parts_keep_their_chains(ctx, tune, qtype, layout, batch, kparts):
     """FP32 mode, 3840 x 15360: no fewer K parts than the power of two that fills the device, so no longer chains
     of fp32 sums (against 64 bits a Q6_K down in 4 parts is 1.42 times as far off as in 8): the planned result is
-    that of 8 parts (3 x 15 tiles of 256 tokens, 5 x 15 of 128) and of 4 parts (6 x 15, 11 x 15) bit for bit."""
+    that of 8 parts (3 x 15 tiles of 256 tokens) and of 4 parts (6 x 15) bit for bit.  (Q4_K on CDNA4 may take fewer:
+    test_q4k_min_term.)"""
     cols, rows = 15360, 3840
     host = N.synth_weights(qtype, 0x63, rows, cols)
     img = host if layout == N.ROW_MAJOR else N.retile(host, qtype, cols, rows, N.ROW_MAJOR, layout)
@@ -74,3 +75,21 @@ def test_down_parts_keep_their_chains(ctx, tune, qtype, layout, batch, kparts):
     torch.cuda.synchronize()
     assert torch.isfinite(y[0]).all()
     assert torch.equal(y[0].view(torch.int32), y[1].view(torch.int32))
+
+
+@pytest.mark.parametrize("cols,rows,batch,kparts,was", [(3840, 512, 70, 1, 1.142e-6), (3840, 512, 70, 0, 1.082e-6),
+                                                        (15360, 3840, 600, 0, 1.253e-6), (21504, 256, 130, 1, 1.626e-6)])
+def test_q4k_min_term(ctx, tune, cols, rows, batch, kparts, was):
+    """Q4_K on CDNA4, FP32 mode, against 64 bits.  The min term's second fragment, an fp16 subnormal, kept 17 of its 22
+    bits, which put the outputs `was` off with 1, 4, 8 (the power of two: 6 now) and 1 K parts.  Scaled, what is left is
+    the fp32 sums: 6.9e-7, 5.8e-7, 8.9e-7 and 1.38e-6 (84 super-blocks in one chain, the longest that a plan makes)."""
+    host = N.synth_weights(N.Q4_K, 0x65, rows, cols)
+    w = torch.from_numpy(np.ascontiguousarray(N.retile(host, N.Q4_K, cols, rows, N.ROW_MAJOR, N.CDNA4))).cuda()
+    x = torch.from_numpy(N.synth_normal_f16(0x66, batch * cols).reshape(batch, cols).view(np.int16)).cuda()
+    dense = torch.empty((rows, cols), dtype=torch.float32, device="cuda")
+    ctx.dequant(w, N.Q4_K, N.CDNA4, cols, rows, 0, rows, out_f32=dense)
+    want = x.view(torch.float16).double() @ dense.double().t().contiguous()
+    y = torch.full((batch, rows), float("nan"), dtype=torch.float32, device="cuda")
+    tune("gemm_kparts", kparts)
+    ctx.matmul(w, N.Q4_K, N.CDNA4, cols, rows, batch, x, y, half_input=True)
+    assert float((y.double() - want).norm() / want.norm()) <= 0.9 * was

@@ -48,6 +48,21 @@ def test_f16_tile_over_many_rounds(cols, rows, batch, tile):
     assert cost[0] == cost[tile]
 
 
+class Grid(ctypes.Structure):
+    _fields_ = [("tiles", U32), ("kparts", U32), ("tokens", U32)]
+
+
+@pytest.mark.parametrize("cols,rows,batch,pair,kparts", [
+    (15360, 3840, 600, False, 6), (15360, 3840, 740, False, 5), (15360, 3840, 1300, False, 3), (3840, 15360, 300, True, 1),
+    (15360, 3840, 512, False, 4), (3840, 15360, 64, True, 4), (3840, 4096, 1500, False, 2), (3840, 3840, 64, False, 4)])
+def test_q4k_parts_leave_no_empty_round(cols, rows, batch, pair, kparts):
+    """Q4_K on CDNA4, FP32 mode: fewer K parts than the power of two (8, 8, 4, 2; 8, 4) where two workgroups per CU
+    would make a nearly empty second round or share a CU for little; that power of two where it fits."""
+    f = function("_ZN2ns13gemm_reg_gridEjjjbRKNS_6TuningE", Grid)
+    g = f(U32(cols), U32(rows), U32(batch), ctypes.c_bool(pair), tuning())
+    assert (g.tokens, g.kparts) == (128, kparts)
+
+
 def test_context_need_covers_every_batch():
     """A context is sized at multiples of 16 tokens: no batch between them needs more, on either kind of kernel."""
     tile = function("_ZN2ns24gemm_tile_workspace_needEiiijjjbRKNS_6TuningEPmS3_", None)
