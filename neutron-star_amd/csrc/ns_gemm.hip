@@ -877,7 +877,13 @@ struct GemmPlan {
 // where they leave no nearly empty second round (Q6_K downs at 600 tokens, 45 tiles: 8 parts 168-189 us,
 // 4 parts 114-118), but a part is one chain of fp32 sums: against 64 bits those outputs are 2.85e-7 off in
 // 8 parts, 4.05e-7 in 4 (scales of 5 bits; with larger ones the tile's rounding, 1.4e-4, hides it).
-GemmPlan plan_gemm(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t) {
+// The pair's h (rounded to fp16) and the FP16 mode (4.4e-4) show nothing of it and take fewer parts by an
+// estimate, in tenths of a microsecond (one workgroup per CU): a round costs 30 us and 4.9 per super-block, and
+// a last arrival reads the parts (2 us each) where the reduce-scatter cannot run.  (Q6_K's super-blocks cost
+// 25 us: at 4.9, 32,768 columns took 16 parts for 32 and 1.2-1.4 times as long.)  Over 12,800 random
+// shapes 0.956 of the power of two's time (the best number of parts: 0.95), more than 5% above it in 0.3% of
+// them, at most 1.15; the pair 8192 x 5120 at 5-256 tokens 180 us in 8 parts, 98 in 4.
+GemmPlan plan_gemm(int type, uint32_t cols, uint32_t rows, uint32_t batch, bool pair, int acc, const Tuning &t) {
     GemmPlan p;
     p.ntok = (batch + TT - 1) / TT;
     const uint32_t rows_per_tile = pair ? TC / 2 : TC;
@@ -885,6 +891,19 @@ GemmPlan plan_gemm(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, cons
     const uint32_t nb = cols / kQK, tiles = p.ntok * p.ncol;
     p.kparts = 1;
     while (tiles * p.kparts < 200 && p.kparts * 2 <= nb / 4) p.kparts *= 2;
+    if (pair || acc == ACC_FP16) {
+        const uint32_t cus = uint32_t(device_cus()), most = p.kparts;
+        const auto cost = [&](uint32_t kp) {
+            const bool scatter = MI % kp == 0 && tiles * kp <= cus;
+            return (tiles * kp + cus - 1) / cus * (300 + (nb + kp - 1) / kp * (type == Q4_K ? 49 : 250)) + (scatter ? 0 : kp * 20);
+        };
+        uint32_t best = ~0u;
+        for (uint32_t kp = 1; kp <= most; ++kp)
+            if (cost(kp) < best) {
+                best = cost(kp);
+                p.kparts = kp;
+            }
+    }
     if (t.gemm_kparts >= 1 && uint32_t(t.gemm_kparts) <= nb) p.kparts = uint32_t(t.gemm_kparts);
     // one split-K part (padded to whole tiles) must stay under 4 GiB: 32-bit offsets in the kernel
     if (uint64_t(pair ? 2 : 1) * p.ntok * TT * p.ncol * rows_per_tile * 4 >= (uint64_t(1) << 32)) p.kparts = 1;
@@ -920,7 +939,7 @@ template <int TYPE, int LAYOUT, bool PAIR>
 hipError_t launch_mode(int acc, const uint8_t *w, const uint8_t *up, const uint16_t *x, const uint16_t *xh,
                        void *out, uint32_t cols, uint32_t rows, uint32_t batch, const Workspace &ws,
                        size_t ws_offset, hipStream_t stream) {
-    const GemmPlan p = plan_gemm(cols, rows, batch, PAIR, ws.tune);
+    const GemmPlan p = plan_gemm(TYPE, cols, rows, batch, PAIR, acc, ws.tune);
     const dim3 grid(p.ntok * p.ncol * p.kparts), block(kThreads);
     const uint32_t wbytes = rows * (cols / kQK) * block_bytes(TYPE);
     float *partial = ws.partial + ws_offset;
@@ -952,8 +971,8 @@ hipError_t launch_layout(int layout, int acc, const uint8_t *w, const uint8_t *u
 
 }  // namespace
 
-TileGrid gemm_grid(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t) {
-    const GemmPlan p = plan_gemm(cols, rows, batch, pair, t);
+TileGrid gemm_grid(int type, uint32_t cols, uint32_t rows, uint32_t batch, bool pair, int acc, const Tuning &t) {
+    const GemmPlan p = plan_gemm(type, cols, rows, batch, pair, acc, t);
     return {p.ntok * p.ncol, p.kparts, TT};
 }
 
@@ -964,7 +983,7 @@ static size_t xs_floats(int type, uint32_t cols, uint32_t batch) {
     return type == Q4_K ? xs_layout(cols, batch).total : 0;
 }
 
-static void gemm_fp32_workspace_need(int type, int layout, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
+static void gemm_main_workspace_need(int type, int layout, int acc, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
                                      const Tuning &t, size_t *floats, size_t *counters);
 
 // Q4_K on the CDNA4 layout runs the register-fragment kernel (ns_gemm_reg.hip)
@@ -986,10 +1005,10 @@ void gemm_workspace_need(int type, int layout, int acc, uint32_t cols, uint32_t 
 void gemm_tile_workspace_need(int type, int layout, int acc, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
                               const Tuning &t, size_t *floats, size_t *counters) {
     if (layout == CDNA4 && acc == ACC_FP16) gemm_f16_workspace_need(cols, rows, batch, pair, t, floats, counters);
-    else gemm_fp32_workspace_need(type, layout, cols, rows, batch, pair, t, floats, counters);
+    else gemm_main_workspace_need(type, layout, acc, cols, rows, batch, pair, t, floats, counters);
 }
 
-static void gemm_fp32_workspace_need(int type, int layout, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
+static void gemm_main_workspace_need(int type, int layout, int acc, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,
                                      const Tuning &t, size_t *floats, size_t *counters) {
     if (use_gemm_reg(type, layout, t)) {
         size_t part = 0;
@@ -997,7 +1016,7 @@ static void gemm_fp32_workspace_need(int type, int layout, uint32_t cols, uint32
         *floats = xs_floats(type, cols, batch) + part;
         return;
     }
-    const GemmPlan p = plan_gemm(cols, rows, batch, pair, t);
+    const GemmPlan p = plan_gemm(type, cols, rows, batch, pair, acc, t);
     *floats = xs_floats(type, cols, batch) +
               (p.kparts > 1 ? size_t(p.kparts) * (pair ? 2 : 1) * (p.ntok * TT) * (p.ncol * (pair ? TC / 2 : TC)) : 0);
     *counters = 2 * size_t(p.ntok) * p.ncol;  // arrivals; and departures of the reduce-scatter

@@ -837,7 +837,7 @@ double skinny_us(const Route &r, const Plan &p, uint32_t cols, const uint32_t *r
 double tile_us(const Route &r, int type, int layout, uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t) {
     const auto &c = r.tile;
     const bool reg = layout == CDNA4 && type == Q4_K;
-    const TileGrid g = reg ? gemm_reg_grid(cols, rows, batch, pair, t) : gemm_grid(cols, rows, batch, pair, t);
+    const TileGrid g = reg ? gemm_reg_grid(cols, rows, batch, pair, t) : gemm_grid(type, cols, rows, batch, pair, ACC_FP32, t);
     const double n = double(g.tiles) * g.kparts, q = n / device_cus();
     const uint32_t nb = cols / kQK, sb = (nb + g.kparts - 1) / g.kparts;
     const double rounds = reg ? (q <= 2 ? 1 : q / 2 + c.over) : (q <= 1 ? 1 : q + c.over);

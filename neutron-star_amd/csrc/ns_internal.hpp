@@ -213,7 +213,7 @@ struct TileGrid {
     uint32_t tiles, kparts, tokens;
 };
 TileGrid gemm_reg_grid(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t);
-TileGrid gemm_grid(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const Tuning &t);
+TileGrid gemm_grid(int type, uint32_t cols, uint32_t rows, uint32_t batch, bool pair, int acc, const Tuning &t);
 
 // The prefill GEMM for few tokens (ns_gemm_skinny.hip): CDNA4 in both modes, ROW_MAJOR in the FP32
 // mode without the pair.  Up to three matrices that share x (rows, w and out arrays of nseg

@@ -63,6 +63,19 @@ def test_q4k_parts_leave_no_empty_round(cols, rows, batch, pair, kparts):
     assert (g.tokens, g.kparts) == (128, kparts)
 
 
+@pytest.mark.parametrize("qtype,cols,rows,batch,pair,acc,kparts", [
+    (N.Q4_K, 8192, 5120, 64, True, N.ACC_FP32, 4), (N.Q4_K, 8192, 11520, 64, False, N.ACC_FP16, 4),
+    (N.Q4_K, 8192, 11520, 64, False, N.ACC_FP32, 8), (N.Q4_K, 2304, 49152, 5, False, N.ACC_FP16, 1),
+    (N.Q4_K, 2304, 49152, 5, False, N.ACC_FP32, 2), (N.Q6_K, 32768, 1024, 55, False, N.ACC_FP16, 32),
+    (N.Q6_K, 15360, 3840, 600, False, N.ACC_FP16, 5), (N.Q6_K, 15360, 3840, 600, False, N.ACC_FP32, 8)])
+def test_lds_tile_parts(qtype, cols, rows, batch, pair, acc, kparts):
+    """The LDS-tile GEMM: the pair and the FP16 mode (results rounded to fp16) take fewer K parts where the power of two
+    would make a nearly empty second round; plain FP32-mode outputs keep it, as their error grows with the chains."""
+    f = function("_ZN2ns9gemm_gridEijjjbiRKNS_6TuningE", Grid)
+    g = f(qtype, U32(cols), U32(rows), U32(batch), ctypes.c_bool(pair), acc, tuning())
+    assert (g.tokens, g.kparts) == (256, kparts)
+
+
 def test_context_need_covers_every_batch():
     """A context is sized at multiples of 16 tokens: no batch between them needs more, on either kind of kernel."""
     tile = function("_ZN2ns24gemm_tile_workspace_needEiiijjjbRKNS_6TuningEPmS3_", None)
