@@ -903,6 +903,8 @@ bool gemm_skinny_eligible(int type, int layout, int acc, uint32_t cols, uint32_t
     // (and a bound: past two rounds the weights are read once per token tile from beyond L2, which the
     // estimate leaves out: downs at 600 tokens 124-130 us here, 109 there)
     if (acc == ACC_FP16) return p.cost <= std::min(800u, gemm_f16_cost(cols, rows, batch, pair, plain));
+    // one super-block and up to two workgroups per CU, which the estimate has in turn: 10.8 us here, 15.3 there
+    if (type == Q4_K && layout == CDNA4 && cols == kQK && p.mi == 1 && p.ncol * p.ntok <= 2 * uint32_t(device_cus())) return true;
     const Route &r = route_of(type, layout, pair);
     return skinny_us(r, p, cols, &rows, 1, batch, pair) <= 0.95 * tile_us(r, type, layout, cols, rows, batch, pair, plain);
 }
@@ -927,10 +929,13 @@ double small_us(int type, int layout, uint32_t cols, uint32_t rows, uint32_t bat
 
 }  // namespace
 
-// Row-major tensors by the two estimates (Q4_K at 3-4 tokens, where that of the small-batch kernel is low, by 5%
-// more); short rows, whose estimates are loose, stay there.  Over 8,900 random shapes the choice is more than 5%
-// slower than the small-batch kernels in 0.7% of them, and more than 5% slower than this one in 3% (2,048 x
-// 3,840 at 3 tokens 9.4 us here, 12.4 there; Q6_K 64 x 3,840 13 / 10, 65,536 x 2,304 55 / 76).  Q4_K on CDNA4:
+// Row-major tensors by the two estimates (but for Q4_K at 2 tokens by 5% more, as that of the small-batch kernel is
+// low); short rows, whose estimates are loose, stay there.  Q6_K of many super-blocks, and many Q6_K rows at 3-4
+// tokens, are always here, where the small-batch kernel may take 1.5 times what its estimate has and this one does
+// not (21,504 rows: 2,304 columns at 3 tokens 27 us here, 48 there, 15,360 at 2 tokens 140 / 208).  Over 31,300
+// random shapes the choice is more than 5% slower than the small-batch kernels in 0.9% of them, and more than 5%
+// slower than this one in 2.1% (2,048 x 3,840 at 3 tokens 9.4 us here, 12.4 there; Q6_K 64 x 3,840 13 / 10, 65,536 x
+// 2,304 55 / 76).  Q4_K on CDNA4:
 // here but for tall matrices of up to 15 super-blocks, which the small-batch kernel walks with a wave per slab and
 // no hand-off (at up to two slabs per CU 0.58-1.00 of its time, at 65,536-262,144 rows 1.1-2.0 of it).  Q6_K on
 // CDNA4: not exact here (kExact).
@@ -939,11 +944,12 @@ bool skinny_small_batch(int type, int layout, uint32_t cols, uint32_t rows, cons
     if (t.gemm_skinny > 0) return batch <= uint32_t(t.gemm_skinny);
     const uint32_t nb = cols / kQK;
     if (layout == CDNA4) return nb > 15 || rows <= 2 * uint32_t(device_cus()) * kRowTile;
+    if (type == Q6_K && ((batch > 2 && nb >= 3 && rows >= 20480) || (nb >= 6 && uint64_t(rows) * nb >= 61440))) return true;
     if (nb < (type == Q4_K ? 2u : 6u)) return false;
     Tuning plain = t;
     plain.gemm_kparts = 0;
     return skinny_us(route_of(type, layout, false), plan_skinny(type, cols, &rows, 1, batch, false, false, plain), cols, &rows, 1,
-                     batch, false) <= (type == Q4_K && batch > 2 ? 1.05 : 1.0) * small_us(type, layout, cols, rows, batch);
+                     batch, false) <= (type == Q4_K && batch == 2 ? 1.0 : 1.05) * small_us(type, layout, cols, rows, batch);
 }
 
 // Q, K and V (or Q and a K that is V too) in one launch: against the launches of their own that they would take.

@@ -76,6 +76,25 @@ def test_lds_tile_parts(qtype, cols, rows, batch, pair, acc, kparts):
     assert (g.tokens, g.kparts) == (256, kparts)
 
 
+@pytest.mark.parametrize("qtype,layout,cols,rows,batch,here", [
+    (N.Q6_K, N.ROW_MAJOR, 2304, 21504, 3, True), (N.Q6_K, N.ROW_MAJOR, 15360, 21504, 2, True),
+    (N.Q6_K, N.ROW_MAJOR, 1024, 32768, 4, True), (N.Q6_K, N.ROW_MAJOR, 1024, 2048, 4, False),
+    (N.Q6_K, N.ROW_MAJOR, 512, 262144, 4, False), (N.Q6_K, N.ROW_MAJOR, 3840, 64, 3, False),
+    (N.Q4_K, N.ROW_MAJOR, 3840, 21504, 3, True), (N.Q4_K, N.ROW_MAJOR, 256, 21504, 3, False)])
+def test_small_batch_rule(qtype, layout, cols, rows, batch, here):
+    """Batch 2-4 on row-major tensors: where the few-token GEMM takes a call from the small-batch kernel, which is 1.2 to
+    1.8 times as fast or slow on these."""
+    f = function("_ZN2ns18skinny_small_batchEiijjPKvjRKNS_6TuningE", ctypes.c_bool)
+    assert f(qtype, layout, U32(cols), U32(rows), ctypes.c_void_p(4096), U32(batch), tuning()) is here
+
+
+@pytest.mark.parametrize("rows,batch,here", [(32768, 5, True), (32768, 32, True), (32768, 33, False), (65536, 16, False)])
+def test_one_super_block_pair(rows, batch, here):
+    """The gate/up pair at 256 columns: up to two workgroups per CU run at once (10.8 us, the tile kernel 15.3)."""
+    f = function("_ZN2ns20gemm_skinny_eligibleEiiijjjbRKNS_6TuningE", ctypes.c_bool)
+    assert f(N.Q4_K, N.CDNA4, N.ACC_FP32, U32(256), U32(rows), U32(batch), ctypes.c_bool(True), tuning()) is here
+
+
 def test_context_need_covers_every_batch():
     """A context is sized at multiples of 16 tokens: no batch between them needs more, on either kind of kernel."""
     tile = function("_ZN2ns24gemm_tile_workspace_needEiiijjjbRKNS_6TuningEPmS3_", None)

@@ -80,11 +80,11 @@ def test_noalloc_prefill_matches_matmul_with_one_k_part(ctx, first, second):
 @pytest.mark.parametrize("qtype,layout,rows,cols,batch", [
     (N.Q6_K, N.CDNA4, 3840, 15360, 5), (N.Q4_K, N.CDNA4, 3840, 15360, 5), (N.Q6_K, N.CDNA4, 3840, 15360, 32),
     (N.Q4_K, N.CDNA4, 3840, 15360, 256), (N.Q4_K, N.CDNA4, 15360, 3840, 300), (N.Q4_K, N.ROW_MAJOR, 2048, 3840, 64),
-    (N.Q4_K, N.CDNA4, 3840, 15360, 600), (N.Q6_K, N.ROW_MAJOR, 2048, 15360, 3)])
+    (N.Q4_K, N.CDNA4, 1024, 15360, 600), (N.Q6_K, N.ROW_MAJOR, 2048, 15360, 3)])
 def test_noalloc_few_tokens_match_matmul(ctx, qtype, layout, rows, cols, batch):
     """Where ns_matmul takes the few-token GEMM, whose parts fit the scratch, the call runs the same plan: equal
-    bit for bit with nothing tuned, whatever the tile kernels would have needed (at 600 tokens of a 15,360-column
-    Q4_K down more than the scratch even with one K part)."""
+    bit for bit with nothing tuned, whatever the tile kernels would have needed (at 600 tokens of 15,360 columns
+    more than the scratch even with one K part; 1,024 rows, where the route is still this one)."""
     host = N.synth_weights(qtype, 340, rows, cols)
     img = host if layout == N.ROW_MAJOR else N.retile(host, qtype, cols, rows, N.ROW_MAJOR, layout)
     w = torch.from_numpy(np.ascontiguousarray(img)).cuda()
