@@ -885,9 +885,9 @@ hipError_t launch_mixed(const Plan &p, const Args &a, hipStream_t stream) {
 // (gate/up 128 tokens: 44 us here, 50 there; 225: 75 / 65; downs 225: 43-46 / 48-55; 320: 63-67 / 63).
 // FP32 mode: by the two estimates of Route, 5% for their error.  Over 37,000 random shapes (256 to 32,768
 // columns, 64 to 262,144 rows, 5 to 2,048 tokens) the choice is more than 5% slower than the tile kernels in
-// 0.2% of them and more than 5% slower than this kernel in 1%; it takes 0.362 of the tile kernels' time
-// (geometric mean), the better one of each two 0.361.  MI355X, this kernel against them (us):
-//   gate/up 192 tokens: 81 / 94, 225: 106 / 95;  downs 512: 78-96 / 114-127, 775: 157-180 / 134-145
+// 0.2% of them (0.5% for Q4_K on CDNA4) and more than 5% slower than this kernel in 1%; it takes 0.362 of the tile
+// kernels' time (geometric mean), the better one of each two 0.361.  MI355X, this kernel against them (us):
+//   gate/up 192 tokens: 81 / 94, 225: 106 / 95;  downs 512: 78-96 / 105-127, 775: 157-180 / 134-145
 //   4096 x 3840, 1536 tokens: 89 / 114, row-major 93 / 95;  2048: 121 / 103, row-major 125 / 106
 //   256 columns: 65,536 rows at 71 tokens 55 / 23 (the pair), Q6_K at 217 62 / 20
 bool gemm_skinny_eligible(int type, int layout, int acc, uint32_t cols, uint32_t rows, uint32_t batch, bool pair,

@@ -107,3 +107,11 @@ def test_noalloc_refuses_shapes_past_the_scratch():
     with pytest.raises(N.NsError, match="static scratch"):
         N.matmul_noalloc(w, N.Q4_K, N.CDNA4, cols, rows, batch, x, y, half_input=True)
     N.noalloc_status()
+
+
+def test_context_room_for_other_shapes():
+    """A new context holds 39.1 M floats of parts whatever the plans of the model's own shapes come to (36.1 M with
+    the estimated K parts): under capture, where it cannot grow, the pair 1,344 x 16,384 at 2,586 tokens needs 38.4 M."""
+    c = N.Context(0)
+    assert c.workspace_bytes() >= 39139264 * 4
+    c.close()
