@@ -597,8 +597,8 @@ RegPlan plan_reg(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const 
     // parts 148 us / 6 parts 113, 700-768 (90 tiles) 167 / 5 parts 128, 1300 (165 tiles) 4 parts 232 / 3 parts
     // 199; the pair at 257-384 (360 tiles) 2 parts 139 / 1 part 122.  Over 8,840 random shapes 0.914 of the time
     // (the best number of parts: 0.899), more than 5% above it in 2% of them, at most 1.16.  A part is one chain
-    // of fp32 sums: plain outputs are 1.03e-6 off against 64 bits where one chain walks 84 super-blocks, and no
-    // fewer parts than that are taken.
+    // of fp32 sums: plain outputs are 1.03e-6 off against 64 bits where one chain walks 84 super-blocks, and the
+    // estimate makes none longer (the pair's h is rounded to fp16, which hides it).
     uint32_t most = 1, best = ~0u;
     while (tiles * most < 400 && most * 2 <= nb / 2) most *= 2;
     const uint32_t cus = uint32_t(device_cus()), slots = 2 * cus;
@@ -609,7 +609,7 @@ RegPlan plan_reg(uint32_t cols, uint32_t rows, uint32_t batch, bool pair, const 
         if (kp > 1) c += kp == uint32_t(MI) && n <= slots ? 40 : 40 + 25 * kp;
         return c;
     };
-    for (uint32_t kp = std::min(most, (nb + 83) / 84); kp <= most; ++kp)
+    for (uint32_t kp = pair ? 1 : std::min(most, (nb + 83) / 84); kp <= most; ++kp)
         if (cost(kp) < best) {
             best = cost(kp);
             p.kparts = kp;

@@ -82,7 +82,7 @@ def test_down_parts_keep_their_chains(ctx, tune, qtype, layout, batch, kparts):
 def test_q4k_min_term(ctx, tune, cols, rows, batch, kparts, was):
     """Q4_K on CDNA4, FP32 mode, against 64 bits.  The min term's second fragment, an fp16 subnormal, kept 17 of its 22
     bits, which put the outputs `was` off with 1, 4, 8 (the power of two: 6 now) and 1 K parts.  Scaled, what is left is
-    the fp32 sums: 6.9e-7, 5.8e-7, 8.9e-7 and 1.38e-6 (84 super-blocks in one chain, the longest that a plan makes)."""
+    the fp32 sums: 6.9e-7, 5.8e-7, 8.9e-7 and 1.38e-6 (84 super-blocks in one chain, the longest that the estimate makes)."""
     host = N.synth_weights(N.Q4_K, 0x65, rows, cols)
     w = torch.from_numpy(np.ascontiguousarray(N.retile(host, N.Q4_K, cols, rows, N.ROW_MAJOR, N.CDNA4))).cuda()
     x = torch.from_numpy(N.synth_normal_f16(0x66, batch * cols).reshape(batch, cols).view(np.int16)).cuda()

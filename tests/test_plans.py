@@ -54,10 +54,12 @@ class Grid(ctypes.Structure):
 
 @pytest.mark.parametrize("cols,rows,batch,pair,kparts", [
     (15360, 3840, 600, False, 6), (15360, 3840, 740, False, 5), (15360, 3840, 1300, False, 3), (3840, 15360, 300, True, 1),
-    (15360, 3840, 512, False, 4), (3840, 15360, 64, True, 4), (3840, 4096, 1500, False, 2), (3840, 3840, 64, False, 4)])
+    (15360, 3840, 512, False, 4), (3840, 15360, 64, True, 4), (3840, 4096, 1500, False, 2), (3840, 3840, 64, False, 4),
+    (32768, 3776, 1652, True, 1)])
 def test_q4k_parts_leave_no_empty_round(cols, rows, batch, pair, kparts):
     """Q4_K on CDNA4, FP32 mode: fewer K parts than the power of two (8, 8, 4, 2; 8, 4) where two workgroups per CU
-    would make a nearly empty second round or share a CU for little; that power of two where it fits."""
+    would make a nearly empty second round or share a CU for little; that power of two where it fits.  The pair may walk
+    all of K in one chain."""
     f = function("_ZN2ns13gemm_reg_gridEjjjbRKNS_6TuningE", Grid)
     g = f(U32(cols), U32(rows), U32(batch), ctypes.c_bool(pair), tuning())
     assert (g.tokens, g.kparts) == (128, kparts)
